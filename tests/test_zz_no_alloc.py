@@ -11,6 +11,7 @@ The file sorts last on purpose: a failure here must not hide the other tests
 under `pytest -x`.
 """
 import ctypes
+import gc
 
 import pytest
 import torch
@@ -65,6 +66,7 @@ def _run_static(lib, m, desc, img, obs, k, warm):
     see only torch's allocator) must not move across the call."""
     B, n_log = obs.shape[0], N_ACTION_HEADS * m.n_gears
     lg, v = _outputs(B, n_log)
+    gc.collect()                 # an earlier test's tensors that only the cyclic collector frees must not go inside the measured window
     torch.cuda.synchronize()
     before, free_before = torch.cuda.memory_allocated(), torch.cuda.mem_get_info()[0]
     _call_static(lib, m, desc, img, obs, k, lg, v)
