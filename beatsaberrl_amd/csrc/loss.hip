@@ -44,7 +44,8 @@ __global__ __launch_bounds__(256) void hl_loss_kernel(const float* __restrict__ 
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const float c0 = centers[0], half = 0.5f * (centers[1] - c0);
-    const float v = fminf(fmaxf(v_tgt[row], c0 - half), centers[n - 1] + half);
+    const float vt = v_tgt[row];                             // a NaN return stays NaN (fmin / fmax would drop it): loss and gradient show it
+    const float v = vt != vt ? vt : fminf(fmaxf(vt, c0 - half), centers[n - 1] + half);
     const float* x = logits + row * n;
     float l[PER], p[PER], m = -INFINITY, tot = 0.f;
 #pragma unroll
