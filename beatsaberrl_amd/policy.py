@@ -179,12 +179,20 @@ def hl_target(v, centers, sigma: float):
     return p / p.sum(-1, keepdim=True)
 
 
+def _hl_kernel_takes(logits, v_tgt, centers, sigma) -> bool:
+    """Whether the loss kernel covers these arguments: one row of bins per env, one return per row, one centre per bin, all on
+    one device.  Everything else is torch's expression, with its broadcasting and its errors."""
+    return (logits.dim() == 2 and 2 <= logits.shape[1] <= 512 and logits.shape[0] > 0 and v_tgt.shape == logits.shape[:1]
+            and centers.shape == logits.shape[1:] and centers.dtype is torch.float32
+            and v_tgt.device == logits.device and centers.device == logits.device
+            and not v_tgt.requires_grad and not centers.requires_grad and isinstance(sigma, (int, float)) and sigma > 0)
+
+
 def hl_loss(logits, v_tgt, centers, sigma: float):
     """Cross-entropy between the critic's bin distribution and the HL-Gauss target, batch mean
     (reference python/policy.py:776-781); logits (B, K) fp32 = `policy._value_logits` of the update forward.  On the
     device one kernel forms loss and gradient."""
-    if (logits.is_cuda and logits.dim() == 2 and 2 <= logits.shape[1] <= 512 and logits.shape[0] > 0 and v_tgt.shape == logits.shape[:1]
-            and centers.dtype is torch.float32 and not v_tgt.requires_grad and not centers.requires_grad):
+    if logits.is_cuda and _hl_kernel_takes(logits, v_tgt, centers, sigma):
         return HlLossFn.apply(logits.float().contiguous(), v_tgt.float().contiguous(), centers.contiguous(), float(sigma))
     return -(hl_target(v_tgt, centers, sigma) * F.log_softmax(logits.float(), dim=-1)).sum(-1).mean()
 

@@ -88,3 +88,13 @@ def test_simbav2_init_and_projection():
     assert torch.allclose(p.trunk_w1.weight.norm(dim=1), torch.ones(128), atol=1e-6)
     assert torch.count_nonzero(p.trunk_w1.bias) == 0
     assert not NotePolicy(embed=64, trunk_dim=96, n_blocks=2, n_heads=2).project_trunk_weights()
+
+
+def test_hl_loss_kernel_takes_only_what_it_covers():
+    from beatsaberrl_amd.policy import _hl_kernel_takes
+    x, v, c = torch.randn(4, 51), torch.randn(4), torch.linspace(-6, 6, 51)
+    assert _hl_kernel_takes(x, v, c, 0.1) and _hl_kernel_takes(x.double(), v.long(), c, 1)
+    for args in ((x, v.to("meta"), c, 0.1), (x, v, c.to("meta"), 0.1), (x, v, c[:50], 0.1), (x, v, c[None], 0.1), (x, v[:3], c, 0.1),
+                 (x[:0], v[:0], c, 0.1), (x[0], v, c, 0.1), (x[:, :1], v, c[:1], 0.1), (x, v, c.double(), 0.1), (x, v, c, 0.0),
+                 (x, v, c, torch.tensor(0.1)), (x, v.clone().requires_grad_(), c, 0.1), (torch.randn(4, 513), v, torch.randn(513), 0.1)):
+        assert not _hl_kernel_takes(*args)

@@ -33,3 +33,17 @@ def test_hl_loss_of_returns_that_are_not_finite(K):
     assert torch.isnan(loss) and torch.isnan(_hl_torch(x, v, centers, sigma))
     g, = torch.autograd.grad(loss, x)
     assert torch.isnan(g).any(-1).tolist() == [i == 3 for i in range(7)]
+
+
+def test_hl_loss_arguments_the_kernel_does_not_cover():
+    """A tensor on the host is refused, never handed to the kernel; other shapes get torch's broadcasting and errors."""
+    x, v, centers, sigma = _bins(6, 101)
+    for args in ((x, v.cpu(), centers, sigma), (x, v, centers.cpu(), sigma), (x, v, centers[:50], sigma), (x, v[:5], centers, sigma)):
+        with pytest.raises(RuntimeError):
+            hl_loss(*args)
+    one = x[:, :1].detach()
+    assert torch.equal(hl_loss(one, v, centers, sigma), _hl_torch(one, v, centers, sigma))            # logits broadcast over the bins
+    s = torch.tensor(sigma, device=DEV, requires_grad=True)                                           # a width that is learned
+    g, = torch.autograd.grad(hl_loss(x, v, centers, s), s)
+    assert torch.isfinite(g) and g.item() != 0.0
+    assert torch.isnan(hl_loss(x[:0], v[:0], centers, sigma))
