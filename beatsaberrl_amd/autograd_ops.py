@@ -22,6 +22,8 @@ from __future__ import annotations
 import ctypes
 
 import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 from . import fp16_linear as _fl
@@ -292,43 +294,58 @@ class AttnQKVFn(torch.autograd.Function):
         return dq, dkv, None, None
 
 
+def _plain_eager(*ts) -> bool:
+    """No transform is watching: nothing of torch.func, forward-mode AD, a batch of gradients or a dispatch mode (tracing, fake
+    tensors), which would not see a launch through ctypes, and no tensor subclass."""
+    return (not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_legacy_batchedtensor(t) for t in ts))
+
+
 class HeadsLogpFn(torch.autograd.Function):
     """(logprob, entropy, per-head entropy) of given actions on fp32 logits (B, n_heads, K): the sampling kernel's evaluation
-    forward, one kernel back.  The per-head entropy carries no gradient."""
+    forward, one kernel back.  The per-head entropy carries no gradient.  A backward that is itself differentiated is torch's."""
 
     @staticmethod
     def forward(ctx, logits, action):
-        logits = logits.contiguous()
-        action = action.contiguous()
-        _, logprob, entropy, ent_h, _ = ops.sample_heads(logits, action=action, want_ent_h=True)
+        _, logprob, entropy, ent_h, _ = ops.sample_heads(logits.contiguous(), action=action.contiguous(), want_ent_h=True)
         ctx.save_for_backward(logits, action)
         ctx.mark_non_differentiable(ent_h)
         ctx.set_materialize_grads(False)
         return logprob, entropy, ent_h
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, glp, gent, _):
         logits, action = ctx.saved_tensors
         if glp is None and gent is None:
             return None, None
+        if torch.is_grad_enabled() or not _plain_eager(logits, *(g for g in (glp, gent) if g is not None)):
+            logsm = torch.log_softmax(logits, dim=-1)
+            p, d = logsm.exp(), 0.0
+            if glp is not None:
+                d = glp[:, None, None] * (F.one_hot(action, logits.shape[-1]) - p)
+            if gent is not None:
+                d = d - gent[:, None, None] * p * (logsm - (p * logsm).sum(-1, keepdim=True))
+            return d, None
         c = lambda g: None if g is None else g.contiguous()
-        return ops.heads_logp_bwd(logits, action, c(glp), c(gent)), None
+        return ops.heads_logp_bwd(c(logits), c(action), c(glp), c(gent)), None
 
 
 class HlLossFn(torch.autograd.Function):
-    """Batch mean of the HL-Gauss critic loss on fp32 bin logits; the row kernel leaves its gradient beside the loss."""
+    """Batch mean of the HL-Gauss critic loss on fp32 bin logits; the row kernel leaves its gradient, softmax(logits) - target,
+    beside the loss."""
 
     @staticmethod
     def forward(ctx, logits, v_tgt, centers, sigma):
         loss, grad = ops.hl_loss_rows(logits, v_tgt, centers, sigma)
-        ctx.save_for_backward(grad)
+        ctx.save_for_backward(grad, logits)
         return loss.mean()
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, g):
-        grad, = ctx.saved_tensors
+        grad, logits = ctx.saved_tensors
+        if torch.is_grad_enabled():                            # to be differentiated again: the softmax as a function of the logits
+            p = torch.softmax(logits, dim=-1)
+            grad = p - (p.detach() - grad)
         return grad * (g / grad.shape[0]), None, None, None
 
 

@@ -44,7 +44,7 @@ from . import _lib
 from . import fp16_linear as _fl
 from . import obs_layout as L
 from . import ops
-from .autograd_ops import AttnPackedFn, AttnQKVFn, ChainFn, FusedFfnFn, HeadsLogpFn, HlLossFn, LinearFn, LnResFn, NoteTrainFn, NoteTrainPlan
+from .autograd_ops import AttnPackedFn, AttnQKVFn, ChainFn, FusedFfnFn, HeadsLogpFn, HlLossFn, LinearFn, LnResFn, NoteTrainFn, NoteTrainPlan, _plain_eager
 from .fused_ln import FusedLayerNorm
 
 OBS_DIM = L.OBS_DIM
@@ -192,7 +192,7 @@ def hl_loss(logits, v_tgt, centers, sigma: float):
     """Cross-entropy between the critic's bin distribution and the HL-Gauss target, batch mean
     (reference python/policy.py:776-781); logits (B, K) fp32 = `policy._value_logits` of the update forward.  On the
     device one kernel forms loss and gradient."""
-    if logits.is_cuda and _hl_kernel_takes(logits, v_tgt, centers, sigma):
+    if logits.is_cuda and _plain_eager(logits, v_tgt, centers) and _hl_kernel_takes(logits, v_tgt, centers, sigma):
         return HlLossFn.apply(logits.float().contiguous(), v_tgt.float().contiguous(), centers.contiguous(), float(sigma))
     return -(hl_target(v_tgt, centers, sigma) * F.log_softmax(logits.float(), dim=-1)).sum(-1).mean()
 

@@ -1,6 +1,7 @@
-"""The update's loss kernels at inputs where they could part from torch's expression: returns that are not numbers."""
+"""The update's loss kernels at inputs and under transforms where they could part from torch's expression."""
 import pytest
 import torch
+import torch.autograd.forward_ad  # noqa: F401
 import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,47 @@ def test_hl_loss_arguments_the_kernel_does_not_cover():
     g, = torch.autograd.grad(hl_loss(x, v, centers, s), s)
     assert torch.isfinite(g) and g.item() != 0.0
     assert torch.isnan(hl_loss(x[:0], v[:0], centers, sigma))
+
+
+def test_hl_loss_differentiated_twice_and_under_transforms():
+    """What torch's expression gives: a Hessian-vector product, grad / vmap / jvp of torch.func, a forward-mode tangent."""
+    x, v, centers, sigma = _bins(9, 101)
+    u = torch.randn(9, 101, device=DEV)
+    hvp = []
+    for f in (hl_loss, _hl_torch):
+        g, = torch.autograd.grad(f(x, v, centers, sigma), x, create_graph=True)
+        hvp.append((g.detach(), torch.autograd.grad((g * u).sum(), x)[0]))
+    for got, want in zip(*hvp):         # fp32 softmax, erf and their differences: a few ulp of values up to 1 / B
+        assert torch.allclose(got, want, atol=3e-5 / 9)
+    f, t = (lambda a: hl_loss(a, v, centers, sigma)), (lambda a: _hl_torch(a, v, centers, sigma))
+    y = x.detach()
+    assert torch.equal(torch.func.grad(f)(y), torch.func.grad(t)(y))
+    batch = torch.stack([y, 2 * y, -y])
+    assert torch.equal(torch.func.vmap(f)(batch), torch.func.vmap(t)(batch))
+    assert all(torch.equal(a, b) for a, b in zip(torch.func.jvp(f, (y,), (u,)), torch.func.jvp(t, (y,), (u,))))
+    with torch.autograd.forward_ad.dual_level():
+        d = torch.autograd.forward_ad.make_dual(y, u)
+        a, b = (torch.autograd.forward_ad.unpack_dual(g(d)).tangent for g in (f, t))
+        assert torch.equal(a, b)
+
+
+def test_heads_logp_differentiated_twice():
+    from beatsaberrl_amd.autograd_ops import HeadsLogpFn
+
+    def torch_form(x, a):
+        ls = torch.log_softmax(x, -1)
+        return ls.gather(-1, a.unsqueeze(-1)).squeeze(-1).sum(-1), -(ls.exp() * ls).sum(-1).sum(-1)
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(5, 29, 7, generator=g, device=DEV).transpose(0, 1).contiguous().transpose(0, 1).requires_grad_(True)      # rows out of order
+    a, w, u = (torch.randint(0, 7, (5, 29), generator=g, device=DEV), torch.randn(2, 5, generator=g, device=DEV),
+               torch.randn(5, 29, 7, generator=g, device=DEV))
+    out = []
+    for f in (lambda x, a: HeadsLogpFn.apply(x, a)[:2], torch_form):
+        lp, ent = f(x, a)
+        d, = torch.autograd.grad((w[0] * lp + w[1] * ent).sum(), x, create_graph=True)
+        d1, = torch.autograd.grad(lp.sum(), x, retain_graph=True)
+        out.append((d.detach(), d1, torch.autograd.grad((d * u).sum(), x, retain_graph=True)[0],
+                    torch.autograd.grad(lp, x, torch.eye(5, device=DEV), retain_graph=True, is_grads_batched=True)[0]))
+    for got, want in zip(*out):
+        assert torch.allclose(got, want, atol=1e-5)
