@@ -301,13 +301,21 @@ def _plain_eager(*ts) -> bool:
             and all(type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_legacy_batchedtensor(t) for t in ts))
 
 
+def heads_logp(logits, action):
+    """(logprob, entropy, per-head entropy) of given actions, in torch ops."""
+    logsm = torch.log_softmax(logits, dim=-1)
+    ent_h = -(logsm.exp() * logsm).sum(-1)
+    return logsm.gather(-1, action.unsqueeze(-1)).squeeze(-1).sum(-1), ent_h.sum(-1), ent_h.detach()
+
+
 class HeadsLogpFn(torch.autograd.Function):
-    """(logprob, entropy, per-head entropy) of given actions on fp32 logits (B, n_heads, K): the sampling kernel's evaluation
-    forward, one kernel back.  The per-head entropy carries no gradient.  A backward that is itself differentiated is torch's."""
+    """`heads_logp` on fp32 logits (B, n_heads, K) and one action per head: the sampling kernel's evaluation forward, one kernel
+    back.  An action outside its head makes log-probability and gradient of its env NaN: torch's gather would refuse it, and
+    nothing here waits for the device.  A backward that is itself differentiated is torch's."""
 
     @staticmethod
     def forward(ctx, logits, action):
-        _, logprob, entropy, ent_h, _ = ops.sample_heads(logits.contiguous(), action=action.contiguous(), want_ent_h=True)
+        _, logprob, entropy, ent_h, _ = ops.sample_heads(logits.contiguous(), action=action.contiguous(), want_ent_h=True, strict=True)
         ctx.save_for_backward(logits, action)
         ctx.mark_non_differentiable(ent_h)
         ctx.set_materialize_grads(False)

@@ -24,13 +24,13 @@ __global__ __launch_bounds__(256) void heads_logp_bwd_kernel(const float* __rest
     const float ls = logf(s), gl = glp ? glp[env] : 0.f, ge = gent ? gent[env] : 0.f;
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) if (k < K) { v[k] = (v[k] - m) - ls; ent -= expf(v[k]) * v[k]; }
-    int64_t act = action[row];
-    act = act < 0 ? 0 : (act >= K ? K - 1 : act);            // clamped into the row, as in the sampling kernel
+    const int64_t act = action[row];
+    const float hit = act < 0 || act >= K ? NAN : 1.f;       // an action outside its head has no log-probability
 #pragma unroll
     for (int k = 0; k < KMAX; ++k)
         if (k < K) {
             const float p = expf(v[k]);
-            dlogits[row * K + k] = gl * ((k == act ? 1.f : 0.f) - p) - ge * p * (v[k] + ent);
+            dlogits[row * K + k] = gl * ((k == act ? 1.f : hit - 1.f) - p) - ge * p * (v[k] + ent);
         }
 }
 

@@ -69,10 +69,12 @@ __global__ __launch_bounds__(256) void sample_heads_kernel(SampleArgs a) {
 #pragma unroll
         for (int k = 0; k < KMAX; ++k) v[k] = (v[k] - m) - ls;          // log-softmax (lanes >= K: -inf, never read)
         int act;
+        bool outside = false;
         if (a.action_in) {
-            act = a.action_in_u8 ? (int)static_cast<const uint8_t*>(a.action_in)[row]
-                                 : (int)static_cast<const int64_t*>(a.action_in)[row];
-            act = act < 0 ? 0 : (act >= K ? K - 1 : act);               // out-of-range actions are clamped into the row (documented in bsrl.h): never index out of it
+            const int64_t in = a.action_in_u8 == 1 ? (int64_t)static_cast<const uint8_t*>(a.action_in)[row]
+                                                   : static_cast<const int64_t*>(a.action_in)[row];
+            outside = a.action_in_u8 == 2 && (in < 0 || in >= K);
+            act = in < 0 ? 0 : (in >= K ? K - 1 : (int)in);             // never index out of the row (documented in bsrl.h)
         } else {
             const int nvalid = a.head_sizes ? a.head_sizes[h] : K;
             uint32_t r[8];
@@ -104,6 +106,7 @@ __global__ __launch_bounds__(256) void sample_heads_kernel(SampleArgs a) {
             if (k == act) lp = v[k];
             if (k < K) { const float p = expf(v[k]); ent -= p * v[k]; }
         }
+        if (outside) lp = NAN;
         if (a.ent_h) a.ent_h[row] = ent;
     }
     s_lp[e][h] = lp; s_ent[e][h] = ent;
@@ -140,6 +143,7 @@ extern "C" int bsrl_sample_heads(const float* logits, int64_t B, int64_t n_heads
     if (B < 0 || n_heads < 1 || n_heads > 32 || K < 1 || K > KMAX)
         BSRL_FAIL(BSRL_EINVAL, "bsrl_sample_heads: need B >= 0, 1 <= n_heads <= 32, 1 <= K <= %d", KMAX);
     if (!action_in && !action_out) BSRL_FAIL(BSRL_EINVAL, "bsrl_sample_heads: sampling needs action_out");
+    if (action_in_u8 < 0 || action_in_u8 > 2) BSRL_FAIL(BSRL_EINVAL, "bsrl_sample_heads: action_in_u8 must be 0, 1 or 2");
     if (B == 0) return BSRL_OK;
     SampleArgs a{logits, B, (int)n_heads, (int)K, head_sizes, exp_noise, seed, offset, offset_dev, action_in, action_in_u8,
                  action_out, logprob, entropy, ent_h, noise_out};

@@ -749,12 +749,13 @@ def note_frontend(obs, saber_idx, body_idx, dtype, note_geo=False, flux=False, z
 
 
 def sample_heads(logits, head_sizes=None, exp_noise=None, seed=0, offset=0, action=None,
-                 need_entropy=True, want_ent_h=False, want_noise=False, counter=None, validate_action=False):
+                 need_entropy=True, want_ent_h=False, want_noise=False, counter=None, validate_action=False, strict=False):
     """Action epilogue on fp32 logits (B, n_heads, K).  action=None samples (Gumbel-max with the
     caller's Exp(1) draws `exp_noise`, or the kernel's Philox stream keyed by (seed, offset));
     otherwise evaluates the given (B, n_heads) int64 / uint8 actions.  counter: a one-element
     int64 device tensor whose value is added to `offset` on the device and advanced by one after
-    a sampling launch (a captured launch then draws fresh noise on every replay).
+    a sampling launch (a captured launch then draws fresh noise on every replay).  strict: a given int64 action outside
+    [0, K) makes its env's log-probability NaN instead of being clamped.
     Returns (action int64, logprob, entropy | None, ent_h | None, noise | None)."""
     _need_cuda(logits, head_sizes, exp_noise, action)
     if logits.dtype is not torch.float32 or logits.dim() != 3 or not logits.is_contiguous():
@@ -770,7 +771,7 @@ def sample_heads(logits, head_sizes=None, exp_noise=None, seed=0, offset=0, acti
     if action is not None:
         if action.shape != (B, NH) or action.dtype not in (torch.int64, torch.uint8) or not action.is_contiguous():
             raise TypeError("sample_heads: action must be a contiguous (B, n_heads) int64 or uint8 tensor")
-        u8 = int(action.dtype is torch.uint8)
+        u8 = 1 if action.dtype is torch.uint8 else 2 if strict else 0
         if validate_action:             # a host round trip (synchronises): off on the rollout / captured paths
             lo, hi = int(action.min()), int(action.max())
             if lo < 0 or hi >= K:

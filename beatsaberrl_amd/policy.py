@@ -44,7 +44,7 @@ from . import _lib
 from . import fp16_linear as _fl
 from . import obs_layout as L
 from . import ops
-from .autograd_ops import AttnPackedFn, AttnQKVFn, ChainFn, FusedFfnFn, HeadsLogpFn, HlLossFn, LinearFn, LnResFn, NoteTrainFn, NoteTrainPlan, _plain_eager
+from .autograd_ops import AttnPackedFn, AttnQKVFn, ChainFn, FusedFfnFn, HeadsLogpFn, HlLossFn, LinearFn, LnResFn, NoteTrainFn, NoteTrainPlan, _plain_eager, heads_logp
 from .fused_ln import FusedLayerNorm
 
 OBS_DIM = L.OBS_DIM
@@ -982,7 +982,10 @@ class NotePolicy(nn.Module):
         generator, the stream the reference rides."""
         if torch.is_grad_enabled() and action is not None:
             logits, value = self.forward_stacked(obs)
-            logprob, entropy, ent_h = HeadsLogpFn.apply(logits, action.long())
+            action_l = action.long()
+            # one action per head, beside the logits: the kernels; other shapes are torch's, with its broadcasting and errors
+            fits = action_l.shape == logits.shape[:2] and action_l.device == logits.device
+            logprob, entropy, ent_h = (HeadsLogpFn.apply if fits else heads_logp)(logits, action_l)
             if need_entropy:
                 # carries no gradient: the stash outlives the backward and must not pin the micro-batch's autograd graph
                 # (reference python/policy.py:1509-1515)

@@ -434,10 +434,10 @@ int bsrl_note_frontend_padded(const void* obs, int64_t obs_ld, int obs_dtype,
  * a graph draws fresh noise on each replay once bsrl_counter_add follows it on
  * the stream (the part torch's graph-registered generator offset plays in the
  * reference's captured rollout, python/rollout_graph.py:43-78).  noise_out, if
- * not NULL, receives the E used.  Evaluation (action_in != NULL, int64 or uint8 when action_in_u8):
- * no sampling; action_out may be NULL.  A given action outside [0, K) is clamped into the row (the
- * reference's torch.gather would raise): validate on the host where that matters - no entry point
- * synchronises, so the kernel cannot report it.
+ * not NULL, receives the E used.  Evaluation (action_in != NULL: int64 when action_in_u8 is 0 or 2,
+ * uint8 when it is 1): no sampling; action_out may be NULL.  A given action outside [0, K), for which the
+ * reference's torch.gather would raise, makes its env's log-probability NaN when action_in_u8 is 2 and is
+ * clamped into the row otherwise: no entry point synchronises, so the kernel cannot report it.
  * Outputs: action_out (B, n_heads) int64; logprob (B); entropy (B) or NULL;
  * ent_h (B, n_heads) or NULL. */
 int bsrl_sample_heads(const float* logits, int64_t B, int64_t n_heads, int64_t K,
@@ -636,7 +636,7 @@ int bsrl_note_train_backward(const bsrl_note_desc* desc, const float* const* par
 
 /* ---- update losses ---------------------------------------------------------------
  * bsrl_heads_logp_bwd: dlogits (B, n_heads, K) of sum_b glp[b] logprob[b] + gent[b] entropy[b], the summed
- * log-probability of `action` (B, n_heads, int64; clamped into [0, K)) and summed entropy of the heads that
+ * log-probability of `action` (B, n_heads, int64; outside [0, K): NaN) and summed entropy of the heads that
  * bsrl_sample_heads evaluates; glp / gent (B) or NULL (zero).  K <= 8.
  * bsrl_hl_loss: HL-Gauss critic loss per row (python/policy.py:759-781): target = the mass of N(v_tgt, sigma^2)
  * in n equally spaced bins, v_tgt clamped into the support, renormalised; loss (B) = its cross-entropy with

@@ -92,3 +92,31 @@ def test_heads_logp_differentiated_twice():
                     torch.autograd.grad(lp, x, torch.eye(5, device=DEV), retain_graph=True, is_grads_batched=True)[0]))
     for got, want in zip(*out):
         assert torch.allclose(got, want, atol=1e-5)
+
+
+@pytest.mark.parametrize("bad", [-1, 5, 2 ** 32 + 1, -2 ** 40])
+def test_update_of_an_action_outside_its_head(bad):
+    """NaN log-probability and gradient for that env alone; fewer rows of actions are torch's case, as before the kernels."""
+    from beatsaberrl_amd.autograd_ops import HeadsLogpFn
+    x = torch.randn(6, 29, 5, device=DEV, requires_grad=True)
+    a = torch.randint(0, 5, (6, 29), device=DEV)
+    a[2, 11] = bad
+    lp, ent, _ = HeadsLogpFn.apply(x, a)
+    assert torch.isnan(lp).tolist() == [i == 2 for i in range(6)] and torch.isfinite(ent).all()
+    g, = torch.autograd.grad(lp.sum() + ent.sum(), x)
+    assert torch.isnan(g[2, 11]).all() and torch.isnan(g).sum() == 5
+
+
+def test_update_actions_of_other_shapes():
+    from beatsaberrl_amd.policy import NotePolicy
+    from oracle import note_policy_ref as nr
+    m = NotePolicy(embed=128, trunk_dim=64, n_blocks=1, n_heads=4, n_gears=5).to(DEV)
+    m.fp16 = True
+    obs, a = torch.randn(6, nr.OBS_DIM, device=DEV), torch.randint(0, 5, (6, 29), device=DEV)
+    _, lp, ent, _ = m.get_action_and_value(obs, a)
+    _, lp4, ent4, _ = m.get_action_and_value(obs, a[:4])
+    assert lp4.shape == (4,) and torch.allclose(lp4, lp[:4], atol=1e-5) and torch.allclose(ent4, ent, atol=1e-5)
+    assert lp4.requires_grad
+    for wrong in (a.cpu(), a[:, :, None].expand(6, 29, 2), torch.zeros(7, 29, device=DEV)):
+        with pytest.raises((RuntimeError, TypeError)):
+            m.get_action_and_value(obs, wrong)
