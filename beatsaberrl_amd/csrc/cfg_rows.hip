@@ -11,10 +11,14 @@ struct Bump {
     void* take(size_t n) { void* r = p ? p + used : nullptr; used += (n + 255) & ~(size_t)255; return r; }
 };
 
+// d = 256 keeps the residual stream fp32 between the kernels in either form: the block-stack kernel, which smaller batches of
+// the model take, keeps it in fp32 registers, and no batch size lowers the precision
+bool stream_f32(const bsrl_cfg_desc& d) { return d.d == 256 && d.dtype != BSRL_F32; }
+
 struct RowsPlan {
     int32_t* noff; void *x0, *x1, *h, *q, *att, *hid, *lead; size_t bytes;
     RowsPlan(const bsrl_cfg_desc& d, int64_t B, bool tail, char* ws) {
-        const size_t es = d.dtype == BSRL_F32 ? 4 : 2, R = (size_t)B * d.T, D = d.d, xs = tail && d.d == 256 ? 4 : es;
+        const size_t es = d.dtype == BSRL_F32 ? 4 : 2, R = (size_t)B * d.T, D = d.d, xs = stream_f32(d) ? 4 : es;
         Bump b{ws};
         noff = static_cast<int32_t*>(b.take((B + 1) * 4));
         x0 = b.take(R * D * xs);
@@ -56,9 +60,11 @@ extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows
     int rc;
 #define STEP(call) do { if ((rc = (call)) != BSRL_OK) return rc; } while (0)
     auto at = [&](const void* q, int64_t elems) { return static_cast<const char*>(q) + elems * es; };
-    // y = act(x W^T + b) (+ res) on rows [+ *extra] rows
-    auto linear = [&](const void* x, int64_t ldx, const void* W, const float* b, const void* res, void* y, int64_t K, int64_t M, int a_, bool all) {
-        LinArgs a{x, ldx, W, b, res, D, y, M, nullptr, 0, 0, all ? R : B, (int)K, (int)M, 0, 0, 0, nullptr, 0};
+    // y = act(x W^T + b) (+ res) on rows [+ *extra] rows; res_f32, y_f32: that operand is fp32
+    auto linear = [&](const void* x, int64_t ldx, const void* W, const float* b, const void* res, void* y, int64_t K, int64_t M, int a_, bool all,
+                      bool res_f32 = false, bool y_f32 = false) {
+        LinArgs a{x, ldx, W, b, res, D, y, M, nullptr, 0, 0, all ? R : B, (int)K, (int)M, y_f32, 0, 0, nullptr, 0};
+        a.res_f32 = res_f32;
         if (all) { a.extra = extra; a.base = B; }
         if (!bsrl_linear_small(a, a_, dt, st)) return (int)BSRL_UNSUPPORTED;
         const hipError_t e = hipGetLastError();
@@ -69,16 +75,16 @@ extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows
     STEP(bsrl_cfg_tokens(obs, obs_ld, obs_dtype, w->prop_w, w->prop_b, w->obj_w, w->obj_b, p.noff, p.x0, B, D, d->prop_dim, d->obj_dim, dt, stream));
     const float eps = 1e-5f;
     void *x = p.x0, *xn = p.x1;
-    const bool f32s = tail && D == 256;         // the residual stream stays fp32 between blocks, as in the block-stack kernel
+    const bool f32s = stream_f32(*d);
     auto next_cols = [&](int i) { return prune && i + 1 == L ? 2 * D : 3 * D; };      // the final block projects keys and values only
     if (tail) STEP(bsrl_block_tail(w->lead_img, nullptr, x, nullptr, nullptr, 0.f, w->blk[0].ln_attn_w, w->blk[0].ln_attn_b, eps, nullptr,
                                    next_cols(0) == 2 * D ? p.h : nullptr, B, p.q, next_cols(0), B, extra, R - B, D, 0, act, dt, 0, stream));
     for (int i = 0; i < L; ++i) {
         const auto& k = w->blk[i];
-        const bool pruned = prune && i + 1 == L;
+        const bool pruned = prune && i + 1 == L, xf = f32s && i > 0, last = i + 1 == L;      // xf: this block's rows come in as fp32
         const int64_t qn = next_cols(i);
         if (!tail) {
-            STEP(bsrl_ln_rows(x, D, k.ln_attn_w, k.ln_attn_b, p.h, D, nullptr, nullptr, B, extra, R, D, eps, dt, stream));
+            STEP(bsrl_ln_rows(x, D, k.ln_attn_w, k.ln_attn_b, p.h, D, nullptr, nullptr, B, extra, R, D, eps, dt, stream, xf));
             STEP(linear(p.h, D, at(k.qkv_w, (3 * D - qn) * D), k.qkv_b + (3 * D - qn), nullptr, p.q, D, qn, BSRL_ACT_NONE, true));
         }
         const void *qp = p.q, *kp = at(p.q, qn - 2 * D), *vp = at(p.q, qn - D);
@@ -92,18 +98,17 @@ extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows
         const int64_t extra_max = pruned ? 0 : R - B;
         const int32_t* ex = pruned ? nullptr : extra;
         if (tail) {
-            const bool last = i + 1 == L;
             const int64_t nn = last ? 0 : next_cols(i + 1);
             const auto* nk = last ? nullptr : &w->blk[i + 1];
-            const int x_f32 = !f32s ? 0 : (i > 0 ? 1 : 0) | (last ? 0 : 2);
+            const int x_f32 = (xf ? 1 : 0) | (f32s && !last ? 2 : 0);
             STEP(bsrl_block_tail(k.tail_img, p.att, x, k.ln_ffn_w, k.ln_ffn_b, eps, nk ? nk->ln_attn_w : nullptr, nk ? nk->ln_attn_b : nullptr, eps,
                                  xn, nn == 2 * D ? p.h : nullptr, B, nn ? p.q : nullptr, nn, B, ex, extra_max, D, F, act, dt, x_f32, stream));
             void* t = x; x = xn; xn = t;
         } else {
-            STEP(linear(p.att, D, k.out_w, k.out_b, x, xn, D, D, BSRL_ACT_NONE, !pruned));
-            STEP(bsrl_ln_rows(xn, D, k.ln_ffn_w, k.ln_ffn_b, p.h, D, nullptr, nullptr, B, ex, B + extra_max, D, eps, dt, stream));
+            STEP(linear(p.att, D, k.out_w, k.out_b, x, xn, D, D, BSRL_ACT_NONE, !pruned, xf, f32s));
+            STEP(bsrl_ln_rows(xn, D, k.ln_ffn_w, k.ln_ffn_b, p.h, D, nullptr, nullptr, B, ex, B + extra_max, D, eps, dt, stream, f32s));
             STEP(linear(p.h, D, k.w0, k.b0, nullptr, p.hid, D, F, act, !pruned));
-            STEP(linear(p.hid, F, k.w2, k.b2, xn, x, F, D, BSRL_ACT_NONE, !pruned));
+            STEP(linear(p.hid, F, k.w2, k.b2, xn, x, F, D, BSRL_ACT_NONE, !pruned, f32s, f32s && !last));
         }
     }
     if (d->final_ln) {

@@ -20,6 +20,7 @@ struct LinArgs {
     // rows counted on the device: base + *extra of them, `rows` their host-side bound (NULL: exactly `rows`)
     const int32_t* extra = nullptr; int64_t base = 0;
     bool vec_ok = false;               // linear_small.hip: filled in by its launch
+    bool res_f32 = false;              // 16-bit operands with an fp32 residual (linear_small.hip alone)
 };
 
 __device__ __forceinline__ int64_t lin_rows(const LinArgs& a) { return a.extra ? a.base + (int64_t)*a.extra : a.rows; }
@@ -61,9 +62,10 @@ bool bsrl_linear_small(const LinArgs& a, int act, int dtype, hipStream_t st);
 // The dispatch behind bsrl_linear / bsrl_linear_gated (linear.hip), for host code that composes forwards and backwards.
 int bsrl_linear_run(const LinArgs& a, int act, int dtype, int out_dtype, hipStream_t st, const char* what);
 
-// LayerNorm of rows + *extra rows (ln.hip; `bound`: their host-side bound) at row pitches ldx, ldy; mean, rstd optional
+// LayerNorm of rows + *extra rows (ln.hip; `bound`: their host-side bound) at row pitches ldx, ldy; mean, rstd optional;
+// x_f32: x is fp32 whatever dtype is y's
 int bsrl_ln_rows(const void* x, int64_t ldx, const float* w, const float* b, void* y, int64_t ldy, float* mean, float* rstd, int64_t rows, const int32_t* extra,
-                 int64_t bound, int64_t d, float eps, int dtype, bsrl_stream stream);
+                 int64_t bound, int64_t d, float eps, int dtype, bsrl_stream stream, bool x_f32 = false);
 
 // The backward side over device-counted rows, for host code that composes a backward (ln_bwd.hip, wgrad.hip, attn_bwd.hip)
 int bsrl_ln_bwd_rows(const void* x, const void* dy, const float* weight, const float* mean, const float* rstd, const void* gx,

@@ -56,7 +56,7 @@ __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, i
             for (int e = 0; e < 4; ++e) o[e] = keep_f32(Mma<DT>::template act<ACT>(acc[i][j][e] + bv[e], f32out));
             if (a.vec_ok) {               // M % 4 == 0, aligned rows, no split: 8- / 16-byte pieces
                 if (a.res) {
-                    if (ES == 4) {
+                    if (ES == 4 || a.res_f32) {
                         const float4 r = *reinterpret_cast<const float4*>(static_cast<const float*>(a.res) + row * a.ldr + col);
                         o[0] += r.x; o[1] += r.y; o[2] += r.z; o[3] += r.w;
                     } else {
@@ -82,7 +82,7 @@ __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, i
                     const int c = col + e;
                     if (c >= a.M) break;
                     float v = o[e];
-                    if (a.res) v += Mma<DT>::ld(a.res, row * a.ldr + c);
+                    if (a.res) v += a.res_f32 ? static_cast<const float*>(a.res)[row * a.ldr + c] : Mma<DT>::ld(a.res, row * a.ldr + c);
                     if (a.gate && !(Mma<DT>::ld(a.gate, row * a.ldgate + c) > 0.f)) v = 0.f;
                     const bool second = a.y2 && c >= a.split;
                     void* dst = second ? a.y2 : a.y;
@@ -280,7 +280,7 @@ bool bsrl_linear_small(const LinArgs& a_, int act, int dtype, hipStream_t st) {
     if (((a.rows + 31) / 32) * (int64_t)((a.M + 31) / 32) > 0x3fffffff) return false;
     const int osz = a.out_f32 ? 4 : es;
     a.vec_ok = !a.y2 && a.M % 4 == 0 && a.ldy % 4 == 0 && a.y_gstride % 4 == 0 && bsrl_aligned(a.y, 4 * osz) &&
-               (!a.res || (a.ldr % 4 == 0 && bsrl_aligned(a.res, 4 * es))) && (!a.gate || (a.ldgate % 4 == 0 && bsrl_aligned(a.gate, 4 * es)));
+               (!a.res || (a.ldr % 4 == 0 && bsrl_aligned(a.res, a.res_f32 ? 16 : 4 * es))) && (!a.gate || (a.ldgate % 4 == 0 && bsrl_aligned(a.gate, 4 * es)));
     if (dtype == BSRL_F32) by_act<F32IO>(a, act, st);
     else if (dtype == BSRL_F16) by_act<F16>(a, act, st);
     else by_act<BF16>(a, act, st);

@@ -13,7 +13,8 @@
 
 namespace {
 
-template <typename IO, int LPR, int NCH, bool ADD>
+// XF32: the rows come in as fp32 (a 16-bit stream's fp32 residual)
+template <typename IO, int LPR, int NCH, bool ADD, bool XF32>
 __global__ __launch_bounds__(256) void ln_kernel(const void* __restrict__ a, const void* __restrict__ b,
                                                  const float* __restrict__ bb, const float* __restrict__ w,
                                                  const float* __restrict__ bias, void* __restrict__ xo,
@@ -38,7 +39,10 @@ __global__ __launch_bounds__(256) void ln_kernel(const void* __restrict__ a, con
 #pragma unroll
         for (int j = 0; j < VEC; ++j) v[c][j] = 0.f;
         if (on) {
-            io::load(a, row * lda + e0, v[c]);
+            if constexpr (XF32) {
+#pragma unroll
+                for (int j = 0; j < VEC; j += 4) LnIO<F32IO>::load(a, row * lda + e0 + j, v[c] + j);
+            } else io::load(a, row * lda + e0, v[c]);
             if (ADD) {
                 float t[VEC];
                 io::load(b, base + e0, t);
@@ -83,20 +87,21 @@ __global__ __launch_bounds__(256) void ln_kernel(const void* __restrict__ a, con
 }
 
 template <typename IO, int LPR, int NCH>
-void launch(bool add, const void* a, const void* b, const float* bb, const float* w, const float* bias,
+void launch(bool add, bool xf32, const void* a, const void* b, const float* bb, const float* w, const float* bias,
             void* x, void* y, float* mean, float* rstd, int64_t rows, int d, float eps, hipStream_t st, const int32_t* extra, int64_t bound, int64_t lda, int64_t ldy) {
     constexpr int RPB = 4 * (WAVE / LPR);
     const unsigned grid = (unsigned)((bound + RPB - 1) / RPB);
-    if (add) hipLaunchKernelGGL((ln_kernel<IO, LPR, NCH, true>), dim3(grid), dim3(256), 0, st, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, extra, lda, ldy);
-    else hipLaunchKernelGGL((ln_kernel<IO, LPR, NCH, false>), dim3(grid), dim3(256), 0, st, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, extra, lda, ldy);
+    auto kern = add ? ln_kernel<IO, LPR, NCH, true, false> : ln_kernel<IO, LPR, NCH, false, false>;
+    if constexpr (LnIO<IO>::VEC == 8) if (xf32) kern = ln_kernel<IO, LPR, NCH, false, true>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, extra, lda, ldy);
 }
 
 template <typename IO>
-int dispatch(bool add, const void* a, const void* b, const float* bb, const float* w, const float* bias,
+int dispatch(bool add, bool xf32, const void* a, const void* b, const float* bb, const float* w, const float* bias,
              void* x, void* y, float* mean, float* rstd, int64_t rows, int64_t d, float eps, hipStream_t st, const int32_t* extra, int64_t bound, int64_t lda, int64_t ldy) {
     constexpr int VEC = LnIO<IO>::VEC;
     const int c16 = 16 * VEC, c32 = 32 * VEC, c64 = 64 * VEC;
-#define LN_GO(LPR, NCH) do { launch<IO, LPR, NCH>(add, a, b, bb, w, bias, x, y, mean, rstd, rows, (int)d, eps, st, extra, bound, lda, ldy); return BSRL_OK; } while (0)
+#define LN_GO(LPR, NCH) do { launch<IO, LPR, NCH>(add, xf32, a, b, bb, w, bias, x, y, mean, rstd, rows, (int)d, eps, st, extra, bound, lda, ldy); return BSRL_OK; } while (0)
     if (d <= c16) LN_GO(16, 1);
     if (d <= 2 * c16 && d % c16 == 0) LN_GO(16, 2);
     if (d <= c32) LN_GO(32, 1);
@@ -112,7 +117,7 @@ int dispatch(bool add, const void* a, const void* b, const float* bb, const floa
 
 int ln_entry(bool add, const void* a, const void* b, const float* bb, const float* w, const float* bias,
              void* x, void* y, float* mean, float* rstd, int64_t rows, int64_t d, float eps, int dtype,
-             bsrl_stream stream, const int32_t* extra = nullptr, int64_t bound = -1, int64_t lda = -1, int64_t ldy = -1) {
+             bsrl_stream stream, const int32_t* extra = nullptr, int64_t bound = -1, int64_t lda = -1, int64_t ldy = -1, bool xf32 = false) {
     if (bound < 0) bound = rows;
     if (lda < 0) lda = d;
     if (ldy < 0) ldy = d;
@@ -127,9 +132,9 @@ int ln_entry(bool add, const void* a, const void* b, const float* bb, const floa
         return BSRL_UNSUPPORTED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int rc;
-    if (dtype == BSRL_F32) rc = dispatch<F32IO>(add, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
-    else if (dtype == BSRL_F16) rc = dispatch<F16>(add, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
-    else rc = dispatch<BF16>(add, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
+    if (dtype == BSRL_F32) rc = dispatch<F32IO>(add, xf32, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
+    else if (dtype == BSRL_F16) rc = dispatch<F16>(add, xf32, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
+    else rc = dispatch<BF16>(add, xf32, a, b, bb, w, bias, x, y, mean, rstd, rows, d, eps, st, extra, bound, lda, ldy);
     if (rc == BSRL_OK) BSRL_CHECK_LAUNCH(what);
     return rc;
 }
@@ -137,8 +142,8 @@ int ln_entry(bool add, const void* a, const void* b, const float* bb, const floa
 }  // namespace
 
 int bsrl_ln_rows(const void* x, int64_t ldx, const float* w, const float* b, void* y, int64_t ldy, float* mean, float* rstd, int64_t rows, const int32_t* extra,
-                 int64_t bound, int64_t d, float eps, int dtype, bsrl_stream stream) {
-    return ln_entry(false, x, nullptr, nullptr, w, b, nullptr, y, mean, rstd, rows, d, eps, dtype, stream, extra, bound, ldx, ldy);
+                 int64_t bound, int64_t d, float eps, int dtype, bsrl_stream stream, bool x_f32) {
+    return ln_entry(false, x, nullptr, nullptr, w, b, nullptr, y, mean, rstd, rows, d, eps, dtype, stream, extra, bound, ldx, ldy, x_f32 && dtype != BSRL_F32);
 }
 
 extern "C" int bsrl_ln_fwd(const void* x, const float* weight, const float* bias, void* y, float* mean,
