@@ -36,8 +36,8 @@ _ffn_mode = "off"
 
 
 def bump_weights_version():
-    """Call after every in-place update of the fp32 masters (optimizer step, load):
-    16-bit replicas are recast, in place, on their next use."""
+    """Call after every in-place update of the fp32 masters (optimizer step, load) and after a module that holds some was
+    replaced: 16-bit replicas and images are recast, in place, on their next use."""
     global _weights_version
     _weights_version += 1
 

@@ -569,8 +569,9 @@ class NotePolicy(nn.Module):
                 with torch.no_grad():
                     r_out, r_value = self.forward_stacked(obs)       # the rollout's own routes, grad-free
                 plan = self._train_plan()
-                if plan is not None:
-                    return self._forward_train_native(plan, obs, r_out, r_value)
+                params = None if plan is None else self._train_params()
+                if params is not None and [p.shape for p in params] == plan.param_shapes and all(p.is_cuda for p in params):
+                    return self._forward_train_native(plan, params, obs, r_out, r_value)
                 out, value = self._forward_train(obs)
                 return _ValuesOf.apply(out, r_out), _ValuesOf.apply(value, r_value)
             return self._forward_train(obs)
@@ -582,34 +583,66 @@ class NotePolicy(nn.Module):
             return self._forward_stacked(obs)
 
     # ---- the fused routes as native calls ------------------------------------------------------
-    def _note_desc(self, dt):
-        return dict(n_blocks=len(self.blocks), d=self.embed, n_heads=self.n_heads, ffn=self.blocks[0].ffn[0].out_features,
-                    trunk=self.trunk_proj.out_features, hidden=self.trunk_fc1.out_features, n_gears=self.k_max, bins=self.value_bins,
-                    note_geo=self.note_geo, flux=self.game == "flux", dtype=ops.dt_code(dt), z_asinh=self.z_asinh)
+    def _native_desc(self, dt):
+        """What bsrl_note_* are told of the architecture, or None where the modules hold something that those calls do not
+        compute as the op-by-op forward would: an architecture option, another eps or activation."""
+        if self.value_residual or self.emb_ln is not None or self.final_ln is not None or self.trunk_arch != "simba":
+            return None
+        M = self._modules                          # the dicts themselves: a lookup by attribute or index costs several times this walk
+        try:
+            for k in ("trunk_ln1", "trunk_ln2", "critic_ln"):
+                if M[k].eps != 1e-5:
+                    return None
+            seqs = [M[k]._modules for k in ("saber_mlp", "torso_mlp", "leg_mlp", "note_mlp")]
+            for b in M["blocks"]._modules.values():
+                m = b._modules
+                if type(b) is not Block or m["ln_attn"].eps != 1e-5 or m["ln_ffn"].eps != 1e-5:
+                    return None
+                seqs.append(m["ffn"]._modules)
+            mlp = M["critic_mlp"]._modules
+            if (any(len(m) != 3 or not isinstance(m["1"], nn.ReLU) for m in seqs)
+                    or len(mlp) != 5 or not isinstance(mlp["1"], nn.ReLU) or not isinstance(mlp["3"], nn.ReLU)):
+                return None
+            return dict(n_blocks=len(seqs) - 4, d=self.embed, n_heads=self.n_heads, ffn=seqs[4]["0"].out_features,
+                        trunk=M["trunk_proj"].out_features, hidden=M["trunk_fc1"].out_features, n_gears=self.k_max, bins=self.value_bins,
+                        note_geo=self.note_geo, flux=self.game == "flux", dtype=ops.dt_code(dt), z_asinh=self.z_asinh)
+        except (KeyError, AttributeError):
+            return None
 
-    def _plain_arch(self):
-        """True for the architecture that the native forward and update are written for."""
-        return (not self.value_residual and self.emb_ln is None and self.final_ln is None and self.trunk_arch == "simba"
-                and all(isinstance(b.ffn[1], nn.ReLU) and b.ln_attn.eps == b.ln_ffn.eps == 1e-5 for b in self.blocks)
-                and self.trunk_ln1.eps == self.trunk_ln2.eps == self.critic_ln.eps == 1e-5)
+    def _native_shapes(self, c):
+        """Shapes of `_train_params` for the descriptor c."""
+        d, ffn, tr, hid = c["d"], c["ffn"], c["trunk"], c["hidden"]
+        lin, ln = lambda m, k: [(m, k), (m,)], lambda n: [(n,), (n,)]
+        out = []
+        for k in (SABER_FEAT + 2, TORSO_FEAT, LEG_FEAT + 2, NOTE_FEAT + (NOTE_GEO_FEAT if c["note_geo"] else 0)):
+            out += lin(d, k) + lin(d, d)
+        out += c["n_blocks"] * (ln(d) + 4 * lin(d, d) + ln(d) + lin(ffn, d) + lin(d, ffn))
+        out += lin(tr, self.n_lead * d) + ln(tr) + lin(hid, tr) + lin(tr, hid) + ln(tr)
+        for k in self.head_sizes:
+            out += lin(k, tr)
+        return out + ln(d) + 4 * lin(d, d) + lin(tr, d + tr) + lin(tr, tr) + lin(c["bins"], tr)
 
     def _native_image(self, dt):
         """(descriptor, weight image) of the native forward for the current weights version, or None where the forward runs op
         by op.  The image is rebuilt IN PLACE, as `blocks_image` is: its address is stable under a captured graph."""
-        if (dt is torch.float32 or not self.fused_blocks_ok(dt) or not self._plain_arch() or not self.critic_pool
+        if (dt is torch.float32 or not self.fused_blocks_ok(dt) or not self.critic_pool
                 or not ops.critic_pool_supported(self.n_lead + N_NOTE_SLOTS, self.embed, self.n_heads, dt)):
             return None
-        dev = self.critic_q.weight.device
+        arch = self._native_desc(dt)
+        if arch is None:
+            return None
+        dev, key = self.critic_ln.weight.device, dt
         c = self._native_cache
-        if c is None or c[1] is not dt or c[2].device != dev:
-            desc = _lib.NoteDesc(**self._note_desc(dt))
+        if c is None or c[1] != key or c[2].device != dev:
+            desc = _lib.NoteDesc(**arch)
             n = _lib.load().bsrl_note_pack_size(desc)
-            c = self._native_cache = [-1, dt, torch.zeros(n, dtype=torch.uint8, device=dev), desc]
+            c = self._native_cache = [-1, key, torch.zeros(n, dtype=torch.uint8, device=dev), desc]
         if c[2].numel() == 0:
             return None
         if c[0] != _fl._weights_version:
             params = self._train_params()
-            if any(p.dtype is not torch.float32 or not p.is_contiguous() for p in params):
+            if params is None or [p.shape for p in params] != self._native_shapes(arch) or any(
+                    p.dtype is not torch.float32 or not p.is_contiguous() or p.device != dev for p in params):
                 return None
             ptrs = (ctypes.c_void_p * len(params))(*[p.data_ptr() for p in params])
             gears = (ctypes.c_int32 * N_ACTION_HEADS)(*self.head_sizes)
@@ -623,25 +656,40 @@ class NotePolicy(nn.Module):
     def _overlaps(self, B):
         return B >= (2048 if self.critic_overlap_min_batch is None else self.critic_overlap_min_batch)
 
-    def _forward_native(self, desc, image, obs):
+    def _native_masters(self, c):
+        """What the native forward's kernels read from the masters themselves - the encoder, trunk and critic biases, the trunk
+        and critic LayerNorms - in bsrl_note_train_forward's order; None where one of them is not what they take."""
+        M, i_trunk = self._modules, 16 + 16 * c.n_blocks
+        i_critic = i_trunk + 10 + 2 * N_ACTION_HEADS
+        d, tr = c.d, c.trunk
+        at = []
+        for e, k in enumerate(("saber_mlp", "torso_mlp", "leg_mlp", "note_mlp")):
+            m = M[k]._modules
+            at += ((4 * e, m["0"], d), (4 * e + 2, m["2"], d))
+        mlp = M["critic_mlp"]._modules
+        for i, k, n in ((0, "trunk_proj", tr), (2, "trunk_ln1", tr), (4, "trunk_fc1", c.hidden), (6, "trunk_fc2", tr), (8, "trunk_ln2", tr)):
+            at.append((i_trunk + i, M[k], n))
+        for i, m, n in ((0, M["critic_ln"], d), (2, M["critic_q"], d), (4, M["critic_k"], d), (6, M["critic_v"], d), (8, M["critic_out"], d),
+                        (10, mlp["0"], tr), (12, mlp["2"], tr), (14, mlp["4"], c.bins)):
+            at.append((i_critic + i, m, n))
+        params = (ctypes.c_void_p * (i_critic + 16))()
+        lns = (i_trunk + 2, i_trunk + 8, i_critic)
+        for i, m, n in at:
+            for j, k in enumerate(("weight", "bias")):
+                if j or i in lns:
+                    p = m._parameters.get(k)
+                    if p is None or p.dtype is not torch.float32 or p.numel() != n or not p.is_cuda or not p.is_contiguous():
+                        return None
+                    params[i + j] = p.data_ptr()
+        return params
+
+    def _forward_native(self, desc, image, params, obs):
         """_forward_stacked on the fused routes: one call, or its four parts with the critic on the second stream."""
         lib, B, dev = _lib.load(), obs.shape[0], obs.device
         logits = torch.empty(B, N_ACTION_HEADS, self.k_max, dtype=torch.float32, device=dev)
         value = torch.empty(B, dtype=torch.float32, device=dev)
         n = lib.bsrl_note_forward_size(desc, B)
         ws = torch.empty(n, dtype=torch.uint8, device=dev)
-        # what the kernels read from the masters: encoder, trunk and critic biases, trunk and critic LayerNorms
-        i_trunk = 16 + 16 * len(self.blocks)
-        i_critic = i_trunk + 10 + 2 * N_ACTION_HEADS
-        params = (ctypes.c_void_p * (i_critic + 16))()
-        for e, seq in enumerate((self.saber_mlp, self.torso_mlp, self.leg_mlp, self.note_mlp)):
-            params[4 * e + 1], params[4 * e + 3] = seq[0].bias.data_ptr(), seq[2].bias.data_ptr()
-        mlp = self.critic_mlp
-        for at, ms in ((i_trunk, (self.trunk_proj, self.trunk_ln1, self.trunk_fc1, self.trunk_fc2, self.trunk_ln2)),
-                       (i_critic, (self.critic_ln, self.critic_q, self.critic_k, self.critic_v, self.critic_out, mlp[0], mlp[2], mlp[4]))):
-            for i, m in enumerate(ms):
-                p = m._parameters
-                params[at + 2 * i], params[at + 2 * i + 1] = p["weight"].data_ptr(), p["bias"].data_ptr()
         args = (desc, params, image.data_ptr(), obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype), self._saber_idx32.data_ptr(),
                 self._body_idx32.data_ptr(), self.value_centers.data_ptr(), logits.data_ptr(), value.data_ptr(), B)
 
@@ -670,10 +718,11 @@ class NotePolicy(nn.Module):
         B, d = obs.shape[0], self.embed
         if obs.shape[0]:
             native = self._native_image(dt)
-            if native is not None:
+            masters = None if native is None else self._native_masters(native[0])
+            if masters is not None:
                 if obs.dtype is not torch.float32 and obs.dtype is not dt:
                     obs = obs.float()
-                return self._forward_native(*native, obs if obs.stride(1) == 1 else obs.contiguous())
+                return self._forward_native(*native, masters, obs if obs.stride(1) == 1 else obs.contiguous())
         # preamble in one kernel: the obs is rounded once to the stream dtype (policy.py:1200-1209),
         # gathered into the four encoder inputs (+ note-geometry lanes, one-hots) and the key bias
         if obs.dtype is not torch.float32 and obs.dtype is not dt:
@@ -799,8 +848,9 @@ class NotePolicy(nn.Module):
         return out.view(B, N_ACTION_HEADS, self.k_max), value
 
     def _train_params(self):
-        """The trained tensors in the order of bsrl_note_train_forward's `params`."""
-        M, out = self._modules, []                 # the dicts themselves: a lookup by attribute or index costs several times this walk
+        """The trained tensors in the order of bsrl_note_train_forward's `params`; None where one of them is not a parameter of
+        its module (parametrized or pruned weights, a Linear without a bias, another module in its place)."""
+        M, out = self._modules, []
 
         def add(m):
             p = m._parameters
@@ -812,40 +862,46 @@ class NotePolicy(nn.Module):
             for i in at:
                 add(m[i])
 
-        for k in ("saber_mlp", "torso_mlp", "leg_mlp", "note_mlp"):
-            add_seq(M[k], "0", "2")
-        for b in M["blocks"]._modules.values():
-            m = b._modules
-            for k in ("ln_attn", "q_proj", "k_proj", "v_proj", "out_proj", "ln_ffn"):
-                add(m[k])
-            add_seq(m["ffn"], "0", "2")
-        for k in ("trunk_proj", "trunk_ln1", "trunk_fc1", "trunk_fc2", "trunk_ln2"):
-            add(M[k])
-        for m in M["heads"]._modules.values():
-            add(m)
-        for k in ("critic_ln", "critic_q", "critic_k", "critic_v", "critic_out"):
-            add(M[k])
-        add_seq(M["critic_mlp"], "0", "2", "4")
-        return out
+        try:
+            for k in ("saber_mlp", "torso_mlp", "leg_mlp", "note_mlp"):
+                add_seq(M[k], "0", "2")
+            for b in M["blocks"]._modules.values():
+                m = b._modules
+                for k in ("ln_attn", "q_proj", "k_proj", "v_proj", "out_proj", "ln_ffn"):
+                    add(m[k])
+                add_seq(m["ffn"], "0", "2")
+            for k in ("trunk_proj", "trunk_ln1", "trunk_fc1", "trunk_fc2", "trunk_ln2"):
+                add(M[k])
+            for m in M["heads"]._modules.values():
+                add(m)
+            for k in ("critic_ln", "critic_q", "critic_k", "critic_v", "critic_out"):
+                add(M[k])
+            add_seq(M["critic_mlp"], "0", "2", "4")
+        except KeyError:
+            return None
+        return None if any(p is None for p in out) else out
 
     def _train_plan(self):
-        """The native update's plan, or None where the update runs op by op: architecture options without a place in it, a
-        fused FFN asked for, LayerNorms with another eps."""
-        if not self._plain_arch() or self._gear_idx is not None or self.fused_ffn != "off":
+        """The native update's plan, or None where the update runs op by op: an architecture without a place in it, a fused FFN
+        asked for, parameters of other shapes or kinds."""
+        if self._gear_idx is not None or self.fused_ffn != "off":
             return None
-        c, dt = self._train_plan_cache, self.stream_dtype
-        if c is None or c[0] is not dt:
-            c = self._train_plan_cache = (dt, NoteTrainPlan(self._note_desc(dt), [p.shape for p in self._train_params()]))
+        arch = self._native_desc(self.stream_dtype)
+        if arch is None:
+            return None
+        c, key = self._train_plan_cache, self.stream_dtype
+        if c is None or c[0] != key:
+            c = self._train_plan_cache = (key, NoteTrainPlan(arch, self._native_shapes(arch)))
         return c[1] if c[1].supported else None
 
-    def _forward_train_native(self, plan, obs, r_out, r_value):
+    def _forward_train_native(self, plan, params, obs, r_out, r_value):
         """The update forward as one native call (its backward is another); outputs are the rollout's, see NoteTrainFn."""
         obs = obs.detach()
         if obs.dtype is not torch.float32 and obs.dtype is not self.stream_dtype:
             obs = obs.float()
         if obs.stride(1) != 1:
             obs = obs.contiguous()
-        params = [p if p.dtype is torch.float32 and p.is_contiguous() else p.float().contiguous() for p in self._train_params()]
+        params = [p if p.dtype is torch.float32 and p.is_contiguous() else p.float().contiguous() for p in params]
         out, value, self._value_logits = NoteTrainFn.apply(plan, obs, self._saber_idx32, self._body_idx32, self.value_centers,
                                                            r_out, r_value, *params)
         return out, value

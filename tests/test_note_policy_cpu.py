@@ -98,3 +98,28 @@ def test_hl_loss_kernel_takes_only_what_it_covers():
                  (x[:0], v[:0], c, 0.1), (x[0], v, c, 0.1), (x[:, :1], v, c[:1], 0.1), (x, v, c.double(), 0.1), (x, v, c, 0.0),
                  (x, v, c, torch.tensor(0.1)), (x, v.clone().requires_grad_(), c, 0.1), (torch.randn(4, 513), v, torch.randn(513), 0.1)):
         assert not _hl_kernel_takes(*args)
+
+
+def _small(**kw):
+    return NotePolicy(**{**dict(embed=128, trunk_dim=64, n_blocks=2, n_heads=4, n_gears=5), **kw})
+
+
+def test_native_calls_take_only_parameters_of_the_expected_shapes():
+    from torch import nn
+    from torch.nn.utils import parametrizations
+    for kw in ({}, dict(note_geo=True, trunk_hidden=96, value_bins=51), dict(head_gears=(3,) * 10 + (5,) * 19)):
+        m = _small(**kw)
+        assert [p.shape for p in m._train_params()] == m._native_shapes(m._native_desc(torch.float16))
+    for change in (lambda m: parametrizations.weight_norm(m.trunk_fc1), lambda m: parametrizations.spectral_norm(m.blocks[1].k_proj),
+                   lambda m: setattr(m, "critic_q", nn.Linear(128, 128, bias=False)), lambda m: setattr(m, "critic_out", nn.Identity())):
+        m = _small()
+        change(m)
+        assert m._train_params() is None
+    for change in (lambda m: m.critic_mlp.__setitem__(1, nn.Tanh()), lambda m: m.saber_mlp.append(nn.ReLU()), lambda m: m.blocks[0].ffn.__setitem__(1, nn.GELU()),
+                   lambda m: setattr(m.blocks[1].ln_ffn, "eps", 1e-6), lambda m: delattr(m, "leg_mlp")):
+        m = _small()
+        change(m)
+        assert m._native_desc(torch.float16) is None and m._train_plan() is None
+    m = _small()
+    m.heads[3] = nn.Linear(64, 7)
+    assert [p.shape for p in m._train_params()] != m._native_shapes(m._native_desc(torch.float16))
