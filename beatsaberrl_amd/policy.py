@@ -427,8 +427,8 @@ class NotePolicy(nn.Module):
         # "auto": the 16-bit stream runs the whole block stack as one persistent kernel when the
         # shape has one (ops.blocks_pack_size > 0); "off": always the per-op launch train
         self.fused_blocks = "auto"
-        self._train_plan_cache = None           # (stream dtype, NoteTrainPlan)
-        self._native_cache = None               # [weights version, dtype, uint8 image, descriptor]
+        self._train_plan_cache = None           # (descriptor's values, NoteTrainPlan)
+        self._native_cache = None               # [weights version, descriptor's values, uint8 image, descriptor]
         self._blocks_image = None               # [weights version, dtype, uint8 image]
         # True: the critic's one-query attention runs as a pool over LN(x_res) with the k | v projections folded
         # around it (no (B T, 2d) keys / values); False: the reference's op order
@@ -631,7 +631,7 @@ class NotePolicy(nn.Module):
         arch = self._native_desc(dt)
         if arch is None:
             return None
-        dev, key = self.critic_ln.weight.device, dt
+        dev, key = self.critic_ln.weight.device, tuple(arch.values())
         c = self._native_cache
         if c is None or c[1] != key or c[2].device != dev:
             desc = _lib.NoteDesc(**arch)
@@ -889,7 +889,7 @@ class NotePolicy(nn.Module):
         arch = self._native_desc(self.stream_dtype)
         if arch is None:
             return None
-        c, key = self._train_plan_cache, self.stream_dtype
+        c, key = self._train_plan_cache, tuple(arch.values())
         if c is None or c[0] != key:
             c = self._train_plan_cache = (key, NoteTrainPlan(arch, self._native_shapes(arch)))
         return c[1] if c[1].supported else None

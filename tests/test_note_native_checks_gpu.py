@@ -71,3 +71,18 @@ def test_masters_of_another_type_or_place_are_refused():
     m.critic_mlp[1] = nn.Tanh()
     with pytest.raises(RuntimeError):
         _grads(m, obs)
+
+
+def test_settings_changed_after_a_forward_are_followed():
+    obs = _obs()
+    m = _policy(note_geo=True)
+    before = _grads(m, obs)
+    lg, v = m.forward_stacked(obs)
+    m.z_asinh, fresh = 3.0, _policy(note_geo=True, z_asinh=3.0)
+    fresh.load_state_dict(m.state_dict())
+    want = fresh.forward_stacked(obs)
+    assert all(torch.equal(a, b) for a, b in zip(m.forward_stacked(obs), want)) and not torch.equal(want[0], lg)
+    with torch.no_grad():
+        assert torch.equal(m.forward_stacked(obs)[0], want[0])
+    after, ref = _grads(m, obs), _grads(fresh, obs)
+    assert all(torch.equal(after[n], ref[n]) for n in ref) and any(not torch.equal(after[n], before[n]) for n in ref)
