@@ -39,6 +39,7 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _lib
 from . import fp16_linear as _fl
@@ -585,13 +586,16 @@ class NotePolicy(nn.Module):
     # ---- the fused routes as native calls ------------------------------------------------------
     def _native_desc(self, dt):
         """What bsrl_note_* are told of the architecture, or None where the modules hold something that those calls do not
-        compute as the op-by-op forward would: an architecture option, another eps or activation."""
-        if self.value_residual or self.emb_ln is not None or self.final_ln is not None or self.trunk_arch != "simba":
+        compute as the op-by-op forward would: an architecture option, another eps or activation, a LayerNorm that this forward
+        calls as a module (trunk, critic) of another class or with hooks."""
+        if self.value_residual or self.emb_ln is not None or self.final_ln is not None or self.trunk_arch != "simba" or _has_any_global_hook():
             return None
         M = self._modules                          # the dicts themselves: a lookup by attribute or index costs several times this walk
         try:
             for k in ("trunk_ln1", "trunk_ln2", "critic_ln"):
-                if M[k].eps != 1e-5:
+                m = M[k]
+                if (type(m) is not FusedLayerNorm or m.eps != 1e-5 or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                        or m._backward_pre_hooks or "forward" in m.__dict__):
                     return None
             seqs = [M[k]._modules for k in ("saber_mlp", "torso_mlp", "leg_mlp", "note_mlp")]
             for b in M["blocks"]._modules.values():

@@ -86,3 +86,24 @@ def test_settings_changed_after_a_forward_are_followed():
         assert torch.equal(m.forward_stacked(obs)[0], want[0])
     after, ref = _grads(m, obs), _grads(fresh, obs)
     assert all(torch.equal(after[n], ref[n]) for n in ref) and any(not torch.equal(after[n], before[n]) for n in ref)
+
+
+@pytest.mark.parametrize("k", ["trunk_ln1", "trunk_ln2", "critic_ln"])
+def test_layernorms_that_are_called_as_modules_keep_their_hooks_and_class(k):
+    m, obs, seen = _policy(), _obs(), []
+    want = [t.detach() for t in m.forward_stacked(obs)]
+    h = getattr(m, k).register_forward_hook(lambda *a: seen.append(1))
+    with torch.no_grad():
+        m.forward_stacked(obs)
+    n = len(seen)
+    _grads(m, obs)                                               # the rollout's forward and the update's own
+    assert n == 1 and len(seen) == 3
+    h.remove()
+    assert all(torch.equal(a, b) for a, b in zip(m.forward_stacked(obs), want)) and len(seen) == 3
+
+    class Shifted(type(getattr(m, k))):
+        def forward(self, x):
+            return super().forward(x) + 1
+
+    getattr(m, k).__class__ = Shifted
+    assert not torch.equal(m.forward_stacked(obs)[1], want[1])
