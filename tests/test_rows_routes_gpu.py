@@ -37,3 +37,28 @@ def test_no_batch_size_rounds_the_residual_stream(arch, dtype):
     for n in (200, 300, 512, 513, B):
         mine, blocks = err(m.forward_stacked(obs[:n], k[:n])), err(m.forward_stacked(obs[:n], k[:n], route="blocks"))
         assert mine <= 1.03 * blocks, (n, mine, blocks)
+
+
+@pytest.mark.parametrize("arch,dtype", [((2, 128, 4, 512, 16), "f32"), ((2, 384, 12, 1536, 48), "f16")])
+def test_masters_of_another_type_place_or_shape_are_refused(arch, dtype):
+    """By pointer go LayerNorm masters in fp32 on the device and weights of the descriptor's shapes: the checks of ops.ln_fwd and
+    ops.linear, which the route calls no more."""
+    spec, _, m = _model(arch, dtype)
+    obs, k = cm.make_inputs(spec, 9, 6, "uniform")
+    obs, k = obs.to(DEV), k.to(DEV)
+    m.forward_stacked(obs, k)
+    m.half()
+    with pytest.raises((RuntimeError, TypeError)):
+        m.forward_stacked(obs, k)
+    m.float().blocks[1].ln_ffn.cpu()
+    m.bump_weights_version()
+    with pytest.raises((RuntimeError, TypeError)):
+        m.forward_stacked(obs, k)
+    m.to(DEV)
+    m.forward_stacked(obs, k)
+    m.blocks[1].ffn[0], m.blocks[1].ffn[2] = torch.nn.Linear(m.d, 96).to(DEV), torch.nn.Linear(96, m.d).to(DEV)
+    m.bump_weights_version()
+    with pytest.raises(RuntimeError):
+        m.forward_stacked(obs, k, route="ragged")
+    if dtype == "f32":          # its op-by-op route takes any hidden width
+        assert torch.equal(m.forward_stacked(obs, k)[0], m.forward_stacked(obs, k, route="ops")[0])
