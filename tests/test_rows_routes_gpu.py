@@ -62,3 +62,16 @@ def test_masters_of_another_type_place_or_shape_are_refused(arch, dtype):
         m.forward_stacked(obs, k, route="ragged")
     if dtype == "f32":          # its op-by-op route takes any hidden width
         assert torch.equal(m.forward_stacked(obs, k)[0], m.forward_stacked(obs, k, route="ops")[0])
+
+
+@pytest.mark.parametrize("arch,dtype", [((2, 128, 4, 512, 16), "f32"), ((2, 384, 12, 1536, 48), "f16")])
+def test_another_eps_reaches_the_forward(arch, dtype):
+    spec, _, m = _model(arch, dtype)
+    obs, k = cm.make_inputs(spec, 9, 6, "uniform")
+    obs, k = obs.to(DEV), k.to(DEV)
+    want = m.forward_stacked(obs, k)
+    for blk in m.blocks:
+        blk.ln_attn.eps = blk.ln_ffn.eps = 0.5
+    got = m.forward_stacked(obs, k)
+    assert (got[0] - want[0]).norm() > 0.05 * want[0].norm()
+    assert torch.equal(got[0], m.forward_stacked(obs, k, route="ops")[0])
