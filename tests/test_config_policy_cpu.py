@@ -25,3 +25,37 @@ def test_compacted_route_leaves_another_eps_to_the_ops():
                 assert not m.ragged_supported()
                 ln.eps = 1e-5
         assert m.ragged_supported()
+
+
+def test_auto_routes_by_shape_and_batch(monkeypatch):
+    """Which route and form `auto` takes on either side of its lines: no batch size gives up the fp32 residual stream that the
+    block-stack kernel has, and the forms change where they were measured to cross."""
+    got = []
+    for n in ("fused", "blocks", "rows", "ops"):
+        monkeypatch.setattr(ConfigPolicy, f"_forward_{n}", lambda s, o, k, dt, tail=None, w=None, n=n: got.append(n if n != "rows" else "tail" if tail else "by op"))
+    monkeypatch.setattr(ConfigPolicy, "_replicas", lambda *a: None)
+    monkeypatch.setattr(ConfigPolicy, "_rows_weights", lambda *a: None)
+
+    class Obs:          # a batch on the GPU, as far as the choice of a route looks at it
+        is_cuda, device = True, "cuda"
+
+        def __init__(self, *shape):
+            self.shape = shape
+
+        def dim(self):
+            return 2
+
+    def route(B, **kw):
+        m = ConfigPolicy(**kw)
+        got.clear()
+        m.forward_stacked(Obs(B, m.obs_dim))
+        return got[0]
+
+    wide, deep = dict(n_layers=4, d=256, n_heads=8, ffn=1024, T=32), dict(n_layers=6, d=384, n_heads=12, ffn=1536, T=48)
+    assert [route(B, **wide) for B in (1, 256, 257, 448, 449, 32768)] == ["blocks", "blocks", "by op", "by op", "tail", "tail"]
+    assert [route(B, **{**wide, "n_layers": 1}) for B in (256, 257, 4096)] == ["blocks", "by op", "by op"]
+    assert [route(B, **{**wide, "T": 40}) for B in (1, 358, 359)] == ["by op", "by op", "tail"]
+    assert [route(B, **deep) for B in (1, 234, 235, 65536)] == ["by op", "by op", "tail", "tail"]
+    assert {route(B, n_layers=3, d=192, n_heads=4, ffn=768, T=29) for B in (1, 300, 9000)} == {"blocks"}
+    assert [route(B, n_layers=3, d=192, n_heads=6, ffn=768, T=29) for B in (1, 494, 495)] == ["by op", "by op", "tail"]
+    assert {route(B, dtype="f32") for B in (1, 20000)} == {"by op"} and {route(B) for B in (1, 20000)} == {"fused"}
