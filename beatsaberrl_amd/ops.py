@@ -665,30 +665,35 @@ def block_tail_pack(wo, bo, w0, b0, w2, b2, wn=None, bn=None, image=None):
     return image
 
 
-def block_tail(att, x, image, F, ln2, ln, n_next, rows, extra, act, ho_rows=None):
+def block_tail(att, x, image, F, ln2, ln, n_next, rows, extra, act, ho_rows=None, xo_dtype=None):
     """One block from the attention output on over the first rows + *extra rows of x (n, d) (extra: one-element int32 device
-    tensor or None = n rows).  ln2 / ln: (weight, bias, eps) or None; F = 0: the lead form.  Returns (xo, ho, qo); ho is
-    allocated for ho_rows rows (None: all; 0: not written)."""
+    tensor or None = n rows).  ln2 / ln: (weight, bias, eps) or None; F = 0: the lead form.  x, and with xo_dtype xo, may be
+    fp32 beside a 16-bit att (the fp32 residual stream, d = 256).  Returns (xo, ho, qo); ho is allocated for ho_rows rows (None:
+    all; 0: not written)."""
     _need_cuda(att, x, image, extra)
     n, d = x.shape
-    if not x.is_contiguous() or (att is not None and (not att.is_contiguous() or att.shape != x.shape or att.dtype is not x.dtype)):
-        raise RuntimeError("block_tail: att and x contiguous, one shape, one dtype")
-    if image.numel() != _lib.load().bsrl_block_tail_pack_size(d, F, n_next, dt_code(x.dtype)) or image.device != x.device:
+    dt = x.dtype if att is None else att.dtype
+    xo_dtype = dt if xo_dtype is None else xo_dtype
+    if not x.is_contiguous() or (att is not None and (not att.is_contiguous() or att.shape != x.shape)) or any(
+            t is not dt and t is not torch.float32 for t in (x.dtype, xo_dtype)):
+        raise RuntimeError("block_tail: att and x contiguous, one shape; x and xo in att's dtype or fp32")
+    x_f32 = 0 if dt is torch.float32 else int(x.dtype is torch.float32) | 2 * int(xo_dtype is torch.float32)
+    if image.numel() != _lib.load().bsrl_block_tail_pack_size(d, F, n_next, dt_code(dt)) or image.device != x.device:
         raise RuntimeError("block_tail: image does not belong to this shape / dtype / device")
     if extra is None:
         rows = n
     ho_rows = n if ho_rows is None else ho_rows
-    xo = torch.empty_like(x) if F else None
-    ho = torch.empty(ho_rows, d, device=x.device, dtype=x.dtype) if ln is not None and ho_rows else None
-    qo = torch.empty(n, n_next, device=x.device, dtype=x.dtype) if n_next else None
+    xo = torch.empty(n, d, device=x.device, dtype=xo_dtype) if F else None
+    ho = torch.empty(ho_rows, d, device=x.device, dtype=dt) if ln is not None and ho_rows else None
+    qo = torch.empty(n, n_next, device=x.device, dtype=dt) if n_next else None
     w2, b2, e2 = ln2 if ln2 is not None else (None, None, 0.0)
     w1, b1, e1 = ln if ln is not None else (None, None, 0.0)
     with torch.cuda.device(x.device):
         rc = _lib.load().bsrl_block_tail(image.data_ptr(), _ptr(att), x.data_ptr(), _ptr(w2), _ptr(b2), float(e2), _ptr(w1), _ptr(b1),
                                          float(e1), _ptr(xo), _ptr(ho), ho_rows, _ptr(qo), n_next, rows, _ptr(extra),
-                                         n - rows if extra is not None else 0, d, F, _ACT[act], dt_code(x.dtype), 0, _stream(x))
+                                         n - rows if extra is not None else 0, d, F, _ACT[act], dt_code(dt), x_f32, _stream(x))
     if not _lib.check(rc, "bsrl_block_tail"):
-        raise Unsupported(f"block_tail d={d} F={F} n_next={n_next} dtype={x.dtype}")
+        raise Unsupported(f"block_tail d={d} F={F} n_next={n_next} dtype={dt} x={x.dtype} xo={xo_dtype}")
     return xo, ho, qo
 
 

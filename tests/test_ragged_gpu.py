@@ -139,3 +139,41 @@ def test_ragged_route(arch, dtype, ceil, mask):
     m.prune_final = False
     lg4, _ = m.forward_stacked(obs.to(DEV), None if mask == "none" else k.to(DEV), route="ragged")
     assert (lg4 - lg).abs().max().item() <= ceil[1]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("act,Fh", [("gelu", 1024), ("relu", 96)])
+@pytest.mark.parametrize("n", [1, 63, 700, 35000])
+@pytest.mark.parametrize("form", ["into", "along", "out of"])
+def test_block_tail_fp32_stream(dtype, act, Fh, n, form):
+    """The forms that carry the residual stream in fp32 (d = 256): into it (16-bit x), along it, out of it (no LayerNorm behind).
+    Neither x1 nor an fp32 xo is rounded; h2, the hidden, ho and qo are."""
+    d = 256
+    mk = lambda *s, seed, scale=1.0, dt=torch.float32: _rand(*s, seed=seed, scale=scale, dtype=dt)
+    lead, last = (n + 3) // 4, form == "out of"
+    x, att = mk(n + 5, d, seed=1, dt=dtype if form == "into" else torch.float32), mk(n + 5, d, seed=2, dt=dtype)
+    wo, w0, w2, wn = (mk(d, d, seed=3, scale=d ** -0.5, dt=dtype), mk(Fh, d, seed=4, scale=d ** -0.5, dt=dtype),
+                      mk(d, Fh, seed=5, scale=Fh ** -0.5, dt=dtype), mk(3 * d, d, seed=6, scale=d ** -0.5, dt=dtype))
+    bo, b0, b2, bn = mk(d, seed=7), mk(Fh, seed=8), mk(d, seed=9), mk(3 * d, seed=10)
+    l2, l1 = (mk(d, seed=11) + 1, mk(d, seed=12), 1e-5), (mk(d, seed=13) + 1, mk(d, seed=14), 1e-5)
+    img = ops.block_tail_pack(wo, bo, w0, b0, w2, b2, *(() if last else (wn, bn)))
+    extra = torch.tensor([n - lead], dtype=torch.int32, device=DEV)
+    xo, ho, qo = ops.block_tail(att, x, img, Fh, l2, None if last else l1, 0 if last else 3 * d, lead, extra, act, ho_rows=lead,
+                                xo_dtype=dtype if last else torch.float32)
+    r = lambda t: t.to(dtype).float()
+    u = 2.0 ** -10 if dtype is torch.float16 else 2.0 ** -7
+    x1 = x[:n].float() + att[:n].float() @ wo.float().t() + bo
+    h2 = F.layer_norm(x1, (d,), *l2)
+    hid = r(h2) @ w0.float().t() + b0
+    hid = r(F.gelu(hid) if act == "gelu" else F.relu(hid))
+    ref = x1 + hid @ w2.float().t() + b2
+    lim = lambda got, want, k: ((got.float() - want).abs() <= k * u * want.abs().clamp_min(1.0)).all()
+    e = (xo[:n].float() - ref).abs()
+    if last:
+        assert lim(xo[:n], ref, 8.0)
+    else:
+        # fp32 out: what is left are single ulps of h2 and of the hidden that moved with the summation order.  One of h2
+        # (u h2 at most) reaches xo through two matrices of unit gain; the typical value has none and shows fp32 sums
+        assert e.max() <= 8.0 * u and e.median() <= 0.2 * u, (e.max().item(), e.median().item())
+        hr = F.layer_norm(xo[:n], (d,), *l1)                      # both LayerNorms see unrounded rows
+        assert lim(ho, hr[:lead], 1.0) and lim(qo[:n], r(hr) @ wn.float().t() + bn, 12.0)
