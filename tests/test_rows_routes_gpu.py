@@ -75,3 +75,35 @@ def test_another_eps_reaches_the_forward(arch, dtype):
     got = m.forward_stacked(obs, k)
     assert (got[0] - want[0]).norm() > 0.05 * want[0].norm()
     assert torch.equal(got[0], m.forward_stacked(obs, k, route="ops")[0])
+
+
+@pytest.mark.parametrize("arch,dtype,B,ceil", [
+    ((4, 256, 8, 1024, 32), "bf16", 449, (4.3e-2, 4.1e-2)), ((4, 256, 8, 1024, 32), "f16", 449, (5.0e-3, 6.0e-3)),
+    ((6, 384, 12, 1536, 48), "f16", 235, (6.7e-3, 6.2e-3)), ((2, 192, 6, 384, 17), "bf16", 844, (4.2e-2, 2.6e-2))])
+@pytest.mark.parametrize("mask", ["uniform", "quarter_empty", "none"])
+def test_block_tail_form_of_the_compacted_route(arch, dtype, B, ceil, mask):
+    """The first batch that takes the form (config wide's and config deep's, d = 192): distance to the fp32 oracle and to the
+    rounding-emulating one (ceilings: 1.3 times the largest measured over the masks), and agreement with the form and the routes
+    on the other side of the line, which are as far from that oracle."""
+    spec, p, m = _model(arch, dtype, seed=41, act="gelu", final_ln=True)
+    assert (B - 1) * spec.T <= m._rows_by_op(torch.float16) < B * spec.T
+    obs, k = cm.make_inputs(spec, B, 42, mask)
+    o, kk = obs.to(DEV), None if mask == "none" else k.to(DEV)
+    got = _out(m.forward_stacked(o, kk, route="ragged"))
+    ref = _out(cm.forward(p, spec, obs, k))
+    em = _out(cm.forward(p, spec, obs, k, emulate=dtype, round_residual=spec.d != 256))
+    e = [(got - ref).abs().max().item(), (got - em).abs().max().item()]
+    print(f"\nGATE16 tail {arch} {dtype} {mask} fp32={e[0]:.3e} class={e[1]:.3e}")
+    assert e[0] <= ceil[0] and e[1] <= ceil[1], e
+    less = [m.forward_stacked(o[:-1], None if kk is None else kk[:-1], route=r) for r in ("ragged", "ops", None)]      # by op
+    for other in less:
+        assert (_out(other) - got[:-1]).abs().max().item() <= 2 * ceil[1]
+    if mask != "none":      # what a masked slot holds cannot reach an output
+        junk = o.clone()
+        for b in range(B):
+            junk[b, spec.prop_dim + int(k[b]) * spec.obj_dim:] = float("nan")
+        assert torch.equal(_out(m.forward_stacked(junk, kk, route="ragged")), got)
+        perm = torch.randperm(B)            # an env's bits do not depend on its neighbours
+        assert torch.equal(_out(m.forward_stacked(o[perm], kk[perm], route="ragged")), got[perm])
+    m.prune_final = False
+    assert (_out(m.forward_stacked(o, kk, route="ragged")) - got).abs().max().item() <= 2 * ceil[1]
