@@ -544,10 +544,10 @@ __global__ __launch_bounds__(256) void attn_f32_mfma_kernel(F32AttnArgs f) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int key = kt * 16 + 4 * g + i;
-            const bool in = kt < nkt && key < T;
+            const bool in = kt < nkt && key < T && key <= nv;        // a key past n_valid is never looked at, whatever it holds
 #pragma unroll
             for (int c = 0; c < DC; ++c) vf[kt][c][i] = in ? vp[row(key, a.v_bs, a.v_rs) + 16 * c + r16] : 0.f;
-            kb[kt][i] = !in || key > nv ? -INFINITY : a.key_bias ? static_cast<const float*>(a.key_bias)[b * a.T + key] : 0.f;
+            kb[kt][i] = !in ? -INFINITY : a.key_bias ? static_cast<const float*>(a.key_bias)[b * a.T + key] : 0.f;
         }
     }
     for (int qt = 0; qt < nqt; ++qt) {
@@ -568,7 +568,11 @@ __global__ __launch_bounds__(256) void attn_f32_mfma_kernel(F32AttnArgs f) {
                     for (int e = 0; e < 4; ++e) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kt][c][e], qf[c][e], s[kt], 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { s[kt][i] = s[kt][i] * a.scale + kb[kt][i]; m = fmaxf(m, s[kt][i]); }
+            for (int i = 0; i < 4; ++i) {
+                const int key = kt * 16 + 4 * g + i;
+                s[kt][i] = key < T && key <= nv ? s[kt][i] * a.scale + kb[kt][i] : -INFINITY;
+                m = fmaxf(m, s[kt][i]);
+            }
         }
         m = fmaxf(m, __shfl_xor(m, 16, WAVE));
         m = fmaxf(m, __shfl_xor(m, 32, WAVE));

@@ -60,3 +60,17 @@ def test_fp32_attention(B, T, TQ, H, dh):
     rows = torch.cat([qkv[:, 0], torch.cat([qkv[b, 1:1 + int(nv[b])] for b in range(B)])])
     out = ops.attn_ragged(rows[:B, :d], rows[:, d:2 * d], rows[:, 2 * d:], noff, B, 1, T - 1, H, lead_only=True)
     assert (out.double() - ref[:, 0]).abs().max() <= 4e-6
+
+
+@pytest.mark.parametrize("T,TQ,H,dh", [(16, 16, 4, 32), (48, 48, 2, 32), (29, 5, 4, 48), (33, 1, 3, 64)])
+@pytest.mark.parametrize("junk", [float("nan"), float("inf"), 3e38])
+def test_fp32_attention_never_looks_at_masked_keys(T, TQ, H, dh, junk):
+    B, d = 9, H * dh
+    qkv = _rand(B, T, 3 * d, seed=5)
+    nv = torch.arange(B, dtype=torch.int32) * T // B
+    q = qkv[:, :TQ, :d].clone()
+    want = ops.attn_fwd(q, qkv[..., d:2 * d], qkv[..., 2 * d:], H, n_valid=nv.to(DEV))
+    for b in range(B):
+        qkv[b, int(nv[b]) + 1:, d:] = junk
+    got = ops.attn_fwd(q, qkv[..., d:2 * d], qkv[..., 2 * d:], H, n_valid=nv.to(DEV))
+    assert torch.equal(got, want) and torch.isfinite(got).all()
