@@ -21,8 +21,8 @@
 // Three pipelines, chosen on the host by shape and batch (same output bits):
 //   * DMA  - the throughput forms' default: stages go straight from L2 into a 6-slot LDS ring
 //            (global_load_lds_dwordx4), admitted in pairs: one vmcnt wait + barrier per two stages;
-// (up to four envs per CU at F = 512 a kernel of its own, cfg_latency.hip)
-//   * RING - the latency form (B <= 4 per CU): the same transfers 13 stages ahead into a 14-slot ring, one env per wave;
+//   * RING - the latency form (B <= 4 per CU, F other than 512: there a kernel of its own runs, cfg_latency.hip): the same
+//            transfers 13 stages ahead into a 14-slot ring, one env per wave;
 //   * register-staged (models whose vectors + two rings overflow a CU's LDS): global loads three stages ahead into
 //     registers, written to a 2-slot LDS ring one stage ahead, one barrier per stage.
 // HBM traffic is the obs in, the logits out and, in the pruned form, each env's parked token-0 row (768 B).

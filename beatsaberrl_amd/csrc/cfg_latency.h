@@ -1,4 +1,5 @@
-// The one-env-per-workgroup form of the config-model forward (cfg_latency.hip), launched by cfg_forward.hip.
+// The config-model forward with a workgroup's features dealt over its waves, one to four envs per workgroup (cfg_latency.hip),
+// launched by cfg_forward.hip.
 #pragma once
 #include "bsrl_common.h"
 

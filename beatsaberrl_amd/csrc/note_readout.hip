@@ -1,5 +1,5 @@
-// What follows NotePolicy's block stack - trunk, action heads, the critic's projections, the value MLP - for batches of up to 16
-// envs per CU, as two launches around the critic's attention pool instead of seventeen.
+// What follows NotePolicy's block stack - trunk, action heads, the critic's projections, the value MLP - for batches of up to 32
+// envs per CU (READOUT_MOST in note_forward.hip), as two launches around the critic's attention pool instead of seventeen.
 //
 // Every one of those Linears is a few 100 KB of weights against B rows: 4 - 5.5 us a launch whatever B is, 70 us of a one-env
 // forward's 177 and most of its host time.  Here a workgroup takes up to 16 envs - the columns of one MFMA tile - through a chain

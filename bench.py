@@ -81,7 +81,7 @@ def main():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=200)
     ap.add_argument("--warmup", type=int, default=10)
-    ap.add_argument("--route", default="auto", choices=("auto", "fused", "blocks", "ops"))
+    ap.add_argument("--route", default="auto", choices=("auto", "fused", "blocks", "ragged", "ops"))
     ap.add_argument("--config", type=int, default=1, help="benchmark config index (1 = headline)")
     ap.add_argument("--batch", type=int, default=0, help="override B (0 = the config's B)")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
@@ -128,10 +128,10 @@ def main():
     obs, k = obs_cpu.to(dev), k_cpu.to(dev)
     route = args.route
     if route == "auto":
-        route = "fused" if m.fused_supported() else "blocks" if m.blocks_supported() else "ops"
+        route = m.auto_route(B)
 
     def step():
-        return m.forward_stacked(obs, k, route=route)
+        return m.forward_stacked(obs, k, route=args.route)
 
     # parity against the fp32 CPU oracle before timing anything: the error distribution over the first n_par envs
     def error_stats(lg_dev, ref):
@@ -237,7 +237,8 @@ def main():
     # FLOPs per forward: the dense figure (every token of every block), and the ALGORITHMIC figure of the path as
     # the reference runs it - the final block pruned to token 0 (its own n_queries path), every env's 16 token rows
     # (padding rows included: the reference computes and masks them).  Both are side notes of the roofline object;
-    # its fraction is quoted on what the matrix pipe is really issued (below).
+    # its fraction is quoted on what the matrix pipe is really issued (below).  On the compacted route padding rows are not
+    # computed: there both figures are of the attendable tokens.
     dense_flops = cm.flops_per_env(spec) * B
     pruned = (route in ("fused", "ops") and m.prune_final) or route == "blocks"
     exec_flops = dense_flops
@@ -247,6 +248,15 @@ def main():
         if route == "ops":
             saved += (T_ - 1) * (d_ * d_ + 2 * T_ * d_)     # ... and their query projection, scores and weighted sums
         exec_flops = dense_flops - 2 * saved * B
+    if route == "ragged":       # the attendable tokens alone (the compacted stream)
+        d_, F_, L_ = spec.d, spec.ffn, spec.n_layers
+        t_ = (k_cpu.clamp(0, spec.T - 1) + 1).double()
+        s1, s2 = t_.sum().item(), (t_ * t_).sum().item()
+        macs = B * spec.prop_dim * d_ + (s1 - B) * spec.obj_dim * d_ + B * d_ * spec.n_out
+        for i in range(L_):
+            q_ = B if m.prune_final and i + 1 == L_ else s1                  # rows behind the keys and values
+            macs += s1 * 2 * d_ * d_ + q_ * (2 * d_ * d_ + 2 * d_ * F_) + 2 * d_ * (s1 if q_ == B else s2)
+        exec_flops = int(2 * macs)
     # ... and, on the fused route, the 16-row tiles the launch really runs: envs of 5..8 tokens go two to a
     # tile, of at most 4 tokens behind an env of 9..12 tokens or four to a tile (same output bits), so the per-tile
     # work is counted per tile
@@ -273,6 +283,8 @@ def main():
              "cfg_pair_kernel (tile table) + cfg_forward_kernel, one merged launch (final block pruned to token 0, short envs "
              "share tiles)" if tiles is not None else
              "cfg_embed_kernel + blocks_kernel (final block pruned to token 0) + heads" if route == "blocks" else
+             "compacted token stream: cfg_tokens_kernel, then per block attn_ragged_kernel and block_tail_kernel or one kernel per op "
+             "(final block pruned to token 0), heads" if route == "ragged" else
              "cfg_forward_kernel HEAD + TAIL launches (final block pruned to token 0)" if pruned and route == "fused" else
              "cfg_forward_kernel FULL (one persistent launch)" if route == "fused" else
              "launch train (per-op route; final block pruned to token 0)" if pruned else

@@ -211,10 +211,10 @@ int bsrl_ln_proj_packed(const void* image, const void* x, const float* ln_w, con
  *
  * bsrl_token_offsets: noff from n_valid (B, int32; NULL: all of them; clamped to [0, opt]).
  * bsrl_cfg_tokens: the config tokenizer (bsrl_cfg_embed's Linears, one lead token) into the stream,
- * obs fp32 or `dtype`; d in {128, 192, 256, 384}, obj_dim <= 32, 16-bit dtypes.
+ * obs fp32 or `dtype`; obj_dim <= 32; d in {128, 192, 256, 384} in 16 bit, any up to 4096 in fp32.
  * bsrl_attn_ragged: attention over the stream; q, k, v, out row-strided views of it; n_queries = 0:
  * every token queries, else n_queries <= lead per env (q and out then hold n_queries B rows, env by env).  opt_bias: additive bias of the optional keys
- * in `dtype`, indexed by row - lead B (NULL: none).  lead + opt <= 48, dh 32 or 48.
+ * in `dtype`, indexed by row - lead B (NULL: none; 16 bit only).  lead + opt <= 48, dh 32 or 48, in fp32 also 64.
  * bsrl_block_tail: bsrl_proj_ffn_packed for d in {192, 256, 384} on rows + *extra rows (extra a
  * device int32 or NULL; extra_max its bound, 0 without one); ho is written for rows below ho_rows.
  * x_f32 (d = 256): bit 0 - x is fp32, bit 1 - xo is fp32 (x1 then stays unrounded; bit 1 needs ln_w, bit 0
@@ -268,17 +268,16 @@ typedef struct {
 /* bsrl_cfg_forward: keep every env in a tile of its own (see below). */
 #define BSRL_CFG_NO_PACK 1
 /* bsrl_cfg_forward: never take the latency form.  By default a batch of at
- * most 4 envs per CU (B <= 1024 on an MI355X) runs as ONE persistent launch
- * whatever the workspace: one env per wave (1..4 working waves per workgroup,
- * as few as the batch allows), the weight image streamed straight into a
- * 14-slot LDS ring 13 stages ahead, the next stage's fragments fetched into
- * registers while the current one is computed.  At such sizes a forward is one
- * workgroup's walk through the ~100 stages of the image and its time is what a
- * lone CU takes to pull 0.9 MB and to run the dependent chain of each stage
- * (B = 1: 33 us against 52 us for the throughput forms).  The output bits are
- * those of the other forms (tested), so an env's result does not change with
- * the batch it is in.  Shapes whose vectors + ring exceed a workgroup's LDS
- * (n_layers * (9 d + ffn) floats + 112 KB > 158 KB) always take the other forms. */
+ * most 4 envs per CU (B <= 1024 on an MI355X) runs as ONE launch whatever the
+ * workspace.  ffn = 512: one to four envs per workgroup, the features dealt over
+ * its eight waves, weight fragments straight from L2 into the wave that needs
+ * them (2 blocks, B = 1: 13 us).  Other ffn: one env per wave (1..4 working
+ * waves per workgroup, as few as the batch allows), the weight image streamed
+ * straight into a 14-slot LDS ring 13 stages ahead (at ffn = 512 that took
+ * 28 us, the throughput forms 47).  The output bits are those of the other forms
+ * (tested), so an env's result does not change with the batch it is in.  Shapes whose
+ * vectors + ring exceed a workgroup's LDS (n_layers * (9 d + ffn) floats + 112 KB
+ * > 158 KB; ffn other than 512) always take the throughput forms. */
 #define BSRL_CFG_NO_LATENCY 2
 
 /* fp32 master parameter pointers of one transformer block, in the reference's
@@ -368,8 +367,9 @@ int bsrl_cfg_forward_static(const bsrl_cfg_desc* desc, const void* packed,
  * LayerNorm affine fp32.  With tail images (bsrl_block_tail_pack: lead_img = block 0's projection of
  * 3 d columns, 2 d when prune and one layer; blk[i].tail_img with the next block's projection behind,
  * 2 d columns in front of the pruned final block, none behind the last): attention + one kernel per
- * block, the residual stream in fp32 at d = 256; without: one kernel per op (any dtype; K of every
- * Linear a multiple of 8, of 4 in fp32).  prune: the final block computes token 0 alone.
+ * block; without: one kernel per op (any dtype; K of every Linear a multiple of 8, of 4 in fp32).  At
+ * d = 256 the residual stream is fp32 either way (a single block with a tail image rounds it once, in
+ * the middle).  LayerNorm eps 1e-5.  prune: the final block computes token 0 alone.
  * Workspace: bsrl_cfg_rows_workspace_size bytes (tail: images given), 16-byte aligned. */
 typedef struct {
     const void *prop_w, *obj_w, *heads_w;

@@ -107,3 +107,17 @@ def test_block_tail_form_of_the_compacted_route(arch, dtype, B, ceil, mask):
         assert torch.equal(_out(m.forward_stacked(o[perm], kk[perm], route="ragged")), got[perm])
     m.prune_final = False
     assert (_out(m.forward_stacked(o, kk, route="ragged")) - got).abs().max().item() <= 2 * ceil[1]
+
+
+@pytest.mark.parametrize("arch,dtype,sizes", [((2, 256, 8, 1024, 32), "bf16", (500, 1100, 3000)), ((2, 384, 12, 1536, 48), "f16", (250, 345, 1500))])
+def test_one_set_of_bits_per_form(arch, dtype, sizes):
+    """Inside a form (here the tail, over its tile sizes), and on the route that covers every batch size, an env's bits do not
+    depend on the batch."""
+    spec, _, m = _model(arch, dtype)
+    obs, k = cm.make_inputs(spec, sizes[-1], 6, "uniform")
+    obs, k = obs.to(DEV), k.to(DEV)
+    tails = [_out(m.forward_stacked(obs[:n], k[:n], route="ragged")) for n in sizes]
+    assert all(n * spec.T > m._rows_by_op(torch.float16) for n in sizes) and all(torch.equal(t, tails[-1][:n]) for n, t in zip(sizes, tails))
+    route = "blocks" if spec.d == 256 else "ops"
+    whole = _out(m.forward_stacked(obs, k, route=route))
+    assert all(torch.equal(_out(m.forward_stacked(obs[:n], k[:n], route=route)), whole[:n]) for n in (1, 9, *sizes[:2]))
