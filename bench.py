@@ -240,7 +240,9 @@ def main():
     # its fraction is quoted on what the matrix pipe is really issued (below).  On the compacted route padding rows are not
     # computed: there both figures are of the attendable tokens.
     dense_flops = cm.flops_per_env(spec) * B
-    pruned = (route in ("fused", "ops") and m.prune_final) or route == "blocks"
+    # up to four envs per CU the fused route runs the latency kernel, which computes every token of every block
+    latency = route == "fused" and m.latency_form and B <= 4 * torch.cuda.get_device_properties(dev).multi_processor_count
+    pruned = (route in ("fused", "ops") and m.prune_final and not latency) or route == "blocks"
     exec_flops = dense_flops
     if pruned:
         d_, T_, F_ = spec.d, spec.T, spec.ffn
@@ -261,7 +263,7 @@ def main():
     # tile, of at most 4 tokens behind an env of 9..12 tokens or four to a tile (same output bits), so the per-tile
     # work is counted per tile
     tiles, issued_flops = None, None
-    if route == "fused" and m.prune_final and m.pack_short and c["mask"] != "none" and spec.T == 16:
+    if route == "fused" and not latency and m.prune_final and m.pack_short and c["mask"] != "none" and spec.T == 16:
         tiny, mid = int((k_cpu <= 3).sum()), int(((k_cpu >= 4) & (k_cpu <= 7)).sum())
         host = int(((k_cpu >= 8) & (k_cpu <= 11)).sum())                   # 9..12 tokens: a tiny env rides in rows 12..15
         tiles = (mid + 1) // 2 + (max(tiny - host, 0) + 3) // 4 + (B - tiny - mid)
@@ -278,7 +280,8 @@ def main():
     run_flops = issued_flops if issued_flops is not None else exec_flops
     achieved = run_flops / (dev_ms_avg * 1e-3) / 1e12
     peak = MFMA_PEAK_TFLOPS[dtype]
-    kname = ("cfg_forward_kernel, ONE launch (tile table built in the kernel; final block pruned to token 0 and run by the "
+    kname = ("cfg_latency_kernel, ONE launch (one to four envs per workgroup, every token computed)" if latency else
+             "cfg_forward_kernel, ONE launch (tile table built in the kernel; final block pruned to token 0 and run by the "
              "workgroup that parked the rows; short envs share tiles)" if tiles is not None and B <= 16384 else
              "cfg_pair_kernel (tile table) + cfg_forward_kernel, one merged launch (final block pruned to token 0, short envs "
              "share tiles)" if tiles is not None else
