@@ -317,6 +317,8 @@ def build_head_gears(n_gears: int) -> tuple:
 
 
 class NotePolicy(nn.Module):
+    _train_plan_cache = _native_cache = None     # of a module that was pickled before it had them
+
     def __init__(self, embed: int = 128, trunk_dim: int = 256, encoder: str = "transformer", n_blocks: int = 3,
                  n_heads: int = 4, n_gears: int = 3, ffn_mult: int = 4, note_geo: bool = False,
                  value_bins: int = 101, value_vmax: float = 6.0, value_sigma: float = 0.75,

@@ -59,3 +59,19 @@ def test_auto_routes_by_shape_and_batch(monkeypatch):
     assert {route(B, n_layers=3, d=192, n_heads=4, ffn=768, T=29) for B in (1, 300, 9000)} == {"blocks"}
     assert [route(B, n_layers=3, d=192, n_heads=6, ffn=768, T=29) for B in (1, 494, 495)] == ["by op", "by op", "tail"]
     assert {route(B, dtype="f32") for B in (1, 20000)} == {"by op"} and {route(B) for B in (1, 20000)} == {"fused"}
+
+
+def test_copies_and_pickles_leave_the_native_structs_behind():
+    import copy
+    import pickle
+
+    from beatsaberrl_amd import _lib
+    m = ConfigPolicy()
+    m._desc(torch.float16)
+    m._replica = (("key",), {("rows", True, True): (_lib.CfgRowsWeights(), [])})          # as a forward leaves it
+    for c in (copy.deepcopy(m), pickle.loads(pickle.dumps(m))):
+        assert c._replica is None and c._desc_cache is None and torch.equal(c.heads.weight, m.heads.weight)
+    assert m._replica is not None
+    for k in ("_desc_cache", "_ws_rows"):           # a file written before the module had them
+        del m.__dict__[k]
+    assert m.fused_supported()
