@@ -380,6 +380,7 @@ class NoteTrainPlan:
             self.sizes.append(self.total - end)
         self.param_shapes = [torch.Size(s) for s in shapes]
         self.shapes = [tuple(s) if len(s) > 1 else None for s in shapes]
+        self.heads, self.critic = range(16 + 16 * self.desc.n_blocks + 10, len(shapes) - 16), range(len(shapes) - 16, len(shapes))
         # the masters that the backward reads (its matrices are the forward's 16-bit copies): the LayerNorm scales
         L = self.desc.n_blocks
         trunk, critic = 16 + 16 * L, len(shapes) - 16
@@ -425,6 +426,8 @@ class NoteTrainFn(torch.autograd.Function):
         saved, vlogits, centers, *scales = ctx.saved_tensors
         plan, lib, dev, B = ctx.plan, _lib.load(), saved.device, vlogits.shape[0]
         n_pass = 7                                             # inputs ahead of the parameters
+        # what no output in the loss depends on has no gradient, rather than a zero that an optimizer would step on
+        unused = set(plan.heads if g_logits is None else ()) | set(plan.critic if g_value is None and g_vlogits is None else ())
         if g_value is not None:                                # through the expectation over the bins
             p = torch.softmax(vlogits, dim=-1)
             gv = g_value.float().unsqueeze(1) * p * (centers - (p @ centers).unsqueeze(1))
@@ -444,7 +447,7 @@ class NoteTrainFn(torch.autograd.Function):
             raise ops.Unsupported("bsrl_note_train_backward")
         need = ctx.needs_input_grad
         pieces = flat.split_with_sizes(plan.sizes)
-        grads = [None if not need[n_pass + i] else pieces[at] if s is None else pieces[at].view(s)
+        grads = [None if not need[n_pass + i] or i in unused else pieces[at] if s is None else pieces[at].view(s)
                  for i, (at, s) in enumerate(zip(plan.at, plan.shapes))]
         del pieces
         return (None,) * n_pass + tuple(grads)

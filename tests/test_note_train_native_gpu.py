@@ -114,3 +114,48 @@ def test_loss_kernels_match_torch(B, K, bins):
     (3.0 * want).backward()
     assert abs(loss.item() - want.item()) <= 2e-5 * abs(want.item())
     assert torch.allclose(vl.grad.double(), rl.grad, atol=3e-5 / B)
+
+
+@pytest.mark.parametrize("loss", [lambda lg, v, vl: (lg ** 2).mean(), lambda lg, v, vl: (v ** 2).mean(), lambda lg, v, vl: (vl ** 2).mean(),
+                                  lambda lg, v, vl: (lg ** 2).mean() + (vl ** 2).mean()])
+def test_parameters_that_a_loss_does_not_reach_have_no_gradient(loss):
+    """The op-by-op update's: heads without the logits, the critic without value and bin logits."""
+    torch.manual_seed(0)
+    m = NotePolicy(embed=128, trunk_dim=256, n_blocks=2, n_heads=4, n_gears=5).to(DEV)
+    m.fp16 = True
+    m.torso_mlp[0].weight.requires_grad_(False)
+    obs = torch.randn(50, nr.OBS_DIM, device=DEV)
+    grads = {}
+    for mode in ("own", "rollout"):
+        m.update_values = mode
+        m.zero_grad(set_to_none=True)
+        lg, v = m.forward_stacked(obs)
+        (256 * loss(lg, v, m._value_logits)).backward()
+        grads[mode] = {n: p.grad for n, p in m.named_parameters()}
+    none = {k: {n for n, g in d.items() if g is None} for k, d in grads.items()}
+    assert none["rollout"] == none["own"]
+    for n, w in grads["own"].items():
+        if w is not None:
+            assert (grads["rollout"][n] - w).norm() <= 1e-2 * w.norm() + 1e-4
+
+
+def test_native_update_under_saved_tensor_hooks_and_a_second_backward():
+    """Saved tensors kept on the host, a graph that is walked twice, a checkpointed forward, gradients of some parameters: the
+    plain backward's bits."""
+    from torch.utils.checkpoint import checkpoint
+    torch.manual_seed(0)
+    m = NotePolicy(embed=128, trunk_dim=256, n_blocks=2, n_heads=4, n_gears=5).to(DEV)
+    m.fp16 = True
+    obs = torch.randn(130, nr.OBS_DIM, device=DEV)
+    ps = list(m.parameters())
+    loss = lambda outs: 64 * ((outs[0] ** 2).mean() + (outs[1] ** 2).mean())
+    want = torch.autograd.grad(loss(m.forward_stacked(obs)), ps)
+    with torch.autograd.graph.save_on_cpu():
+        out = loss(m.forward_stacked(obs))
+    again = loss(m.forward_stacked(obs))
+    first = torch.autograd.grad(again, ps, retain_graph=True)
+    part = torch.autograd.grad(again, ps[3:9], retain_graph=True)
+    ck = torch.autograd.grad(loss(checkpoint(m.forward_stacked, obs, use_reentrant=False)), ps)
+    for got in (torch.autograd.grad(out, ps), first, torch.autograd.grad(again, ps), ck):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(torch.equal(a, b) for a, b in zip(part, want[3:9]))
