@@ -58,6 +58,7 @@ def test_auto_routes_by_shape_and_batch(monkeypatch):
     assert [route(B, **deep) for B in (1, 234, 235, 65536)] == ["by op", "by op", "tail", "tail"]
     assert {route(B, n_layers=3, d=192, n_heads=4, ffn=768, T=29) for B in (1, 300, 9000)} == {"blocks"}
     assert [route(B, n_layers=3, d=192, n_heads=6, ffn=768, T=29) for B in (1, 494, 495)] == ["by op", "by op", "tail"]
+    assert route(8, **deep, prop_dim=4096) == "by op" and route(8, **deep, prop_dim=4100) == "ops" and route(8, **deep, obj_dim=36) == "ops"
     assert {route(B, dtype="f32") for B in (1, 20000)} == {"by op"} and {route(B) for B in (1, 20000)} == {"fused"}
 
 
