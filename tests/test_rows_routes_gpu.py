@@ -121,3 +121,26 @@ def test_one_set_of_bits_per_form(arch, dtype, sizes):
     route = "blocks" if spec.d == 256 else "ops"
     whole = _out(m.forward_stacked(obs, k, route=route))
     assert all(torch.equal(_out(m.forward_stacked(obs[:n], k[:n], route=route)), whole[:n]) for n in (1, 9, *sizes[:2]))
+
+
+@pytest.mark.parametrize("arch,dtype,B", [((2, 128, 4, 512, 16), "f32", 65), ((2, 256, 8, 1024, 32), "bf16", 300), ((2, 256, 8, 1024, 32), "bf16", 600),
+                                          ((2, 384, 12, 1536, 48), "f16", 40), ((2, 384, 12, 1536, 48), "f16", 400)])
+def test_compacted_route_replays_from_a_captured_graph(arch, dtype, B):
+    """The row count stays on the device: one graph serves every mask of its batch size."""
+    spec, _, m = _model(arch, dtype)
+    obs, k = cm.make_inputs(spec, B, 1, "uniform")
+    obs, k = obs.to(DEV), k.to(DEV)
+    assert m.auto_route(B) == "ragged"
+    m.forward_stacked(obs, k)                                    # replicas and images
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        lg, v = m.forward_stacked(obs, k)
+    for seed, mask in ((2, "uniform"), (3, "none"), (4, "quarter_empty")):
+        o, kk = cm.make_inputs(spec, B, seed, mask)
+        obs.copy_(o.to(DEV)); k.copy_(kk.to(DEV))
+        g.replay()
+        got = (lg.clone(), v.clone())
+        want = m.forward_stacked(o.to(DEV), kk.to(DEV))          # eager work between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), mask
