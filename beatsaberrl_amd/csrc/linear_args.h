@@ -20,7 +20,7 @@ struct LinArgs {
     // rows counted on the device: base + *extra of them, `rows` their host-side bound (NULL: exactly `rows`)
     const int32_t* extra = nullptr; int64_t base = 0;
     bool vec_ok = false;               // linear_small.hip: filled in by its launch
-    bool res_f32 = false;              // 16-bit operands with an fp32 residual (linear_small.hip alone)
+    bool res_f32 = false;              // 16-bit operands with an fp32 residual, no activation (linear_small.hip alone)
 };
 
 __device__ __forceinline__ int64_t lin_rows(const LinArgs& a) { return a.extra ? a.base + (int64_t)*a.extra : a.rows; }

@@ -32,8 +32,9 @@ template <> struct Mma<F32IO> {
 template <typename DT> constexpr int elem_bytes() { return 2; }
 template <> constexpr int elem_bytes<F32IO>() { return 4; }
 
-// acc[column tile][row tile] of the wave tile at (row0, col0) -> y
-template <typename DT, int ACT, int RT, int CT>
+// acc[column tile][row tile] of the wave tile at (row0, col0) -> y.  RF: the residual is fp32 (ACT_NONE alone; as a run-time switch
+// it cost every other instance 1 % of a 16-bit small batch's forward)
+template <typename DT, int ACT, bool RF, int RT, int CT>
 __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, int64_t row0, int col0, int r16, int g, const f32x4 (&acc)[CT][RT]) {
     constexpr int ES = elem_bytes<DT>();
     // lane holds columns col .. col + 3 of its rows
@@ -56,7 +57,7 @@ __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, i
             for (int e = 0; e < 4; ++e) o[e] = keep_f32(Mma<DT>::template act<ACT>(acc[i][j][e] + bv[e], f32out));
             if (a.vec_ok) {               // M % 4 == 0, aligned rows, no split: 8- / 16-byte pieces
                 if (a.res) {
-                    if (ES == 4 || a.res_f32) {
+                    if (ES == 4 || RF) {
                         const float4 r = *reinterpret_cast<const float4*>(static_cast<const float*>(a.res) + row * a.ldr + col);
                         o[0] += r.x; o[1] += r.y; o[2] += r.z; o[3] += r.w;
                     } else {
@@ -82,7 +83,7 @@ __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, i
                     const int c = col + e;
                     if (c >= a.M) break;
                     float v = o[e];
-                    if (a.res) v += a.res_f32 ? static_cast<const float*>(a.res)[row * a.ldr + c] : Mma<DT>::ld(a.res, row * a.ldr + c);
+                    if (a.res) v += RF ? static_cast<const float*>(a.res)[row * a.ldr + c] : Mma<DT>::ld(a.res, row * a.ldr + c);
                     if (a.gate && !(Mma<DT>::ld(a.gate, row * a.ldgate + c) > 0.f)) v = 0.f;
                     const bool second = a.y2 && c >= a.split;
                     void* dst = second ? a.y2 : a.y;
@@ -96,7 +97,7 @@ __device__ __forceinline__ void small_epilogue(const LinArgs& a, int64_t rows, i
 }
 
 // WR wave rows x 4 / WR wave columns per workgroup
-template <typename DT, int ACT, int RT, int CT, int WR, int PF>
+template <typename DT, int ACT, bool RF, int RT, int CT, int WR, int PF>
 __global__ __launch_bounds__(256) void linear_small_kernel(LinArgs a, int ncb) {
     constexpr int ES = elem_bytes<DT>(), WC = 4 / WR, KF = Mma<DT>::KF, KL = KF / 4;       // KL: k per lane and fragment
     const int64_t rows = lin_rows(a);
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(256) void linear_small_kernel(LinArgs a, int ncb) {
             }
         }
     }
-    small_epilogue<DT, ACT, RT, CT>(a, rows, row0, col0, r16, g, acc);
+    small_epilogue<DT, ACT, RF, RT, CT>(a, rows, row0, col0, r16, g, acc);
 }
 
 // The same tiles with the operands shared through LDS, for K a whole number of 128-byte pieces and enough rows that the
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(256) void linear_small_kernel(LinArgs a, int ncb) {
 __device__ __forceinline__ void lds_block_load(uint32_t voff, const void* sbase, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr));
 }
-template <typename DT, int ACT, int RT, int CT, int NS>
+template <typename DT, int ACT, bool RF, int RT, int CT, int NS>
 __global__ __launch_bounds__(256, 2) void linear_lds_kernel(LinArgs a, int ncb) {
     constexpr int XB = 4 * RT, WB = 4 * CT, NB = XB + WB, NL = NB / 4;           // 1 KB blocks per stage, loads per wave
     constexpr int ES = elem_bytes<DT>();
@@ -230,12 +231,12 @@ __global__ __launch_bounds__(256, 2) void linear_lds_kernel(LinArgs a, int ncb) 
                 for (int j = 0; j < RT; ++j) acc[i][j] = Mma<DT>::go(wf[i], xf[j], acc[i][j]);
         }
     }
-    small_epilogue<DT, ACT, RT, CT>(a, rows, row0 + wr * (16 * RT), col0 + wc * (16 * CT), r16, g, acc);
+    small_epilogue<DT, ACT, RF, RT, CT>(a, rows, row0 + wr * (16 * RT), col0 + wc * (16 * CT), r16, g, acc);
 }
-template <typename DT, int ACT, int RT, int CT, int NS>
+template <typename DT, int ACT, bool RF, int RT, int CT, int NS>
 bool go_lds(const LinArgs& a, hipStream_t st) {
     constexpr int BYTES = NS * 4 * (RT + CT) * 1024;
-    auto kern = linear_lds_kernel<DT, ACT, RT, CT, NS>;
+    auto kern = linear_lds_kernel<DT, ACT, RF, RT, CT, NS>;
     static const bool ready = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES) == hipSuccess;
     if (!ready) { (void)hipGetLastError(); return false; }
     const int ncb = (a.M + 32 * CT - 1) / (32 * CT);
@@ -243,31 +244,32 @@ bool go_lds(const LinArgs& a, hipStream_t st) {
     return true;
 }
 
-template <typename DT, int ACT, int RT, int CT, int WR, int PF>
+template <typename DT, int ACT, bool RF, int RT, int CT, int WR, int PF>
 void go(const LinArgs& a, hipStream_t st) {
     const int ncb = (a.M + CT * 16 * (4 / WR) - 1) / (CT * 16 * (4 / WR));
     const int64_t nrb = (a.rows + RT * 16 * WR - 1) / (RT * 16 * WR);
-    hipLaunchKernelGGL((linear_small_kernel<DT, ACT, RT, CT, WR, PF>), dim3((unsigned)(nrb * ncb)), dim3(256), 0, st, a, ncb);
+    hipLaunchKernelGGL((linear_small_kernel<DT, ACT, RF, RT, CT, WR, PF>), dim3((unsigned)(nrb * ncb)), dim3(256), 0, st, a, ncb);
 }
 
-template <typename DT, int ACT>
+template <typename DT, int ACT, bool RF = false>
 void pick(const LinArgs& a, hipStream_t st) {
     const int64_t cus = bsrl_cus(), wg64 = ((a.rows + 63) / 64) * ((a.M + 63) / 64);
     if (a.K * elem_bytes<DT>() % 128 == 0 && a.rows > 16 && a.ldx <= (1 << 22) && a.K <= (1 << 22)) {
         // 32 x 32 tiles until 64 x 64 ones cover the chip, 64 x 128 once three of those per CU would queue
-        if (wg64 >= 3 * cus ? go_lds<DT, ACT, 2, 4, 3>(a, st) : wg64 >= cus ? go_lds<DT, ACT, 2, 2, 4>(a, st)
-                                                                                 : go_lds<DT, ACT, 1, 1, 8>(a, st)) return;
+        if (wg64 >= 3 * cus ? go_lds<DT, ACT, RF, 2, 4, 3>(a, st) : wg64 >= cus ? go_lds<DT, ACT, RF, 2, 2, 4>(a, st)
+                                                                                 : go_lds<DT, ACT, RF, 1, 1, 8>(a, st)) return;
     }
     // the largest tile that still gives every CU a workgroup: 64 x 64, 32 x 64, 32 x 32; one row tile: 16 x 64
-    if (a.rows <= 16) go<DT, ACT, 1, 1, 1, 12>(a, st);
-    else if (wg64 >= cus) go<DT, ACT, 2, 2, 2, 6>(a, st);
-    else if (2 * wg64 >= cus) go<DT, ACT, 1, 2, 2, 8>(a, st);
-    else go<DT, ACT, 1, 1, 2, 12>(a, st);
+    if (a.rows <= 16) go<DT, ACT, RF, 1, 1, 1, 12>(a, st);
+    else if (wg64 >= cus) go<DT, ACT, RF, 2, 2, 2, 6>(a, st);
+    else if (2 * wg64 >= cus) go<DT, ACT, RF, 1, 2, 2, 8>(a, st);
+    else go<DT, ACT, RF, 1, 1, 2, 12>(a, st);
 }
 template <typename DT>
 void by_act(const LinArgs& a, int act, hipStream_t st) {
     if (act == BSRL_ACT_RELU) pick<DT, BSRL_ACT_RELU>(a, st);
     else if (act == BSRL_ACT_GELU) pick<DT, BSRL_ACT_GELU>(a, st);
+    else if constexpr (elem_bytes<DT>() == 2) { if (a.res_f32) pick<DT, BSRL_ACT_NONE, true>(a, st); else pick<DT, BSRL_ACT_NONE>(a, st); }
     else pick<DT, BSRL_ACT_NONE>(a, st);
 }
 
@@ -276,6 +278,7 @@ void by_act(const LinArgs& a, int act, hipStream_t st) {
 bool bsrl_linear_small(const LinArgs& a_, int act, int dtype, hipStream_t st) {
     const int es = dtype == BSRL_F32 ? 4 : 2, per = 16 / es;           // elements per 16-byte lane piece
     LinArgs a = a_;
+    if (a.res_f32 && act != BSRL_ACT_NONE) return false;
     if (a.K % per != 0 || a.ldx % per != 0 || !bsrl_aligned(a.x, 16) || !bsrl_aligned(a.w, 16)) return false;
     if (((a.rows + 31) / 32) * (int64_t)((a.M + 31) / 32) > 0x3fffffff) return false;
     const int osz = a.out_f32 ? 4 : es;
