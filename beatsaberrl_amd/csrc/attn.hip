@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void attn_f32_mfma_kernel(F32AttnArgs f) {
     const int nkt = (T + 15) >> 4, nqt = (TQ + 15) >> 4;
     f32x4 kf[NK][DC], vf[NK][DC];
     float kb[NK][4];
-    const int nv = a.n_valid ? a.n_valid[b] : T;
+    const int nv = a.n_valid ? a.n_valid[b] : T, lim = nv < T ? nv : T - 1;        // the last key that is looked at, whatever those past it hold
 #pragma unroll
     for (int kt = 0; kt < NK; ++kt) {
         if (kt < nkt) {
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void attn_f32_mfma_kernel(F32AttnArgs f) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int key = kt * 16 + 4 * g + i;
-            const bool in = kt < nkt && key < T && key <= nv;        // a key past n_valid is never looked at, whatever it holds
+            const bool in = key <= lim;
 #pragma unroll
             for (int c = 0; c < DC; ++c) vf[kt][c][i] = in ? vp[row(key, a.v_bs, a.v_rs) + 16 * c + r16] : 0.f;
             kb[kt][i] = !in ? -INFINITY : a.key_bias ? static_cast<const float*>(a.key_bias)[b * a.T + key] : 0.f;
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) void attn_f32_mfma_kernel(F32AttnArgs f) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = kt * 16 + 4 * g + i;
-                s[kt][i] = key < T && key <= nv ? s[kt][i] * a.scale + kb[kt][i] : -INFINITY;
+                s[kt][i] = key <= lim ? s[kt][i] * a.scale + kb[kt][i] : -INFINITY;
                 m = fmaxf(m, s[kt][i]);
             }
         }
