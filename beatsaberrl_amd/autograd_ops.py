@@ -378,7 +378,6 @@ class NoteTrainPlan:
             end = offsets[i] + n[i]
         if self.total > end:
             self.sizes.append(self.total - end)
-        self.param_shapes = [torch.Size(s) for s in shapes]
         self.shapes = [tuple(s) if len(s) > 1 else None for s in shapes]
         self.heads, self.critic = range(16 + 16 * self.desc.n_blocks + 10, len(shapes) - 16), range(len(shapes) - 16, len(shapes))
         # the masters that the backward reads (its matrices are the forward's 16-bit copies): the LayerNorm scales

@@ -317,7 +317,7 @@ def build_head_gears(n_gears: int) -> tuple:
 
 
 class NotePolicy(nn.Module):
-    _train_plan_cache = _native_cache = None     # of a module that was pickled before it had them
+    _train_plan_cache = _native_cache = _shapes_kept = None     # of a module that was pickled before it had them
 
     def __init__(self, embed: int = 128, trunk_dim: int = 256, encoder: str = "transformer", n_blocks: int = 3,
                  n_heads: int = 4, n_gears: int = 3, ffn_mult: int = 4, note_geo: bool = False,
@@ -569,21 +569,26 @@ class NotePolicy(nn.Module):
             if self.update_values not in ("rollout", "own"):
                 raise ValueError(f"update_values must be 'rollout' or 'own', got {self.update_values!r}")
             if self.update_values == "rollout" and self.fp16 and not self.rollout_matches_update:
+                arch = self._native_desc(self.stream_dtype)
+                params = None if arch is None else self._native_params(arch)
                 with torch.no_grad():
-                    r_out, r_value = self.forward_stacked(obs)       # the rollout's own routes, grad-free
-                plan = self._train_plan()
-                params = None if plan is None else self._train_params()
-                if params is not None and [p.shape for p in params] == plan.param_shapes and all(p.is_cuda for p in params):
+                    r_out, r_value = self._rollout(obs, arch, params)       # the rollout's own routes, grad-free
+                plan = None if params is None else self._train_plan(arch)
+                if plan is not None:
                     return self._forward_train_native(plan, params, obs, r_out, r_value)
                 out, value = self._forward_train(obs)
                 return _ValuesOf.apply(out, r_out), _ValuesOf.apply(value, r_value)
             return self._forward_train(obs)
+        return self._rollout(obs)
+
+    def _rollout(self, obs, arch=None, params=None):
+        """The forward-only routes.  arch, params: `_native_desc` and `_native_params` of this very call, where the caller has them."""
         with contextlib.ExitStack() as modes:
             if self.fp16 and self.fp16_accum != "off":
                 modes.enter_context(_fl.fp16_accum(self.fp16_accum))
             if self.fp16 and self.fused_ffn != "off":
                 modes.enter_context(_fl.ffn_fusion(self.fused_ffn))
-            return self._forward_stacked(obs)
+            return self._forward_stacked(obs, arch, params)
 
     # ---- the fused routes as native calls ------------------------------------------------------
     def _native_desc(self, dt):
@@ -617,6 +622,9 @@ class NotePolicy(nn.Module):
 
     def _native_shapes(self, c):
         """Shapes of `_train_params` for the descriptor c."""
+        key, kept = (tuple(c.values()), self.head_sizes), self._shapes_kept
+        if kept is not None and kept[0] == key:
+            return kept[1]
         d, ffn, tr, hid = c["d"], c["ffn"], c["trunk"], c["hidden"]
         lin, ln = lambda m, k: [(m, k), (m,)], lambda n: [(n,), (n,)]
         out = []
@@ -626,15 +634,28 @@ class NotePolicy(nn.Module):
         out += lin(tr, self.n_lead * d) + ln(tr) + lin(hid, tr) + lin(tr, hid) + ln(tr)
         for k in self.head_sizes:
             out += lin(k, tr)
-        return out + ln(d) + 4 * lin(d, d) + lin(tr, d + tr) + lin(tr, tr) + lin(c["bins"], tr)
+        out += ln(d) + 4 * lin(d, d) + lin(tr, d + tr) + lin(tr, tr) + lin(c["bins"], tr)
+        self._shapes_kept = (key, out)
+        return out
 
-    def _native_image(self, dt):
+    def _native_params(self, arch):
+        """`_train_params` where every one is what goes in by pointer: contiguous fp32 of the descriptor's shape, all on one GPU;
+        else None."""
+        params, at = self._train_params(), self.critic_ln.weight.get_device()
+        if params is None or at < 0:
+            return None
+        for p, s in zip(params, self._native_shapes(arch)):
+            if p.shape != s or p.dtype is not torch.float32 or p.get_device() != at or not p.is_contiguous():
+                return None
+        return params
+
+    def _native_image(self, dt, arch=None, params=None):
         """(descriptor, weight image) of the native forward for the current weights version, or None where the forward runs op
         by op.  The image is rebuilt IN PLACE, as `blocks_image` is: its address is stable under a captured graph."""
         if (dt is torch.float32 or not self.fused_blocks_ok(dt) or not self.critic_pool
                 or not ops.critic_pool_supported(self.n_lead + N_NOTE_SLOTS, self.embed, self.n_heads, dt)):
             return None
-        arch = self._native_desc(dt)
+        arch = arch or self._native_desc(dt)
         if arch is None:
             return None
         dev, key = self.critic_ln.weight.device, tuple(arch.values())
@@ -646,9 +667,8 @@ class NotePolicy(nn.Module):
         if c[2].numel() == 0:
             return None
         if c[0] != _fl._weights_version:
-            params = self._train_params()
-            if params is None or [p.shape for p in params] != self._native_shapes(arch) or any(
-                    p.dtype is not torch.float32 or not p.is_contiguous() or p.device != dev for p in params):
+            params = params or self._native_params(arch)
+            if params is None:
                 return None
             ptrs = (ctypes.c_void_p * len(params))(*[p.data_ptr() for p in params])
             gears = (ctypes.c_int32 * N_ACTION_HEADS)(*self.head_sizes)
@@ -719,11 +739,11 @@ class NotePolicy(nn.Module):
         self._value_logits = None
         return logits, value
 
-    def _forward_stacked(self, obs):
+    def _forward_stacked(self, obs, arch=None, params=None):
         dt = self.stream_dtype if self.fp16 else torch.float32
         B, d = obs.shape[0], self.embed
         if obs.shape[0]:
-            native = self._native_image(dt)
+            native = self._native_image(dt, arch, params)
             masters = None if native is None else self._native_masters(native[0])
             if masters is not None:
                 if obs.dtype is not torch.float32 and obs.dtype is not dt:
@@ -887,12 +907,12 @@ class NotePolicy(nn.Module):
             return None
         return None if any(p is None for p in out) else out
 
-    def _train_plan(self):
+    def _train_plan(self, arch=None):
         """The native update's plan, or None where the update runs op by op: an architecture without a place in it, a fused FFN
         asked for, parameters of other shapes or kinds."""
         if self._gear_idx is not None or self.fused_ffn != "off":
             return None
-        arch = self._native_desc(self.stream_dtype)
+        arch = arch or self._native_desc(self.stream_dtype)
         if arch is None:
             return None
         c, key = self._train_plan_cache, tuple(arch.values())
@@ -907,7 +927,6 @@ class NotePolicy(nn.Module):
             obs = obs.float()
         if obs.stride(1) != 1:
             obs = obs.contiguous()
-        params = [p if p.dtype is torch.float32 and p.is_contiguous() else p.float().contiguous() for p in params]
         out, value, self._value_logits = NoteTrainFn.apply(plan, obs, self._saber_idx32, self._body_idx32, self.value_centers,
                                                            r_out, r_value, *params)
         return out, value

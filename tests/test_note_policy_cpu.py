@@ -123,3 +123,4 @@ def test_native_calls_take_only_parameters_of_the_expected_shapes():
     m = _small()
     m.heads[3] = nn.Linear(64, 7)
     assert [p.shape for p in m._train_params()] != m._native_shapes(m._native_desc(torch.float16))
+    assert m._native_params(m._native_desc(torch.float16)) is None          # nor on the host
