@@ -144,3 +144,18 @@ def test_compacted_route_replays_from_a_captured_graph(arch, dtype, B):
         want = m.forward_stacked(o.to(DEV), kk.to(DEV))          # eager work between the replays
         torch.cuda.synchronize()
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), mask
+
+
+@pytest.mark.parametrize("dtype,tol", [("f16", 4e-3), ("bf16", 2e-2)])
+@pytest.mark.parametrize("B", [1, 2, 5, 17, 33, 64, 129])
+def test_by_op_fp32_stream_at_the_edges_of_its_tiles(B, dtype, tol):
+    """1 to ~2000 rows with every remainder of the 16-, 32- and 64-row tiles among them, against the block-stack kernel (the same
+    rounding points; tolerance: both are within the type's class of the fp32 model)."""
+    spec, _, m = _model((3, 256, 8, 544, 32), dtype)
+    obs, k = cm.make_inputs(spec, B, B, "uniform")
+    obs, k = obs.to(DEV), k.to(DEV)
+    a, b = _out(m.forward_stacked(obs, k, route="ragged")), _out(m.forward_stacked(obs, k, route="blocks"))
+    assert (a - b).norm() <= tol * b.norm()
+    full = _out(m.forward_stacked(obs, None, route="ragged"))
+    m.prune_final = False
+    assert (_out(m.forward_stacked(obs, None, route="ragged")) - full).norm() <= tol * full.norm()
