@@ -96,6 +96,8 @@ SIGNATURES = {
     "bsrl_cfg_workspace_size": (_i64, [C.POINTER(CfgDesc), _i64]),
     "bsrl_cfg_forward": (_i32, [C.POINTER(CfgDesc), _p, _p, _i64, _i32, _p, _p, _p, _i64, _p, _i64, _p]),
     "bsrl_cfg_forward_static": (_i32, [C.POINTER(CfgDesc), _p, _p, _i64, _i32, _p, _p, _p, _i64, _p]),
+    "bsrl_cfg_rows_pack_size": (_i64, [C.POINTER(CfgDesc)]),
+    "bsrl_cfg_rows_pack": (_i32, [C.POINTER(CfgDesc), C.POINTER(CfgRowsWeights), _p, _p]),
     "bsrl_cfg_rows_workspace_size": (_i64, [C.POINTER(CfgDesc), _i64, _i32]),
     "bsrl_cfg_rows_forward": (_i32, [C.POINTER(CfgDesc), C.POINTER(CfgRowsWeights), _p, _i64, _i32, _p, _p, _p, _i64, _i32, _p, _i64, _p]),
     "bsrl_blocks_pack_size": (_i64, [C.POINTER(BlocksDesc)]),

@@ -2,6 +2,7 @@
 // Two forms of a block: attention + one kernel for the rest (block_tail.h) where images are given, else one kernel per op.
 // The host's share of a forward is this function's launches; composed in Python from the same entry points it was 270 us per
 // forward at two layers, which is what a small batch then took.
+#include "cfg_env_f32.h"
 #include "linear_args.h"
 
 namespace {
@@ -44,6 +45,15 @@ extern "C" int64_t bsrl_cfg_rows_workspace_size(const bsrl_cfg_desc* d, int64_t 
     return (int64_t)RowsPlan(*d, B, tail != 0, nullptr).bytes;
 }
 
+extern "C" int64_t bsrl_cfg_rows_pack_size(const bsrl_cfg_desc* d) { return rows_desc_ok(d) ? bsrl_cfg_env_f32_pack_size(d) : 0; }
+
+extern "C" int bsrl_cfg_rows_pack(const bsrl_cfg_desc* d, const bsrl_cfg_rows_weights* w, void* img, bsrl_stream stream) {
+    if (!rows_desc_ok(d) || !w || !img) BSRL_FAIL(BSRL_EINVAL, "bsrl_cfg_rows_pack: null pointer or bad shape");
+    if (bsrl_cfg_env_f32_pack_size(d) == 0) return BSRL_UNSUPPORTED;
+    if (!bsrl_aligned(img, 16)) BSRL_FAIL(BSRL_EINVAL, "bsrl_cfg_rows_pack: image must be 16-byte aligned");
+    return bsrl_cfg_env_f32_pack(d, w, img, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows_weights* w, const void* obs, int64_t obs_ld,
                                      int obs_dtype, const int32_t* n_valid, float* logits, float* value, int64_t B, int prune,
                                      void* workspace, int64_t workspace_bytes, bsrl_stream stream) {
@@ -58,6 +68,17 @@ extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int32_t* extra = p.noff + B;
     int rc;
+    // One launch, an env's rows in LDS.  It computes all of an env's token slots, the launches below the attendable ones alone: with half of
+    // them masked these win from about ten envs per CU on (us, one launch | launches: 256 envs 42 | 107, 2048 230 | 255, 4096 455 | 394;
+    // no mask: 256 envs 42 | 113, 4096 456 | 554, 16384 1803 | 2041)
+    if (dt == BSRL_F32 && obs_dtype == BSRL_F32 && prune && w->lead_img && bsrl_aligned(w->lead_img, 16) && bsrl_cfg_env_f32_pack_size(d) > 0 &&
+        (!n_valid || B <= 10 * (int64_t)bsrl_cus())) {
+        const CfgEnvF32Args e{*w, static_cast<const float*>(obs), obs_ld, n_valid, logits, value, (int)B, L, d->T, (int)(29 * d->n_gears + 1), d->final_ln, d->prop_dim, d->obj_dim};
+        if (bsrl_cfg_env_f32(d, e, st)) {
+            BSRL_CHECK_LAUNCH("bsrl_cfg_rows_forward");
+            return BSRL_OK;
+        }
+    }
 #define STEP(call) do { if ((rc = (call)) != BSRL_OK) return rc; } while (0)
     auto at = [&](const void* q, int64_t elems) { return static_cast<const char*>(q) + elems * es; };
     // y = act(x W^T + b) (+ res) on rows [+ *extra] rows; res_f32, y_f32: that operand is fp32
