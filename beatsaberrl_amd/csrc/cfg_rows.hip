@@ -3,6 +3,7 @@
 // The host's share of a forward is this function's launches; composed in Python from the same entry points it was 270 us per
 // forward at two layers, which is what a small batch then took.
 #include "cfg_env_f32.h"
+#include "cfg_env_rows.h"
 #include "linear_args.h"
 
 namespace {
@@ -18,6 +19,7 @@ bool stream_f32(const bsrl_cfg_desc& d) { return d.d == 256 && d.dtype != BSRL_F
 
 struct RowsPlan {
     int32_t* noff; void *x0, *x1, *h, *q, *att, *hid, *lead; size_t bytes;
+    u16* ex1; float* epart;                          // the few-envs form (in the place of the others)
     RowsPlan(const bsrl_cfg_desc& d, int64_t B, bool tail, char* ws) {
         const size_t es = d.dtype == BSRL_F32 ? 4 : 2, R = (size_t)B * d.T, D = d.d, xs = stream_f32(d) ? 4 : es;
         Bump b{ws};
@@ -30,6 +32,13 @@ struct RowsPlan {
         hid = b.take(tail ? 0 : R * d.ffn * es);
         lead = b.take((size_t)B * D * es);
         bytes = b.used;
+        if (!tail && bsrl_cfg_env_rows_pack_size(&d) > 0) {
+            Bump e{ws};
+            e.take((B + 1) * 4);
+            ex1 = static_cast<u16*>(e.take((R + B) * D * 2));
+            epart = static_cast<float*>(e.take(4 * R * D * 4));
+            if (e.used > bytes) bytes = e.used;
+        }
     }
 };
 
@@ -45,13 +54,15 @@ extern "C" int64_t bsrl_cfg_rows_workspace_size(const bsrl_cfg_desc* d, int64_t 
     return (int64_t)RowsPlan(*d, B, tail != 0, nullptr).bytes;
 }
 
-extern "C" int64_t bsrl_cfg_rows_pack_size(const bsrl_cfg_desc* d) { return rows_desc_ok(d) ? bsrl_cfg_env_f32_pack_size(d) : 0; }
+extern "C" int64_t bsrl_cfg_rows_pack_size(const bsrl_cfg_desc* d) {
+    return !rows_desc_ok(d) ? 0 : d->dtype == BSRL_F32 ? bsrl_cfg_env_f32_pack_size(d) : bsrl_cfg_env_rows_pack_size(d);
+}
 
 extern "C" int bsrl_cfg_rows_pack(const bsrl_cfg_desc* d, const bsrl_cfg_rows_weights* w, void* img, bsrl_stream stream) {
     if (!rows_desc_ok(d) || !w || !img) BSRL_FAIL(BSRL_EINVAL, "bsrl_cfg_rows_pack: null pointer or bad shape");
-    if (bsrl_cfg_env_f32_pack_size(d) == 0) return BSRL_UNSUPPORTED;
+    if (bsrl_cfg_rows_pack_size(d) == 0) return BSRL_UNSUPPORTED;
     if (!bsrl_aligned(img, 16)) BSRL_FAIL(BSRL_EINVAL, "bsrl_cfg_rows_pack: image must be 16-byte aligned");
-    return bsrl_cfg_env_f32_pack(d, w, img, static_cast<hipStream_t>(stream));
+    return d->dtype == BSRL_F32 ? bsrl_cfg_env_f32_pack(d, w, img, static_cast<hipStream_t>(stream)) : bsrl_cfg_env_rows_pack(d, w, img, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows_weights* w, const void* obs, int64_t obs_ld,
@@ -93,6 +104,11 @@ extern "C" int bsrl_cfg_rows_forward(const bsrl_cfg_desc* d, const bsrl_cfg_rows
         return (int)BSRL_OK;
     };
     STEP(bsrl_token_offsets(n_valid, B, opt, p.noff, stream));
+    if (!tail && prune && bsrl_cfg_env_rows_ok(d, w)) {
+        const CfgEnvRowsArgs e{*w, obs, obs_ld, p.noff, p.ex1, p.epart, logits, value, (int)B, L, d->T, (int)(29 * d->n_gears + 1), d->final_ln, d->prop_dim, d->obj_dim,
+                               obs_dtype == BSRL_F32};
+        return bsrl_cfg_env_rows(d, e, st);
+    }
     STEP(bsrl_cfg_tokens(obs, obs_ld, obs_dtype, w->prop_w, w->prop_b, w->obj_w, w->obj_b, p.noff, p.x0, B, D, d->prop_dim, d->obj_dim, dt, stream));
     const float eps = 1e-5f;
     void *x = p.x0, *xn = p.x1;

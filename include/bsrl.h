@@ -382,8 +382,9 @@ typedef struct {
         const void* tail_img;
     } blk[BSRL_MAX_LAYERS];
 } bsrl_cfg_rows_weights;
-/* fp32, d = 128, 4 heads, ffn = 512, T <= 16: an image of the matrices (bsrl_cfg_rows_pack_size bytes, 16-byte
- * aligned; 0 = the model has none) as lead_img makes a pruned forward of fp32 observations one launch. */
+/* Without tail images, an image of the matrices (bsrl_cfg_rows_pack_size bytes, 16-byte aligned; 0 = the model has
+ * none) as lead_img makes a pruned forward fewer launches: one in fp32 (fp32 observations) at d = 128, 4 heads, ffn =
+ * 512, T <= 16; two per block in 16 bit at d = 384, 12 heads, ffn = 1536. */
 int64_t bsrl_cfg_rows_pack_size(const bsrl_cfg_desc* d);
 int bsrl_cfg_rows_pack(const bsrl_cfg_desc* d, const bsrl_cfg_rows_weights* w, void* img, bsrl_stream stream);
 int64_t bsrl_cfg_rows_workspace_size(const bsrl_cfg_desc* d, int64_t B, int tail);
