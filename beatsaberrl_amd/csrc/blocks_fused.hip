@@ -35,6 +35,7 @@
 // and the stream(s) out.
 #include "block_stage.h"
 #include "blocks_latency.h"
+#include "blocks_pair.h"
 
 namespace {
 
@@ -43,6 +44,7 @@ struct BlkArgs {
     const u16* x_in; const u16* key_bias; u16* x_res; u16* x_out;
     int64_t B; int n_layers, F, T, n_queries, total_stages;
     int per;                                  // blocks_env_kernel: envs per workgroup, 1 .. 8
+    BlocksPairPlan plan;                      // d = 192, tiles not null: nothing to do where pairs pay (blocks_pair.hip)
 };
 
 // Weight-stage pipeline: stage s lives in ring slot s & 1; its global loads were issued three
@@ -85,6 +87,7 @@ __global__ __launch_bounds__(512) void blocks_kernel(BlkArgs a) {
     const int r16 = lane & 15, g = lane >> 4;
     const int el = wave >> 1, rt = wave & 1;
     const float scale_l2e = (DH == 32 ? 0.17677669529663688110f : 0.14433756729740644113f) * 1.44269504088896340736f;
+    if (D == 192 && a.plan.tiles && blocks_pairs_pay(a.plan, blocks_pair_tiles(a.plan, lane))) return;
     const int64_t ntiles = (a.B + 3) / 4;
 
     const uint2* img = a.frags;
@@ -406,6 +409,7 @@ __global__ __launch_bounds__(512, 1) void blocks_env_kernel(BlkArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const float scale_l2e = (DH == 32 ? 0.17677669529663688110f : 0.14433756729740644113f) * 1.44269504088896340736f;
+    if (D == 192 && a.plan.tiles && blocks_pairs_pay(a.plan, blocks_pair_tiles(a.plan, lane))) return;
     const int64_t ntiles = (a.B + a.per - 1) / a.per;
     const int ring_off_u4 = (a.n_layers * G::lv_size(a.F) / 4 + 63) & ~63;
     const uint4* ring = reinterpret_cast<const uint4*>(bvl4) + ring_off_u4;
@@ -909,6 +913,11 @@ extern "C" int bsrl_blocks_pack(const bsrl_blocks_desc* d, const bsrl_blocks_par
 
 extern "C" int bsrl_blocks_forward(const bsrl_blocks_desc* d, const void* packed, const void* x_in, const void* key_bias,
                                    void* x_res, void* x_out, int64_t B, bsrl_stream stream) {
+    return bsrl_blocks_unless(d, packed, x_in, key_bias, x_res, x_out, B, nullptr, stream);
+}
+
+int bsrl_blocks_unless(const bsrl_blocks_desc* d, const void* packed, const void* x_in, const void* key_bias, void* x_res, void* x_out, int64_t B,
+                       const BlocksPairPlan* plan, bsrl_stream stream) {
     if (!d || !packed || !x_in || !key_bias || !x_out) BSRL_FAIL(BSRL_EINVAL, "bsrl_blocks_forward: null pointer");
     if (!blocks_shape_ok(d)) return BSRL_UNSUPPORTED;
     if (B < 0) BSRL_FAIL(BSRL_EINVAL, "bsrl_blocks_forward: B < 0");
@@ -922,6 +931,7 @@ extern "C" int bsrl_blocks_forward(const bsrl_blocks_desc* d, const void* packed
     a.x_res = static_cast<u16*>(x_res); a.x_out = static_cast<u16*>(x_out);
     a.B = B; a.n_layers = d->n_layers; a.F = d->ffn; a.T = d->T; a.n_queries = d->n_queries;
     a.total_stages = (int)blocks_stages(d);
+    a.plan = plan ? *plan : BlocksPairPlan{};
     hipStream_t st = static_cast<hipStream_t>(stream);
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||

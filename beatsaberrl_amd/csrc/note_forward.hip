@@ -7,6 +7,7 @@
 // is copied together.  Every kernel and its operands are those of the op-by-op forward: the same bits.
 // One env, recipe shape: 419 -> 180 us, 157 with the chains of note_readout.hip, 80 of them the block stack (blocks_latency.hip: from
 // 206); a captured rollout step of 2048 envs, default shape: 217 -> 180 us, 151 with the chains; the update of 1500 envs: 3.7 -> 3.3 ms.
+#include "blocks_pair.h"
 #include "note_pack.h"
 #include "note_readout.h"
 
@@ -42,7 +43,7 @@ struct Image {
 };
 
 struct Work {
-    u16 *in[4], *bias, *x, *lead, *xres, *t, *u, *r, *t2, *z, *ln, *q, *qk, *pool, *att, *c1, *c2; float* vl; size_t bytes;
+    u16 *in[4], *bias, *x, *lead, *xres, *t, *u, *r, *t2, *z, *ln, *q, *qk, *pool, *att, *c1, *c2; float* vl; int4* pairs; int* tiles; size_t bytes;
     Work(const bsrl_note_desc& d, int64_t B, char* base) {
         Bump b{base};
         const int64_t D = d.d, TR = d.trunk, HD = (int64_t)d.n_heads * D;
@@ -52,6 +53,8 @@ struct Work {
         t = mat(B, TR); u = mat(B, TR); r = mat(B, d.hidden); t2 = mat(B, TR); z = mat(B, D + TR);
         ln = mat(B, D); q = mat(B, D); qk = mat(B, HD); pool = mat(B, HD); att = mat(B, D); c1 = mat(B, TR); c2 = mat(B, TR);
         vl = b.take<float>((size_t)(B * d.bins));
+        pairs = b.take<int4>((size_t)(bsrl_blocks_pair_chunks(B) * BLOCKS_PAIR_CHUNK));
+        tiles = b.take<int>((size_t)bsrl_blocks_pair_chunks(B));
         bytes = b.used;
     }
 };
@@ -219,7 +222,13 @@ extern "C" int bsrl_note_forward(const bsrl_note_desc* d, const float* const* pa
         }
         if (!bsrl_mlp2_stream(e4, 4, PITCH, dt, st)) return BSRL_UNSUPPORTED;
         const bsrl_blocks_desc s = stack_of(*d);
-        STEP(bsrl_blocks_forward(&s, m.blocks, w.x, w.bias, w.xres, w.lead, B, stream));
+        const int64_t frags = bsrl_blocks_pack_size(&s) - (int64_t)s.n_layers * (9 * D + s.ffn) * 4;
+        const BlocksPairPlan plan{w.tiles, (int)bsrl_blocks_pair_chunks(B), bsrl_cus(), B};
+        const BlocksPairArgs p{static_cast<const uint4*>(m.blocks), reinterpret_cast<const float*>(static_cast<const char*>(m.blocks) + frags), w.x, w.bias, w.xres,
+                               w.lead, w.pairs, plan, s.n_layers, s.ffn, T_TOK, N_LEAD, (int)(frags / (D / 16 * 1024))};
+        const int rc = bsrl_blocks_pair(p, d->d, dt, st);
+        if (rc != BSRL_UNSUPPORTED) STEP(rc);
+        STEP(bsrl_blocks_unless(&s, m.blocks, w.x, w.bias, w.xres, w.lead, B, rc == BSRL_OK ? &plan : nullptr, stream));
     }
     if ((parts & READOUT_PARTS) == READOUT_PARTS) {
         const Readout r(*d, params, m, w, centers, logits, value, B);
