@@ -278,11 +278,17 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
             stage(1, up_into(acc0), idle);
             load_bias(B1, 1, false);
             static_for<0, NH>([&](auto k_) __attribute__((always_inline)) { act_step(k_, acc0, hid0); });
-            for (int ch = 0; ch + 1 < nch; ++ch) {
-                stage(2, up_into(acc1), act_slots(KH{}, KT{}, acc0, hid0));       // W1(ch + 1); W2(ch) is an even stage
+            auto half = [&](int ch, Acc& ca, Hid& ha, Acc& na, Hid& hb) __attribute__((always_inline)) {
+                stage(2, up_into(na), act_slots(KH{}, KT{}, ca, ha));             // W1(ch + 1); W2(ch) is an even stage
                 if (ch + 2 < nch) load_bias(B1, ch + 2, false);
-                stage(1, down(hid0), act_slots(K0{}, KH{}, acc1, hid1));          // W2(ch); an odd stage follows
-                // the next chunk takes this one's place (only what its second half still needs survives as moves)
+                stage(1, down(ha), act_slots(K0{}, KH{}, na, hb));                // W2(ch); an odd stage follows
+            };
+            // two chunks a round: they alternate by name, nothing moves (with one chunk a round, whose accumulators and hidden then took
+            // the other's place, 12 RT moves stood between two chunks: 4 blocks at d = 256, 541k rows, 4.91 -> 4.58 ms; at d = 384 1 %)
+            int ch = 0;
+            for (; ch + 2 < nch; ch += 2) { half(ch, acc0, hid0, acc1, hid1); half(ch + 1, acc1, hid1, acc0, hid0); }
+            if (ch + 1 < nch) {
+                half(ch, acc0, hid0, acc1, hid1);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) { acc0[0][rt] = acc1[0][rt]; acc0[1][rt] = acc1[1][rt]; hid0[rt] = hid1[rt]; }
             }
@@ -339,24 +345,35 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
         }
         if (LN && a.nq > 0) {
             // qo = ho Wn^T + bn: nq stages of 32 columns in the up-projection's form (the first is admitted and its first
-            // fragments are in flight), each stored as it completes
+            // fragments are in flight).  A stage's columns are packed and stored behind the MFMAs of the next one, whose
+            // successor's bias is read behind them too (together: d = 256 as above 4.58 -> 4.55 ms, six at d = 384 31.65 -> 31.28; the q|k|v launch of the first
+            // block is bound by its MFMAs, loads and LayerNorm: without its stores 16 % faster, without the weight stream 16 %)
             const int ldq = 32 * a.nq;
-            auto q_store = [&](int sq) __attribute__((always_inline)) {
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-                    const int64_t row = row0 + 16 * rt + r16;
-                    if (row < rows) {       // the stage's columns in the paired order: 16 bytes per lane
-                        uint4 v;
-                        v.x = bpack2<DT>(acc0[0][rt][0], acc0[0][rt][1]); v.y = bpack2<DT>(acc0[0][rt][2], acc0[0][rt][3]);
-                        v.z = bpack2<DT>(acc0[1][rt][0], acc0[1][rt][1]); v.w = bpack2<DT>(acc0[1][rt][2], acc0[1][rt][3]);
-                        *reinterpret_cast<uint4*>(a.qo + row * ldq + 32 * sq + 8 * g) = v;
-                    }
-                }
+            u16* const qrow = a.qo + (row0 + r16) * ldq + 8 * g;
+            uint4 qv;
+            auto q_step = [&](auto k_, int sq, Acc& acc) __attribute__((always_inline)) {      // three steps per row tile
+                constexpr int rt = decltype(k_)::value / 3, step = decltype(k_)::value % 3;
+                // the stage's columns in the paired order: 16 bytes per lane
+                if constexpr (step == 0) { qv.x = bpack2<DT>(acc[0][rt][0], acc[0][rt][1]); qv.y = bpack2<DT>(acc[0][rt][2], acc[0][rt][3]); }
+                if constexpr (step == 1) { qv.z = bpack2<DT>(acc[1][rt][0], acc[1][rt][1]); qv.w = bpack2<DT>(acc[1][rt][2], acc[1][rt][3]); }
+                if constexpr (step == 2) { if (row0 + 16 * rt + r16 < rows) *reinterpret_cast<uint4*>(qrow + (int64_t)16 * rt * ldq + 32 * sq) = qv; }
             };
-            for (int sq = 0; sq < a.nq; sq += 2) {       // nq is even: an even stage, then an odd one
-                load_bias(BN, sq, true); stage(1, up_into(acc0), idle); q_store(sq);
-                load_bias(BN, sq + 1, true); stage(sq + 2 < a.nq ? 2 : 0, up_into(acc0), idle); q_store(sq + 1);
+            auto q_slots = [&](int sq, Acc& acc) __attribute__((always_inline)) {
+                return [&, sq](auto s_) __attribute__((always_inline)) {
+                    constexpr int n = 3 * RT, NS = SF * RT, s = decltype(s_)::value;
+                    if constexpr (s == 4 * RT) load_bias(BN, sq + 2 < a.nq ? sq + 2 : 0, true);       // (the first 2 RT MFMAs took this stage's)
+                    if constexpr (s >= NS / 4) static_for<(s - NS / 4) * n / (NS - NS / 4), (s + 1 - NS / 4) * n / (NS - NS / 4)>([&](auto k_) __attribute__((always_inline)) { q_step(k_, sq, acc); });
+                };
+            };
+            load_bias(BN, 0, true);
+            stage(1, up_into(acc0), idle);
+            load_bias(BN, 1, true);
+            for (int sq = 0; sq + 2 < a.nq; sq += 2) {       // nq is even: an even stage, then an odd one
+                stage(2, up_into(acc1), q_slots(sq, acc0));
+                stage(1, up_into(acc0), q_slots(sq + 1, acc1));
             }
+            stage(0, up_into(acc1), q_slots(a.nq - 2, acc0));
+            static_for<0, 3 * RT>([&](auto k_) __attribute__((always_inline)) { q_step(k_, a.nq - 1, acc1); });
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no transfer into LDS may outlive the workgroup
