@@ -68,6 +68,10 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
     const float* BO = LNB + D; const float* LN2G = BO + D; const float* LN2B = LN2G + D; const float* BN = LN2B + D;
     auto foff = [&](int nt) __attribute__((always_inline)) { return 32 * (nt >> 1) + 8 * g + 4 * (nt & 1); };
 
+    // the lane for an address that is needed once a tile: computed where it is used, not kept across the tile (kept, addresses and row
+    // conditions were 26 spilled registers at d = 256 and 12 at d = 384, each reload behind the stores in flight: four blocks at
+    // d = 256, 541k rows, 4.55 -> 4.35 ms, six at d = 384, 1.2M rows, 31.3 -> 31.1)
+    auto lane_here = [&] __attribute__((always_inline)) { int l = lane; asm volatile("" : "+v"(l)); return l; };
     R pipe;
     {   // SLOTS - 2 stages in flight (the host checks that the image is longer), then the vectors
         pipe.start(ring, a.frags, a.total_stages, wave, lane);
@@ -83,7 +87,9 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
     const int nch = a.F / 32;
 
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t row0 = (tile * NW + wave) * (RT * 16);
+        // a wave's rows from a scalar base, so that a lane's share of an address is one 32-bit offset
+        const int64_t row0 = (tile * NW + wave) * (RT * 16), base0 = row0 < rows ? row0 : rows - 1;
+        const int left = rows - row0 > RT * 16 ? RT * 16 : rows > row0 ? (int)(rows - row0) : 0, last = left > 0 ? left - 1 : 0;
         f32x4 x[RT][NT];
         BFrag8 hf[RT][KC];
         // The tile's loads: two row tiles of x and every operand row at once (the compiler counts its own loads, not the
@@ -91,25 +97,25 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
         if constexpr (!LEAD)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            int64_t row = row0 + 16 * rt + r16; row = row < rows ? row : rows - 1;
-            const u16* hr = a.att + row * D;
+            const int l = lane_here(), row = 16 * rt + (l & 15) < last ? 16 * rt + (l & 15) : last;
+            const u16* hr = a.att + base0 * D + (uint32_t)(row * D + 8 * (l >> 4));
 #pragma unroll
-            for (int c = 0; c < KC; ++c) hf[rt][c].u = *reinterpret_cast<const uint4*>(hr + 32 * c + 8 * g);
+            for (int c = 0; c < KC; ++c) hf[rt][c].u = *reinterpret_cast<const uint4*>(hr + 32 * c);
         }
 #pragma unroll
         for (int half = 0; half < RT / RH; ++half) {
             uint4 rx[RH][XI32 ? NT : NT / 2];
 #pragma unroll
             for (int rr = 0; rr < RH; ++rr) {
-                int64_t row = row0 + 16 * (half * RH + rr) + r16; row = row < rows ? row : rows - 1;
+                const int l = lane_here(), rl = 16 * (half * RH + rr) + (l & 15), row = rl < last ? rl : last;
                 if constexpr (XI32) {
-                    const float* xr = static_cast<const float*>(a.x) + row * D;
+                    const float* xr = static_cast<const float*>(a.x) + base0 * D + (uint32_t)(row * D + 8 * (l >> 4));
 #pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) rx[rr][nt] = *reinterpret_cast<const uint4*>(xr + foff(nt));
+                    for (int nt = 0; nt < NT; ++nt) rx[rr][nt] = *reinterpret_cast<const uint4*>(xr + 32 * (nt >> 1) + 4 * (nt & 1));
                 } else {
-                    const u16* xr = static_cast<const u16*>(a.x) + row * D;
+                    const u16* xr = static_cast<const u16*>(a.x) + base0 * D + (uint32_t)(row * D + 8 * (l >> 4));
 #pragma unroll
-                    for (int p = 0; p < NT / 2; ++p) rx[rr][p] = *reinterpret_cast<const uint4*>(xr + 32 * p + 8 * g);
+                    for (int p = 0; p < NT / 2; ++p) rx[rr][p] = *reinterpret_cast<const uint4*>(xr + 32 * p);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -298,19 +304,21 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
         // round, store, LayerNorm on the rounded row, its output as operand fragments
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            const int64_t row = row0 + 16 * rt + r16;
+            const int l = lane_here(), row = 16 * rt + (l & 15);
+            const uint32_t at = (uint32_t)((l & 15) * D + 8 * (l >> 4));
+            const int64_t first = (row0 + 16 * rt) * D;
             float s = 0.f, q = 0.f;
             uint2 vprev = make_uint2(0, 0);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 f32x4 r = x[rt][nt];
                 if constexpr (XO32) {
-                    if (row < rows) *reinterpret_cast<f32x4*>(static_cast<float*>(a.xo) + row * D + foff(nt)) = r;
+                    if (row < left) *reinterpret_cast<f32x4*>(static_cast<float*>(a.xo) + first + at + 32 * (nt >> 1) + 4 * (nt & 1)) = r;
                 } else {
                     uint2 v;
                     v.x = bpack2<DT>(r[0], r[1]); v.y = bpack2<DT>(r[2], r[3]);
                     if constexpr (!LEAD) {
-                        if (nt & 1) { if (row < rows) *reinterpret_cast<uint4*>(static_cast<u16*>(a.xo) + row * D + 32 * (nt >> 1) + 8 * g) = make_uint4(vprev.x, vprev.y, v.x, v.y); }
+                        if (nt & 1) { if (row < left) *reinterpret_cast<uint4*>(static_cast<u16*>(a.xo) + first + at + 32 * (nt >> 1)) = make_uint4(vprev.x, vprev.y, v.x, v.y); }
                         else vprev = v;
                     }
                     r[0] = DT::to_f((u16)(v.x & 0xffff)); r[1] = DT::to_f((u16)(v.x >> 16));
@@ -328,7 +336,7 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
                 const float mean = s * (1.0f / D);
                 const float rstd = rsqrtf(fmaxf(fmaf(-mean, mean, q * (1.0f / D)), 0.f) + a.eps);
                 const float shift = -mean * rstd;
-                const bool keep = a.ho && row < rows && row < a.ho_rows;
+                const bool keep = a.ho && row < left && row0 + row < a.ho_rows;
                 uint2 hprev = make_uint2(0, 0);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
@@ -337,7 +345,7 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
                     uint2 v;
                     v.x = bpack2<DT>(fmaf(fmaf(x[rt][nt][0], rstd, shift), gm.x, bt.x), fmaf(fmaf(x[rt][nt][1], rstd, shift), gm.y, bt.y));
                     v.y = bpack2<DT>(fmaf(fmaf(x[rt][nt][2], rstd, shift), gm.z, bt.z), fmaf(fmaf(x[rt][nt][3], rstd, shift), gm.w, bt.w));
-                    if (nt & 1) { if (keep) *reinterpret_cast<uint4*>(a.ho + row * D + 32 * (nt >> 1) + 8 * g) = make_uint4(hprev.x, hprev.y, v.x, v.y); }
+                    if (nt & 1) { if (keep) *reinterpret_cast<uint4*>(a.ho + first + at + 32 * (nt >> 1)) = make_uint4(hprev.x, hprev.y, v.x, v.y); }
                     else hprev = v;
                     hf[rt][nt >> 1].h[nt & 1] = v;
                 }
@@ -349,14 +357,15 @@ __global__ __launch_bounds__(256, 1) void block_tail_kernel(TailArgs a) {
             // successor's bias is read behind them too (together: d = 256 as above 4.58 -> 4.55 ms, six at d = 384 31.65 -> 31.28; the q|k|v launch of the first
             // block is bound by its MFMAs, loads and LayerNorm: without its stores 16 % faster, without the weight stream 16 %)
             const int ldq = 32 * a.nq;
-            u16* const qrow = a.qo + (row0 + r16) * ldq + 8 * g;
+            const int ql = lane_here();
+            const uint32_t qat = (uint32_t)((ql & 15) * ldq + 8 * (ql >> 4));
             uint4 qv;
             auto q_step = [&](auto k_, int sq, Acc& acc) __attribute__((always_inline)) {      // three steps per row tile
                 constexpr int rt = decltype(k_)::value / 3, step = decltype(k_)::value % 3;
                 // the stage's columns in the paired order: 16 bytes per lane
                 if constexpr (step == 0) { qv.x = bpack2<DT>(acc[0][rt][0], acc[0][rt][1]); qv.y = bpack2<DT>(acc[0][rt][2], acc[0][rt][3]); }
                 if constexpr (step == 1) { qv.z = bpack2<DT>(acc[1][rt][0], acc[1][rt][1]); qv.w = bpack2<DT>(acc[1][rt][2], acc[1][rt][3]); }
-                if constexpr (step == 2) { if (row0 + 16 * rt + r16 < rows) *reinterpret_cast<uint4*>(qrow + (int64_t)16 * rt * ldq + 32 * sq) = qv; }
+                if constexpr (step == 2) { if (16 * rt + (ql & 15) < left) *reinterpret_cast<uint4*>(a.qo + (row0 + 16 * rt) * ldq + 32 * sq + qat) = qv; }
             };
             auto q_slots = [&](int sq, Acc& acc) __attribute__((always_inline)) {
                 return [&, sq](auto s_) __attribute__((always_inline)) {
