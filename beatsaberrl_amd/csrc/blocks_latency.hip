@@ -10,7 +10,8 @@
 // six blocks do not fit an XCD's L2), and the barriers and LayerNorms between.
 // Per-row arithmetic and its order are those of blocks_kernel: an accumulator starts at its bias or at the residual and takes the
 // k chunks in ascending order; LayerNorm's sums and softmax's reductions run in the same lane layout.
-// Six blocks at d = 192, 1 .. 256 envs: 206 - 216 -> 79 - 84 us; three at d = 128: 55 - 59 -> 19 - 23 us.
+// Six blocks at d = 192, 1 .. 256 envs: 206 - 216 -> 66 - 71 us (79 - 84 while the key mask and row addresses were spilled); three at
+// d = 128: 55 - 59 -> 19 - 23 us.
 #include "block_stage.h"
 #include "blocks_latency.h"
 
@@ -34,6 +35,7 @@ __global__ __launch_bounds__(D * 4) void blocks_latency_kernel(BlocksLatencyArgs
     uint4* hid = un;                                                     // [row tile][chunk][lane]
     const int un_u4 = 3 * NT * 64 + 2 * KC * 64 > 2 * nch * 64 ? 3 * NT * 64 + 2 * KC * 64 : 2 * nch * 64;
     float4* vb = reinterpret_cast<float4*>(un + un_u4);                  // fp32 vectors of two blocks
+    float* km = reinterpret_cast<float*>(vb + 2 * nv4);                  // the env's 32 slots
     const float scale_l2e = (DH == 32 ? 0.17677669529663688110f : 0.14433756729740644113f) * 1.44269504088896340736f;
 
     // group gi of a block: KC fragments in the order of their use (0 .. 2: q | k | v tiles w, w + NT, w + 2 NT; 3: output
@@ -66,14 +68,9 @@ __global__ __launch_bounds__(D * 4) void blocks_latency_kernel(BlocksLatencyArgs
     static_for<0, NBUF>([&](auto i) __attribute__((always_inline)) { load(buf[decltype(i)::value], 0, i); });
     for (int i = tid; i < nv4; i += NTHR) vb[i] = reinterpret_cast<const float4*>(a.vec)[i];
     for (int64_t env = blockIdx.x; env < a.B; env += gridDim.x) {
-        float kmask[2][4];       // additive key bias * log2(e) for keys 16 kt + 4 g + i; -inf past T
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = 16 * kt + 4 * g + i;
-                kmask[kt][i] = key < a.T ? DT::to_f(a.key_bias[env * a.T + key]) * 1.44269504088896340736f : -INFINITY;
-            }
+        // additive key bias * log2(e) of every slot, -inf past T: read where attention wants it (kept in registers it was spilled, and
+        // its reload waited behind the weights in flight)
+        if (tid < 32) km[tid] = tid < a.T ? DT::to_f(a.key_bias[env * a.T + tid]) * 1.44269504088896340736f : -INFINITY;
         f32x4 x[2];              // this wave's feature tile of the residual stream, both row tiles
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
@@ -88,7 +85,9 @@ __global__ __launch_bounds__(D * 4) void blocks_latency_kernel(BlocksLatencyArgs
             if (tiles == 2) xs[(NT + w) * 64 + lane_] = x[1];
         };
         auto store_rows = [&](int rt, u16* dst, int rows_per_env, int nrows_valid) __attribute__((always_inline)) {
-            const int row = 16 * rt + r16;
+            int l = lane_;                                                // opaque: as in layer()
+            asm volatile("" : "+v"(l));
+            const int row = 16 * rt + (l & 15), g = l >> 4;
             if (row < nrows_valid) {
                 uint2 v;
                 v.x = bpack2<DT>(x[rt][0], x[rt][1]); v.y = bpack2<DT>(x[rt][2], x[rt][3]);
@@ -218,6 +217,9 @@ __global__ __launch_bounds__(D * 4) void blocks_latency_kernel(BlocksLatencyArgs
                     }
                 }
                 float sv[2][4], mx = -INFINITY, sum = 0.f;
+                f32x4 kmask[2];
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt) kmask[kt] = *reinterpret_cast<const f32x4*>(km + 16 * kt + 4 * g);
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(D * 4) void blocks_latency_kernel(BlocksLatencyArgs
 template <int D> size_t latency_bytes() {
     constexpr int NT = Geo<D>::NT, KC = Geo<D>::KC, F = 4 * D;
     const size_t qkvo = (size_t)(3 * NT + 2 * KC) * 64, hid = (size_t)2 * (F / 32) * 64;
-    return ((size_t)2 * NT * 64 + 2 * KC * 64 + (qkvo > hid ? qkvo : hid)) * 16 + (size_t)2 * Geo<D>::lv_size(F) * 4;
+    return ((size_t)2 * NT * 64 + 2 * KC * 64 + (qkvo > hid ? qkvo : hid)) * 16 + (size_t)2 * Geo<D>::lv_size(F) * 4 + 128;
 }
 template <typename DT, int D, int DH, int ACT>
 bool go(const BlocksLatencyArgs& a, int cus, hipStream_t st) {
