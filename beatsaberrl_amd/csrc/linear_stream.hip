@@ -14,8 +14,8 @@
 // memory latency.
 // Per 32-k chunk a wave reads MT fragments (1 KB each) from LDS for 2 MT MFMAs (two 16-row tiles share
 // each fragment): the LDS read path allows ~50 % of MFMA peak, which is above what the HBM stream needs
-// at these K.  Bias, activation, residual and gate are applied in registers (a lane holds 4 consecutive
-// features of one row); the rounded results of 16 rows then cross a per-wave LDS tile so that they leave as
+// at these K.  Bias, activation and residual are applied in registers (a lane holds 4 consecutive
+// features of one row), the gate on the way out; the rounded results of 16 rows then cross a per-wave LDS tile so that they leave as
 // 16-byte stores covering whole row segments - written as 32-byte pieces straight from the MFMA layout the
 // same kernel ran at 3.1 TB/s instead of the 5 TB/s a plain copy reaches on this part (measured: the stores
 // alone cost as much as the whole read stream).
@@ -31,6 +31,7 @@ namespace {
 constexpr int ST_THREADS = 512;                  // 8 waves share one resident weight block
 constexpr int ST_ROWS = 32;                      // rows per wave tile (2 MFMA row tiles)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4a8 __attribute__((ext_vector_type(4), aligned(8)));       // a gate's rows are 8-byte aligned
 
 // ACT and AUX (0 none, 1 residual, 2 ReLU gate) are compile-time: with run-time switches the epilogue was 2270 VALU
 // instructions and 248 branches per 32-row tile and took 12k of a tile's 18.5k cycles (traced with s_memtime), twice
@@ -112,6 +113,24 @@ __global__ __launch_bounds__(ST_THREADS) void linear_stream_kernel(LinArgs a, in
         }
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) xf1[kc] = *reinterpret_cast<const u32x4*>(wt + r16 * TP + kc * 32 + 8 * g);
+        // The gate's pieces, in the order in which the result is stored: consecutive lanes on consecutive 16-byte pieces of whole row
+        // segments, a half's all at once and ahead of the MFMAs (the other half's behind them: registers).  Read by the lane that
+        // holds a feature quad - 8 bytes, 32 of a row together, each waited for in the epilogue - the gated data gradient of the
+        // FFN (318k rows, 192 -> 768) took 360 us, 3.1 TB/s; now 235, 4.7 TB/s
+        constexpr int OPR = MT * 2;                                       // 16-byte pieces per output row
+        constexpr int NST = (16 * OPR + WAVE - 1) / WAVE;                 // pieces per lane for 16 output rows
+        u32x4 gt[AUX == 2 ? NST : 1][2];
+        auto fetch_gate = [&](auto rt_) __attribute__((always_inline)) {
+            constexpr int rt = decltype(rt_)::value;
+            int l = lane;
+            asm volatile("" : "+v"(l));                                   // addresses are made here, not kept across the tiles
+#pragma unroll
+            for (int it = 0; it < NST; ++it) {
+                const int c = it * WAVE + l, r = c / OPR, col = m0 + c % OPR * 8;
+                const int64_t row = tile * ST_ROWS + rt * 16 + r;         // a piece past the end: any valid one
+                if constexpr (AUX == 2) gt[it][rt] = *reinterpret_cast<const u32x4a8*>(gate + (row < rows ? row : rows - 1) * a.ldgate + (col < a.M ? col : 0));
+            }
+        };
         ST_FETCH(tile + stride)                                         // rows past the end clamp to the last row: always a valid load
         f32x4 acc[MT][2];
 #pragma unroll
@@ -132,6 +151,7 @@ __global__ __launch_bounds__(ST_THREADS) void linear_stream_kernel(LinArgs a, in
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (AUX == 2) { fetch_gate(std::integral_constant<int, 0>()); fetch_gate(std::integral_constant<int, 1>()); }
         // epilogue: lane holds features m0 + 16 mt + 4 g .. + 3 of rows 16 rt + r16
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) {
@@ -150,20 +170,31 @@ __global__ __launch_bounds__(ST_THREADS) void linear_stream_kernel(LinArgs a, in
                     o[0] += DT::to_f((u16)(rv2.x & 0xffff)); o[1] += DT::to_f((u16)(rv2.x >> 16));
                     o[2] += DT::to_f((u16)(rv2.y & 0xffff)); o[3] += DT::to_f((u16)(rv2.y >> 16));
                 }
-                if (AUX == 2 && on) {
-                    const uint2 gv = *reinterpret_cast<const uint2*>(gate + row * a.ldgate + col);
-                    if (!(DT::to_f((u16)(gv.x & 0xffff)) > 0.f)) o[0] = 0.f;
-                    if (!(DT::to_f((u16)(gv.x >> 16)) > 0.f)) o[1] = 0.f;
-                    if (!(DT::to_f((u16)(gv.y & 0xffff)) > 0.f)) o[2] = 0.f;
-                    if (!(DT::to_f((u16)(gv.y >> 16)) > 0.f)) o[3] = 0.f;
-                }
                 uint2 ov;
                 ov.x = DT::pack2(o[0], o[1]);
                 ov.y = DT::pack2(o[2], o[3]);
                 *reinterpret_cast<uint2*>(wt + r16 * TP + mt * 16 + 4 * g) = ov;
             }
             // the tile leaves row-major: 16-byte pieces, consecutive lanes on consecutive pieces of a row
-            constexpr int OPR = MT * 2;                                   // 16-byte pieces per output row
+            if constexpr (AUX == 2) {
+                int l = lane;
+                asm volatile("" : "+v"(l));
+#pragma unroll
+                for (int it = 0; it < NST; ++it) {
+                    const int c = it * WAVE + l, r = c / OPR, pc = c % OPR;
+                    const int64_t orow = tile * ST_ROWS + rt * 16 + r;
+                    if (c < 16 * OPR && orow < rows && m0 + pc * 8 < a.M) {
+                        u32x4 v = *reinterpret_cast<const u32x4*>(wt + r * TP + pc * 8);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t gv = gt[it][rt][e];
+                            if (!(DT::to_f((u16)(gv & 0xffff)) > 0.f)) v[e] &= 0xffff0000u;
+                            if (!(DT::to_f((u16)(gv >> 16)) > 0.f)) v[e] &= 0x0000ffffu;
+                        }
+                        *reinterpret_cast<u32x4*>(y + lin_yoff(a, orow) + m0 + pc * 8) = v;
+                    }
+                }
+            } else
 #pragma unroll 1
             for (int c0 = 0; c0 < 16 * OPR; c0 += WAVE) {
                 const int c = c0 + lane;
