@@ -1133,12 +1133,16 @@ __global__ __launch_bounds__(256, (KRT <= 2 && !RING) ? 2 : 1) void cfg_forward_
     if (PACK && KRT == 2 && a.cus > 0) {
         // (32-bit arithmetic: the packed tile count is an int32, and a 64-bit division is a ~200-instruction routine
         // of which three sat between the prologue and the first pass)
-        const uint32_t nt32 = (uint32_t)ntiles;
-        const int64_t r = nt32 % (uint32_t)a.cus;
-        const int64_t p2 = nt32 - (uint32_t)r;
-        const int64_t nrem = n_units - p2 * ENVS_PER_WG;                 // tiles left for one-tile passes
-        const int q = (int)(((uint32_t)nrem + 3u) / 4u), fb = (int)((uint32_t)p2 % gridDim.x);
-        if (r > 0 && r <= 32 && p2 > 0 && fb + q <= (int)gridDim.x) { n_bulk = p2; rem_tile0 = p2 * ENVS_PER_WG; rem_first_wg = fb; rem_passes = q; }
+        const uint32_t nt32 = __builtin_amdgcn_readfirstlane((uint32_t)ntiles), units = __builtin_amdgcn_readfirstlane((uint32_t)n_units);
+        if (MERGE && units <= 4u * (uint32_t)a.cus && units <= 4u * gridDim.x) {
+            // no more tiles than SIMDs: one to a wave, a wave to a SIMD (two to a wave were the whole two-tile chain on half of the
+            // CUs: 1030 .. 1600 envs with 0 .. 15 objects, f16, 48.5 -> 38 us; between one and two tiles per SIMD both take the same)
+            n_bulk = 0; rem_passes = (int)((units + 3u) / 4u);
+        } else {
+            const uint32_t r = nt32 % (uint32_t)a.cus, p2 = nt32 - r;
+            const int q = (int)((units - p2 * ENVS_PER_WG + 3u) / 4u), fb = (int)(p2 % gridDim.x);       // passes for the tiles left
+            if (r > 0 && r <= 32 && p2 > 0 && fb + q <= (int)gridDim.x) { n_bulk = p2; rem_tile0 = (int64_t)p2 * ENVS_PER_WG; rem_first_wg = fb; rem_passes = q; }
+        }
     }
     typedef std::integral_constant<int, 1> rt_one;
     typedef std::false_type head_pass;
@@ -1451,7 +1455,8 @@ int launch_one(const FwdArgs& a, int cus, hipStream_t st) {
             return BSRL_UNSUPPORTED;
     }
     const int64_t per_wg = RING ? a.ring_epw : 4 * RT * (MODE == MODE_TAIL ? TAIL_ENVS : 1);
-    const int64_t ntiles = (a.B + per_wg - 1) / per_wg;
+    int64_t ntiles = (a.B + per_wg - 1) / per_wg;
+    if (PACK && DMA && ntiles < cus) ntiles = (a.B + 3) / 4 < cus ? (a.B + 3) / 4 : cus;       // room for one-tile passes
     const int64_t resident = (int64_t)cus * ((RT <= 2 && !RING) ? 2 : 1);
     hipLaunchKernelGGL(kern, dim3((unsigned)(ntiles < resident ? ntiles : resident)), dim3(256), dyn, st, a);
     return BSRL_OK;
