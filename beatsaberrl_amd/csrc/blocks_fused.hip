@@ -850,7 +850,7 @@ int fwd_launch(const BlkArgs& a_, int cus, hipStream_t st) {
     BlkArgs a = a_;
     if constexpr (D != 256) {
         // Few envs: one per workgroup, its features over the waves (blocks_latency.hip).  us at d = 192, six blocks | d = 128, three,
-        // with it / without: 1 env 79 / 206 | 19 / 41, 256 envs 84 / 216 | 23 / 44, 512 (two rounds) 176 / 216 | 42 / 47,
+        // with it / without: 1 env 68 / 206 | 18 / 41, 256 envs 76 / 216 | 22 / 44, 512 (two rounds) 148 / 216 | 41 / 47,
         // 1024 321 / 246 | 86 / 54.  All three kernels produce the same bits for an env.
         if (a.B <= 2 * (int64_t)cus) {
             const BlocksLatencyArgs l{reinterpret_cast<const uint4*>(a.frags), a.vec, a.x_in, a.key_bias, a.x_res, a.x_out, a.B, a.n_layers, a.F, a.T, a.n_queries};

@@ -6,12 +6,12 @@
 // w owns feature tile w: the weight fragments that produce its features are read by no other wave, so they go from L2 straight
 // into its registers, a group of KC fragments in use and two (d = 128: three) in flight.  What the waves share - the residual stream (fp32),
 // LayerNorm's output, q | k | v, attention's output, the hidden - crosses LDS as MFMA operand fragments, seven barriers per
-// block.  Bound: the weight stream of a CU, 0.88 MB per block at d = 192 at the ~40 B/clk that it reaches (10 of 13 us per block;
+// block.  Bound: the weight stream of a CU, 0.88 MB per block at d = 192 at the ~40 B/clk that it reaches (10 of 11 us per block;
 // six blocks do not fit an XCD's L2), and the barriers and LayerNorms between.
 // Per-row arithmetic and its order are those of blocks_kernel: an accumulator starts at its bias or at the residual and takes the
 // k chunks in ascending order; LayerNorm's sums and softmax's reductions run in the same lane layout.
-// Six blocks at d = 192, 1 .. 256 envs: 206 - 216 -> 66 - 71 us (79 - 84 while the key mask and row addresses were spilled); three at
-// d = 128: 55 - 59 -> 19 - 23 us.
+// Six blocks at d = 192, 1 .. 256 envs: 206 - 216 -> 68 - 76 us (79 - 84 while the key mask and row addresses were spilled); three at
+// d = 128: 55 - 59 -> 18 - 22 us.
 #include "block_stage.h"
 #include "blocks_latency.h"
 

@@ -5,7 +5,7 @@
 // the masters by three launches, and the forward is one call (or four, where the caller runs the critic on a second stream): the
 // four encoders share a launch, LayerNorms read and write strided rows, so that neither the torso rows nor the value MLP's input
 // is copied together.  Every kernel and its operands are those of the op-by-op forward: the same bits.
-// One env, recipe shape: 419 -> 180 us, 157 with the chains of note_readout.hip, 80 of them the block stack (blocks_latency.hip: from
+// One env, recipe shape: 419 -> 180 us, 145 with the chains of note_readout.hip, 68 of them the block stack (blocks_latency.hip: from
 // 206); a captured rollout step of 2048 envs, default shape: 217 -> 180 us, 151 with the chains; the update of 1500 envs: 3.7 -> 3.3 ms.
 #include "blocks_pair.h"
 #include "note_pack.h"
