@@ -8,7 +8,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbsrl_hip.so")
-ABI_VERSION = 21
+ABI_VERSION = 22
 CFG_NO_PACK = 1                 # bsrl_cfg_desc.flags: one env per tile in the fused forward
 CFG_NO_LATENCY = 2              # bsrl_cfg_desc.flags: small batches take the throughput forms too
 NOTE_ZERO_MASKED = 2            # bsrl_note_frontend: note_flags
@@ -129,6 +129,11 @@ SIGNATURES = {
     "bsrl_note_train_layout": (_i64, [C.POINTER(NoteDesc), _p, _i64]),
     "bsrl_note_train_size": (_i64, [C.POINTER(NoteDesc), _i64, _i32]),
     "bsrl_note_train_forward": (_i32, [C.POINTER(NoteDesc), _p, _p, _i64, _i32, _p, _p, _p, _i64, _p, _i64, _p]),
+    "bsrl_note_train_saves": (_i32, [C.POINTER(NoteDesc), _i64]),
+    "bsrl_note_train_begin": (_i32, [C.POINTER(NoteDesc), _p, _p, _i64, _i32, _p, _p, _i64, _p, _i64, _p]),
+    "bsrl_note_forward_saving": (_i32, [C.POINTER(NoteDesc), _p, _p, _p, _i64, _i32, _p, _p, _p, _p, _p, _i64, _i32, _p, _i64, _p, _i64, _p]),
+    "bsrl_note_train_end": (_i32, [C.POINTER(NoteDesc), _p, _p, _i64, _p, _i64, _p]),
+    "bsrl_note_train_stack_backward": (_i32, [C.POINTER(NoteDesc), _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p]),
     "bsrl_note_train_backward": (_i32, [C.POINTER(NoteDesc), _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p]),
     "bsrl_heads_logp_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "bsrl_hl_loss": (_i32, [_p, _p, _p, _f, _p, _p, _i64, _i64, _p]),

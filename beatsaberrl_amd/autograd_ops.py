@@ -388,6 +388,19 @@ class NoteTrainPlan:
     def pointers(self, params):
         return (ctypes.c_void_p * len(params))(*[p.data_ptr() for p in params])
 
+    def begin(self, params, obs, saber_idx, body_idx):
+        """The update's saved activations with everything in front of the block stack in them, for a rollout forward that writes
+        the blocks'; None where the update computes them itself (the size rule is the library's)."""
+        lib, B = _lib.load(), obs.shape[0]
+        if not lib.bsrl_note_train_saves(self.desc, B):
+            return None
+        saved = torch.empty(lib.bsrl_note_train_size(self.desc, B, 0), dtype=torch.uint8, device=obs.device)
+        rc = lib.bsrl_note_train_begin(self.desc, self.pointers(params), obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype), saber_idx.data_ptr(),
+                                       body_idx.data_ptr(), B, saved.data_ptr(), saved.numel(), ops._stream(obs))
+        if not _lib.check(rc, "bsrl_note_train_begin"):
+            raise ops.Unsupported("bsrl_note_train_begin")
+        return saved
+
     def bwd_pointers(self, tensors):
         ptrs = (ctypes.c_void_p * len(self.shapes))()
         for i, t in zip(self.bwd_params, tensors):
@@ -398,21 +411,26 @@ class NoteTrainPlan:
 class NoteTrainFn(torch.autograd.Function):
     """(logits, value, bin logits) of the NotePolicy update: forward and backward are one native call each over the compacted
     token stream.  The bin logits are this forward's own; logits and value are the rollout's (`r_logits`, `r_value`), whose
-    gradients enter where this forward's would: value = softmax(bin logits) @ centers.  Notes that attention cannot see are
+    gradients enter where this forward's would: value = softmax(bin logits) @ centers.  `saved`: what the rollout has left of this
+    forward (`NoteTrainPlan.begin`), or None.  Notes that attention cannot see are
     never computed: their weight in every softmax is exactly zero."""
 
     @staticmethod
-    def forward(ctx, plan, obs, saber_idx, body_idx, centers, r_logits, r_value, *params):
+    def forward(ctx, plan, obs, saber_idx, body_idx, centers, r_logits, r_value, saved, *params):
         lib, B, dev = _lib.load(), obs.shape[0], obs.device
-        size = lib.bsrl_note_train_size(plan.desc, B, 0)
-        if size <= 0:
-            raise ops.Unsupported(f"note_train B={B}")
-        saved = torch.empty(size, dtype=torch.uint8, device=dev)
         vlogits = torch.empty(B, plan.desc.bins, dtype=torch.float32, device=dev)
+        ctx.stack = saved is not None
         with torch.cuda.device(dev):
-            rc = lib.bsrl_note_train_forward(plan.desc, plan.pointers(params), obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype),
-                                             saber_idx.data_ptr(), body_idx.data_ptr(), vlogits.data_ptr(), B, saved.data_ptr(),
-                                             size, ops._stream(obs))
+            if ctx.stack:                              # the rollout's block stack has left its activations there
+                rc = lib.bsrl_note_train_end(plan.desc, plan.pointers(params), vlogits.data_ptr(), B, saved.data_ptr(), saved.numel(), ops._stream(obs))
+            else:
+                size = lib.bsrl_note_train_size(plan.desc, B, 0)
+                if size <= 0:
+                    raise ops.Unsupported(f"note_train B={B}")
+                saved = torch.empty(size, dtype=torch.uint8, device=dev)
+                rc = lib.bsrl_note_train_forward(plan.desc, plan.pointers(params), obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype),
+                                                 saber_idx.data_ptr(), body_idx.data_ptr(), vlogits.data_ptr(), B, saved.data_ptr(),
+                                                 size, ops._stream(obs))
         if not _lib.check(rc, "bsrl_note_train_forward"):
             raise ops.Unsupported("bsrl_note_train_forward")
         ctx.plan, ctx.logits_shape = plan, r_logits.shape
@@ -424,7 +442,7 @@ class NoteTrainFn(torch.autograd.Function):
     def backward(ctx, g_logits, g_value, g_vlogits):
         saved, vlogits, centers, *scales = ctx.saved_tensors
         plan, lib, dev, B = ctx.plan, _lib.load(), saved.device, vlogits.shape[0]
-        n_pass = 7                                             # inputs ahead of the parameters
+        n_pass = 8                                             # inputs ahead of the parameters
         # what no output in the loss depends on has no gradient, rather than a zero that an optimizer would step on
         unused = set(plan.heads if g_logits is None else ()) | set(plan.critic if g_value is None and g_vlogits is None else ())
         if g_value is not None:                                # through the expectation over the bins
@@ -440,7 +458,8 @@ class NoteTrainFn(torch.autograd.Function):
         n_scratch = lib.bsrl_note_train_size(plan.desc, B, 1)
         scratch = torch.empty(n_scratch, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
-            rc = lib.bsrl_note_train_backward(plan.desc, plan.bwd_pointers(scales), g_logits.data_ptr(), g_vlogits.data_ptr(), flat.data_ptr(),
+            backward = lib.bsrl_note_train_stack_backward if ctx.stack else lib.bsrl_note_train_backward
+            rc = backward(plan.desc, plan.bwd_pointers(scales), g_logits.data_ptr(), g_vlogits.data_ptr(), flat.data_ptr(),
                                               B, saved.data_ptr(), saved.numel(), scratch.data_ptr(), n_scratch, ops._stream(saved))
         if not _lib.check(rc, "bsrl_note_train_backward"):
             raise ops.Unsupported("bsrl_note_train_backward")

@@ -41,6 +41,7 @@ struct AttnBwdArgs {
     // compacted stream: env b's tokens are rows lead b + j (j < lead) and lead B + noff[b] + j - lead of k, v and their
     // gradients (batch strides unused, key_bias: of the optional rows); q, dout, dq likewise, or rows nq b + j with nq set
     const int32_t* noff; int lead, nq;
+    uint32_t q_hs = 0, kv_hs = 0;  // ... elements from a head to the next in q | k and v, where that is not dh
 };
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwd
     u16 kraw[NKT][4];                                            // key bias of keys 16 kt + 4 g + e, raw
     int nv_next = 0;
     const int64_t rss[4] = {a.q_rs, a.do_rs, a.k_rs, a.v_rs};
+    const uint32_t q_hs = RAG && a.q_hs ? a.q_hs : DH, kv_hs = RAG && a.kv_hs ? a.kv_hs : DH, hss[4] = {q_hs, DH, kv_hs, kv_hs};
     const int prows[4] = {TQP, TQP, TP, TP};
     const int offs[4] = {0, TQP * DHP, 2 * TQP * DHP, 2 * TQP * DHP + TP * DHP};          // Qs, dOs, Ks, Vs inside a wave's region
     // piece c = it * gthreads + gt of a matrix is (row c / rp, head (c % rp) / PPR, part (c % rp) % PPR)
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwd
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 buf[mtx][it] = (u32x4v){0u, 0u, 0u, 0u};
-                if (row < nrows[mtx]) buf[mtx][it] = *reinterpret_cast<const u32x4v*>(srcs[mtx] + (!RAG ? (int64_t)row : mtx < 2 && a.nq ? be * a.nq + row : row < a.lead ? lead0 + row : opt0 + row) * rss[mtx] + (cp / PPR) * DH + (cp % PPR) * 8);
+                if (row < nrows[mtx]) buf[mtx][it] = *reinterpret_cast<const u32x4v*>(srcs[mtx] + (!RAG ? (int64_t)row : mtx < 2 && a.nq ? be * a.nq + row : row < a.lead ? lead0 + row : opt0 + row) * rss[mtx] + (uint32_t)(cp / PPR) * hss[mtx] + (cp % PPR) * 8);
                 row += row_step; cp += cp_step;
                 if (cp >= rp) { cp -= rp; ++row; }
             }
@@ -453,21 +455,23 @@ extern "C" int bsrl_attn_bwd(const void* q, int64_t q_bs, int64_t q_rs, const vo
 }
 
 // Backward over the compacted stream (16-bit; workgroup = the heads of one env): dq, dk, dv row for row as q, k, v.  nq: queries
-// per env (q, dout, dq then hold nq B rows), 0 = every token.
+// per env (q, dout, dq then hold nq B rows), 0 = every token.  q_hs, kv_hs: a head's rows of q | k and v by themselves, so many elements
+// from the next head's (0: beside it).
 int bsrl_attn_bwd_ragged(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, const int32_t* noff,
                          const void* opt_bias, const void* dout, int64_t do_ld, void* dq, int64_t dq_ld, void* dk, int64_t dk_ld,
                          void* dv, int64_t dv_ld, int64_t B, int64_t lead, int64_t opt, int64_t nq, int64_t H, int64_t dh, int dtype,
-                         bsrl_stream stream) {
+                         bsrl_stream stream, int64_t q_hs, int64_t kv_hs) {
     const int64_t T = lead + opt, TQ = nq ? nq : T;
     if (!bsrl_attn_bwd_ragged_ok(T, H, dh, dtype) || lead < 1 || opt < 0 || nq < 0 || nq > lead || B * H > 0x7fffffff) return BSRL_UNSUPPORTED;
-    const int64_t lds_[] = {q_ld, k_ld, v_ld, do_ld, dq_ld, dk_ld, dv_ld};
+    const int64_t lds_[] = {do_ld, dq_ld, dk_ld, dv_ld}, in_[] = {q_ld, k_ld, v_ld}, hs_[] = {q_hs, kv_hs, kv_hs};
     for (int64_t s : lds_) if (s % 8 != 0 || s < H * dh) return BSRL_UNSUPPORTED;
+    for (int i = 0; i < 3; ++i) if (in_[i] % 8 != 0 || hs_[i] % 8 != 0 || hs_[i] < 0 || H * hs_[i] > 0xffffffffLL || in_[i] < (hs_[i] ? dh : H * dh)) return BSRL_UNSUPPORTED;
     const void* ptrs[] = {q, k, v, dout, dq, dk, dv};
     for (const void* p : ptrs) if (!p || !bsrl_aligned(p, 16)) return BSRL_UNSUPPORTED;
     if (B == 0) return BSRL_OK;
     const int tp = (int)((T + 15) / 16) * 16, tqp = (int)((TQ + 15) / 16) * 16;
     AttnBwdArgs a{q, k, v, dout, 0, q_ld, 0, k_ld, 0, v_ld, 0, do_ld, opt_bias, nullptr, dq, dk, dv, 0, dq_ld, 0, dk_ld, 0, dv_ld,
-                  B, (int)T, (int)TQ, (int)H, (float)(1.0 / sqrt((double)dh)), wave_elems_of(tp, tqp, (int)dh), 1, noff, (int)lead, (int)nq};
+                  B, (int)T, (int)TQ, (int)H, (float)(1.0 / sqrt((double)dh)), wave_elems_of(tp, tqp, (int)dh), 1, noff, (int)lead, (int)nq, (uint32_t)q_hs, (uint32_t)kv_hs};
     const size_t lds = (size_t)H * a.wave_elems * sizeof(u16);
     const int64_t resident = (int64_t)bsrl_cus() * 2;
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -117,8 +117,10 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
 #pragma unroll
         for (int i = 0; i < SLOTS - 2; ++i) issue(i * STAGE_BYTES);
     }
-    // entry of the next stage (PARITY = its index in its block, mod 2): on return it is readable in slot `cur`
-    template <int PARITY> __device__ __forceinline__ void admit() {
+    // entry of the next stage (PARITY = its index in its block, mod 2): on return it is readable in slot `cur`.  YOUNGER: other memory
+    // instructions that this wave has certainly issued since the loads that are waited for, which need not be waited for then; where `more`
+    // holds, MORE of them
+    template <int PARITY, int YOUNGER = 0, int MORE = YOUNGER> __device__ __forceinline__ void admit(bool more = false) {
         const uint32_t older = prev;
         prev = cur;
         cur = cur + STAGE_BYTES == SLOTS * STAGE_BYTES ? 0 : cur + STAGE_BYTES;
@@ -126,7 +128,12 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
             // this wave's loads of this stage and the next have landed once at most the AHEAD younger stages' are
             // outstanding (loads retire in order; any other load or store in flight, or a wave that loads nothing,
             // only makes the wait stricter) ...
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FPW * AHEAD) : "memory");
+            static_assert(FPW * AHEAD + YOUNGER < 64 && FPW * AHEAD + MORE < 64, "vmcnt is 6 bits");
+            // (the choice inside one statement: as a branch that the compiler sees it splits the stage, and its registers with it)
+            if constexpr (MORE > YOUNGER)
+                asm volatile("s_cmp_eq_u32 %0, 0\n\ts_cbranch_scc1 less%=\n\ts_waitcnt vmcnt(%2)\n\ts_branch done%=\nless%=:\n\ts_waitcnt vmcnt(%1)\ndone%=:"
+                             ::"s"(__builtin_amdgcn_readfirstlane((int)more)), "n"(FPW * AHEAD + YOUNGER), "n"(FPW * AHEAD + MORE) : "memory", "scc");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FPW * AHEAD + YOUNGER) : "memory");
             blk_barrier();             // ... and every wave's have; every wave is done reading the two stages before this one
             issue(older);
             issue(prev);

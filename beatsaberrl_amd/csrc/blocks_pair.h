@@ -24,7 +24,7 @@ inline BlocksPairPlan blocks_pair_plan(int* tiles, int chunks, int cus, int64_t 
 }
 __host__ __device__ inline bool blocks_pairs_pay(const BlocksPairPlan& p, int64_t ntiles) {
     const int64_t pairs = (ntiles + p.cus - 1) / p.cus, envs = (p.B + 8 * p.cus - 1) / (8 * p.cus);
-    return pairs * p.pair_ns <= envs * p.env_ns;
+    return p.env_ns == 0 || pairs * p.pair_ns <= envs * p.env_ns;
 }
 
 // entry of `pairs`: ids of two envs and their attendable optional tokens (bit t: token lead + t)
@@ -45,3 +45,14 @@ int bsrl_blocks_pair(const BlocksPairArgs& a, int d, int dtype, hipStream_t st);
 // bsrl_blocks_forward; with a plan, kernels that return at once where pairs pay
 int bsrl_blocks_unless(const bsrl_blocks_desc* d, const void* packed, const void* x_in, const void* key_bias, void* x_res, void* x_out, int64_t B,
                        const BlocksPairPlan* plan, bsrl_stream stream);
+
+// What the update's backward reads of a block (note_train.hip), written by the stack itself: rows of the update's compacted stream, token t
+// < lead of env b at lead b + t, its i-th attendable note at lead B + noff[b] + i.  x, h: the block's input and its LayerNorm; qkv: q, k, v
+// (k, v in the final block, q by itself: its lead rows), each head after head, a head's rows (d / heads wide) one after another - a whole line
+// at a time, where rows of all heads took its 96 bytes each at a time: 4.1 -> 3.65 ms for the recipe's 16384 envs -, v without its bias; att: attention's output; xm, h2, hid: the stream behind it, its
+// LayerNorm, the FFN's hidden; mean, rstd: of the two LayerNorms.  In the final block q, att and what follows are the lead rows'.
+struct BlocksSaveLayer { u16 *x, *h, *qkv, *q, *att, *xm, *h2, *hid; float *mean1, *rstd1, *mean2, *rstd2; };
+struct BlocksSave { const int32_t* noff; uint32_t rows; BlocksSaveLayer blk[BSRL_MAX_LAYERS]; };       // rows: what every buffer has room for
+// bsrl_blocks_pair (every env, whether pairs pay or not: a plan with env_ns = 0) that saves them
+bool bsrl_blocks_pair_saves(int64_t B, int d, int heads, int F, int T, int cus);
+int bsrl_blocks_pair_save(const BlocksPairArgs& a, const BlocksSave& save, int dtype, hipStream_t st);

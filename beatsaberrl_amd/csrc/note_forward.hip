@@ -7,9 +7,8 @@
 // is copied together.  Every kernel and its operands are those of the op-by-op forward: the same bits.
 // One env, recipe shape: 419 -> 180 us, 145 with the chains of note_readout.hip, 68 of them the block stack (blocks_latency.hip: from
 // 206); a captured rollout step of 2048 envs, default shape: 217 -> 180 us, 151 with the chains; the update of 1500 envs: 3.7 -> 3.3 ms.
-#include "blocks_pair.h"
-#include "note_pack.h"
 #include "note_readout.h"
+#include "note_train.h"
 
 namespace {
 
@@ -196,6 +195,13 @@ extern "C" int bsrl_note_pack(const bsrl_note_desc* d, const float* const* param
 extern "C" int bsrl_note_forward(const bsrl_note_desc* d, const float* const* params, const void* image, const void* obs, int64_t obs_ld, int obs_dtype,
                                  const int32_t* saber_idx, const int32_t* body_idx, const float* centers, float* logits, float* value, int64_t B, int parts,
                                  void* workspace, int64_t workspace_bytes, bsrl_stream stream) {
+    return bsrl_note_forward_saving(d, params, image, obs, obs_ld, obs_dtype, saber_idx, body_idx, centers, logits, value, B, parts, workspace, workspace_bytes,
+                                    nullptr, 0, stream);
+}
+
+extern "C" int bsrl_note_forward_saving(const bsrl_note_desc* d, const float* const* params, const void* image, const void* obs, int64_t obs_ld, int obs_dtype,
+                                        const int32_t* saber_idx, const int32_t* body_idx, const float* centers, float* logits, float* value, int64_t B,
+                                        int parts, void* workspace, int64_t workspace_bytes, void* saved, int64_t saved_bytes, bsrl_stream stream) {
     if (!desc_ok(d)) return BSRL_UNSUPPORTED;
     if (!params || !image || !obs || !saber_idx || !body_idx || !centers || !logits || !value || B < 1) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_forward: bad argument");
     const int64_t need = bsrl_note_forward_size(d, B);
@@ -203,7 +209,13 @@ extern "C" int bsrl_note_forward(const bsrl_note_desc* d, const float* const* pa
         BSRL_FAIL(BSRL_EINVAL, "bsrl_note_forward: workspace too small or unaligned");
     const NoteIndex at{d->n_blocks};
     const Image m(*d, static_cast<char*>(const_cast<void*>(image)));
-    const Work w(*d, B, static_cast<char*>(workspace));
+    Work w(*d, B, static_cast<char*>(workspace));
+    BlocksSave save = {};
+    if (saved) {
+        if (!note_train_saves(*d, B)) return BSRL_UNSUPPORTED;
+        if (saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256)) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_forward_saving: saved too small or unaligned");
+        save = note_train_blocks(*d, B, saved, &w.lead);
+    }
     const int64_t D = d->d, TR = d->trunk, H = d->hidden, HD = (int64_t)d->n_heads * D, NL = (int64_t)N_HEADS_ACT * d->n_gears;
     const int dt = d->dtype;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -228,12 +240,16 @@ extern "C" int bsrl_note_forward(const bsrl_note_desc* d, const float* const* pa
         if (!bsrl_mlp2_stream(e4, 4, PITCH, dt, st)) return BSRL_UNSUPPORTED;
         const bsrl_blocks_desc s = stack_of(*d);
         const int64_t frags = bsrl_blocks_pack_size(&s) - (int64_t)s.n_layers * (9 * D + s.ffn) * 4;
-        const BlocksPairPlan plan = blocks_pair_plan(w.tiles, (int)bsrl_blocks_pair_chunks(B), bsrl_cus(), B, s.n_layers, s.ffn);
+        BlocksPairPlan plan = blocks_pair_plan(w.tiles, (int)bsrl_blocks_pair_chunks(B), bsrl_cus(), B, s.n_layers, s.ffn);
+        if (saved) plan.env_ns = 0;
         const BlocksPairArgs p{static_cast<const uint4*>(m.blocks), reinterpret_cast<const float*>(static_cast<const char*>(m.blocks) + frags), w.x, w.bias, w.xres,
                                w.lead, w.pairs, plan, s.n_layers, s.ffn, T_TOK, N_LEAD, (int)(frags / (D / 16 * 1024))};
-        const int rc = bsrl_blocks_pair(p, d->d, dt, st);
-        if (rc != BSRL_UNSUPPORTED) STEP(rc);
-        STEP(bsrl_blocks_unless(&s, m.blocks, w.x, w.bias, w.xres, w.lead, B, rc == BSRL_OK ? &plan : nullptr, stream));
+        if (saved) STEP(bsrl_blocks_pair_save(p, save, dt, st));
+        else {
+            const int rc = bsrl_blocks_pair(p, d->d, dt, st);
+            if (rc != BSRL_UNSUPPORTED) STEP(rc);
+            STEP(bsrl_blocks_unless(&s, m.blocks, w.x, w.bias, w.xres, w.lead, B, rc == BSRL_OK ? &plan : nullptr, stream));
+        }
     }
     if ((parts & READOUT_PARTS) == READOUT_PARTS) {
         const Readout r(*d, params, m, w, centers, logits, value, B);

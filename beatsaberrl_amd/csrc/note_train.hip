@@ -10,9 +10,12 @@
 //   * gradients that torch would add up in passes of their own ride in epilogues: residual branches in ln_bwd (gx) and in the
 //     data-gradient GEMMs (res = y on the lead rows);
 //   * every launch is enqueued here, ~3 us of host time each.
-// Update of 16384 envs, recipe shape: 26.1 -> 19.6 ms; 1500 envs, default shape: 6.4 -> 3.7 ms (the rollout's forward, the loss
+// Past a round of the rollout's paired block stack (blocks_pair.hip, d = 192, more than 8 envs per CU) the stack's launch leaves the blocks'
+// activations here and this forward is what lies in front of it and behind it: 17.3 -> 13.9 ms for 16384 envs at the recipe's shape.  Up to
+// there the bin logits keep the op-by-op update's bits; past it the forward is the rollout's, nearer the fp32 one.
+// Update of 16384 envs, recipe shape, before that: 26.1 -> 19.6 ms; 1500 envs, default shape: 6.4 -> 3.7 ms (the rollout's forward, the loss
 // and torch's part of the backward included).
-#include "note_pack.h"
+#include "note_train.h"
 
 namespace {
 
@@ -235,6 +238,13 @@ struct Ops {
         return bsrl_attn_bwd_ragged(q, q_ld, k, kv_ld, v, kv_ld, s.noff, s.bias, dout, n.D, dq, q_ld, dk, kv_ld, dv, kv_ld, n.B, N_LEAD, N_NOTES, nq,
                                     n.d.n_heads, n.D / n.d.n_heads, dt, st);
     }
+    // q, k, v as the rollout's block stack left them: a head's rows after another's (blocks_pair.h)
+    int attn_bwd_heads(const u16* q, int64_t q_rows, const u16* k, const u16* v, const Saved& s, const u16* dout, u16* dq, int64_t dq_ld, u16* dk, u16* dv,
+                       int64_t dkv_ld, int64_t nq) const {
+        const int64_t dh = n.D / n.d.n_heads;
+        return bsrl_attn_bwd_ragged(q, dh, k, dh, v, dh, s.noff, s.bias, dout, n.D, dq, dq_ld, dk, dkv_ld, dv, dkv_ld, n.B, N_LEAD, N_NOTES, nq, n.d.n_heads, dh,
+                                    dt, st, q_rows * dh, n.R * dh);
+    }
     void copy(u16* dst, int64_t dld, const u16* src, int64_t sld, int group, int64_t gstride, int64_t rows, int64_t cols) const {
         const int64_t total = rows * (cols / 8);
         hipLaunchKernelGGL(rows_copy_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, reinterpret_cast<uint4*>(dst), dld / 8,
@@ -250,11 +260,11 @@ struct Ops {
 
 #define STEP(call) do { const int rc_ = (call); if (rc_ != BSRL_OK) return rc_; } while (0)
 
-int forward(const Net& n, const Saved& s, const float* const* P, const void* obs, int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
-            const int32_t* body_idx, float* vlogits, hipStream_t st) {
-    const int64_t B = n.B, D = n.D, F = n.F, TR = n.TR, H = n.H, LB = N_LEAD * B;
+// weights, offsets and the encoders; tokens: down to the first block's input (else to the encoders' hidden)
+int front(const Net& n, const Saved& s, const float* const* P, const void* obs, int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
+          const int32_t* body_idx, bool tokens, hipStream_t st) {
+    const int64_t B = n.B, D = n.D, LB = N_LEAD * B;
     const int dt = n.d.dtype;
-    const Ops o{n, s.noff + B, st, dt};
     pack_all(n, s, P, st);
     STEP(bsrl_note_counts(obs, obs_ld, obs_dtype, s.cnt, B, dt, st));
     STEP(bsrl_token_offsets(s.cnt, B, N_NOTES, s.noff, st));
@@ -269,8 +279,14 @@ int forward(const Net& n, const Saved& s, const float* const* P, const void* obs
         LinArgs c{k.hid, D, k.w2, p[3], nullptr, 0, x0 + ENC_AT[e] * D, D, nullptr, 0, 0, B * ENC_ROWS[e], (int)D, (int)D, 0, ENC_ROWS[e], N_LEAD * D, nullptr, 0};
         if (e == 3) { a.extra = c.extra = s.noff + B; c.y = x0 + LB * D; c.y_group = 0; c.y_gstride = 0; }
         STEP(bsrl_linear_run(a, BSRL_ACT_RELU, dt, dt, st, "bsrl_note_train"));
-        STEP(bsrl_linear_run(c, BSRL_ACT_NONE, dt, dt, st, "bsrl_note_train"));
+        if (tokens) STEP(bsrl_linear_run(c, BSRL_ACT_NONE, dt, dt, st, "bsrl_note_train"));
     }
+    return BSRL_OK;
+}
+
+int blocks(const Net& n, const Saved& s, const float* const* P, hipStream_t st) {
+    const int64_t B = n.B, D = n.D, F = n.F, LB = N_LEAD * B;
+    const Ops o{n, s.noff + B, st, n.d.dtype};
     for (int i = 0; i < n.L; ++i) {
         const auto& k = s.blk[i];
         const float* const* p = P + n.p_blk(i);
@@ -289,6 +305,13 @@ int forward(const Net& n, const Saved& s, const float* const* P, const void* obs
         STEP(o.linear(k.h2, D, k.w0, p[13], k.hid, F, D, F, !last, LB, BSRL_ACT_RELU));
         STEP(o.linear(k.hid, F, k.w2, p[15], last ? s.lead : s.blk[i + 1].x, D, F, D, !last, LB, BSRL_ACT_NONE, k.xm, D));
     }
+    return BSRL_OK;
+}
+
+// trunk and critic, from the block stack's rows
+int readout(const Net& n, const Saved& s, const float* const* P, float* vlogits, hipStream_t st) {
+    const int64_t B = n.B, D = n.D, TR = n.TR, H = n.H;
+    const Ops o{n, s.noff + B, st, n.d.dtype};
     const float* const* p = P + n.p_trunk();
     STEP(o.linear(s.lead, N_LEAD * D, s.wp, p[1], s.t, TR, N_LEAD * D, TR, false, B));
     STEP(o.ln(s.t, p + 2, s.u, s.s1, TR, false, B));
@@ -310,7 +333,7 @@ int forward(const Net& n, const Saved& s, const float* const* P, const void* obs
 }
 
 int backward(const Net& n, const Saved& s, const Scratch& c, const float* const* P, const float* dlogits, const float* dvlogits, float* grads,
-             const int64_t* off, hipStream_t st) {
+             const int64_t* off, bool by_head, hipStream_t st) {
     const int64_t B = n.B, D = n.D, F = n.F, TR = n.TR, H = n.H, LB = N_LEAD * B, HP = pad32(n.NL), BP = pad32(n.BINS);
     const Ops o{n, s.noff + B, st, n.d.dtype};
     auto G = [&](int p) { return grads + off[p]; };
@@ -365,7 +388,8 @@ int backward(const Net& n, const Saved& s, const Scratch& c, const float* const*
         batch[nb++] = o.wgrad(c.xm, D, k.att, D, G(q + 8), G(q + 9), D, D, !fin, LB);
         STEP(o.linear(c.xm, D, k.to, nullptr, c.dm, D, D, D, !fin, LB));
         if (fin) {
-            STEP(o.attn_bwd(k.q, D, k.qkv, k.qkv + D, 2 * D, s, c.dm, c.dq5, c.dqkv, c.dqkv + D, N_LEAD));
+            if (by_head) STEP(o.attn_bwd_heads(k.q, LB, k.qkv, k.qkv + n.R * D, s, c.dm, c.dq5, D, c.dqkv, c.dqkv + D, 2 * D, N_LEAD));
+            else STEP(o.attn_bwd(k.q, D, k.qkv, k.qkv + D, 2 * D, s, c.dm, c.dq5, c.dqkv, c.dqkv + D, N_LEAD));
             batch[nb++] = o.wgrad(c.dqkv, 2 * D, k.h, D, G(q + 4), G(q + 5), 2 * D, D, true, 0);
             batch[nb++] = o.wgrad(c.dq5, D, k.h, D, G(q + 2), G(q + 3), D, D, false, LB);
             STEP(o.linear(c.dqkv, 2 * D, k.tqkv, nullptr, c.dm, D, 2 * D, D, true, 0));
@@ -376,7 +400,8 @@ int backward(const Net& n, const Saved& s, const Scratch& c, const float* const*
             const int qc = n.p_critic();
             STEP(o.ln_bwd(c, last.x, c.gx, P[qc], s.sc, c.dqkv, n.R, c.g, G(qc), G(qc + 1), D, true, 0));
         } else {
-            STEP(o.attn_bwd(k.qkv, 3 * D, k.qkv + D, k.qkv + 2 * D, 3 * D, s, c.dm, c.dqkv, c.dqkv + D, c.dqkv + 2 * D, 0));
+            if (by_head) STEP(o.attn_bwd_heads(k.qkv, n.R, k.qkv + n.R * D, k.qkv + 2 * n.R * D, s, c.dm, c.dqkv, 3 * D, c.dqkv + D, c.dqkv + 2 * D, 3 * D, 0));
+            else STEP(o.attn_bwd(k.qkv, 3 * D, k.qkv + D, k.qkv + 2 * D, 3 * D, s, c.dm, c.dqkv, c.dqkv + D, c.dqkv + 2 * D, 0));
             batch[nb++] = o.wgrad(c.dqkv, 3 * D, k.h, D, G(q + 2), G(q + 3), 3 * D, D, true, 0);
             STEP(o.linear(c.dqkv, 3 * D, k.tqkv, nullptr, c.dm, D, 3 * D, D, true, 0));
             STEP(flush());
@@ -425,13 +450,58 @@ extern "C" int bsrl_note_train_forward(const bsrl_note_desc* d, const float* con
     const int64_t need = bsrl_note_train_size(d, B, 0);
     if (!need || !saved || saved_bytes < need || !bsrl_aligned(saved, 256)) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_forward: workspace too small or unaligned");
     const Net n(*d, B);
-    const int rc = forward(n, n.saved(static_cast<char*>(saved)), params, obs, obs_ld, obs_dtype, saber_idx, body_idx, vlogits, static_cast<hipStream_t>(stream));
+    const Saved s = n.saved(static_cast<char*>(saved));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    int rc = front(n, s, params, obs, obs_ld, obs_dtype, saber_idx, body_idx, true, st);
+    if (rc == BSRL_OK) rc = blocks(n, s, params, st);
+    if (rc == BSRL_OK) rc = readout(n, s, params, vlogits, st);
     if (rc == BSRL_OK) BSRL_CHECK_LAUNCH("bsrl_note_train_forward");
     return rc;
 }
 
-extern "C" int bsrl_note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
-                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
+bool note_train_saves(const bsrl_note_desc& d, int64_t B) {
+    return desc_ok(&d) && bsrl_blocks_pair_saves(B, (int)d.d, d.n_heads, d.ffn, N_LEAD + N_NOTES, bsrl_cus());
+}
+
+extern "C" int bsrl_note_train_saves(const bsrl_note_desc* d, int64_t B) { return d && B >= 1 && note_train_saves(*d, B); }
+
+BlocksSave note_train_blocks(const bsrl_note_desc& d, int64_t B, void* saved, u16** lead) {
+    const Net n(d, B);
+    const Saved s = n.saved(static_cast<char*>(saved));
+    BlocksSave b = {s.noff, (uint32_t)n.R, {}};
+    for (int i = 0; i < n.L; ++i) {
+        const auto& k = s.blk[i];
+        b.blk[i] = {k.x, k.h, k.qkv, k.q, k.att, k.xm, k.h2, k.hid, k.s1.mean, k.s1.rstd, k.s2.mean, k.s2.rstd};
+    }
+    *lead = s.lead;
+    return b;
+}
+
+extern "C" int bsrl_note_train_begin(const bsrl_note_desc* d, const float* const* params, const void* obs, int64_t obs_ld, int obs_dtype,
+                                     const int32_t* saber_idx, const int32_t* body_idx, int64_t B, void* saved, int64_t saved_bytes, bsrl_stream stream) {
+    if (!d || !note_train_saves(*d, B)) return BSRL_UNSUPPORTED;
+    if (!params || !obs || !saber_idx || !body_idx) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_begin: bad argument");
+    if (!saved || saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256)) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_begin: workspace too small or unaligned");
+    const Net n(*d, B);
+    const int rc = front(n, n.saved(static_cast<char*>(saved)), params, obs, obs_ld, obs_dtype, saber_idx, body_idx, false, static_cast<hipStream_t>(stream));
+    if (rc == BSRL_OK) BSRL_CHECK_LAUNCH("bsrl_note_train_begin");
+    return rc;
+}
+
+extern "C" int bsrl_note_train_end(const bsrl_note_desc* d, const float* const* params, float* vlogits, int64_t B, void* saved, int64_t saved_bytes,
+                                   bsrl_stream stream) {
+    if (!d || !note_train_saves(*d, B)) return BSRL_UNSUPPORTED;
+    if (!params || !vlogits) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_end: bad argument");
+    if (!saved || saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256)) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_end: workspace too small or unaligned");
+    const Net n(*d, B);
+    const int rc = readout(n, n.saved(static_cast<char*>(saved)), params, vlogits, static_cast<hipStream_t>(stream));
+    if (rc == BSRL_OK) BSRL_CHECK_LAUNCH("bsrl_note_train_end");
+    return rc;
+}
+
+static int note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
+                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bool by_head,
+                               bsrl_stream stream) {
     if (!desc_ok(d)) return BSRL_UNSUPPORTED;
     if (!params || !dlogits || !dvlogits || !grads || B < 1) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_backward: bad argument");
     if (!saved || saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256) || !scratch || scratch_bytes < bsrl_note_train_size(d, B, 1) ||
@@ -441,7 +511,17 @@ extern "C" int bsrl_note_train_backward(const bsrl_note_desc* d, const float* co
     n.layout(off);
     const Saved s = n.saved(static_cast<char*>(saved));
     const Scratch c(n, static_cast<char*>(scratch));
-    const int rc = backward(n, s, c, params, dlogits, dvlogits, grads, off, static_cast<hipStream_t>(stream));
+    const int rc = backward(n, s, c, params, dlogits, dvlogits, grads, off, by_head, static_cast<hipStream_t>(stream));
     if (rc == BSRL_OK) BSRL_CHECK_LAUNCH("bsrl_note_train_backward");
     return rc;
+}
+
+extern "C" int bsrl_note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
+                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
+    return note_train_backward(d, params, dlogits, dvlogits, grads, B, saved, saved_bytes, scratch, scratch_bytes, false, stream);
+}
+
+extern "C" int bsrl_note_train_stack_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
+                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
+    return note_train_backward(d, params, dlogits, dvlogits, grads, B, saved, saved_bytes, scratch, scratch_bytes, true, stream);
 }

@@ -262,6 +262,13 @@ class Block(nn.Module):
         return r + (v,) if want_v else r
 
 
+class _Update:
+    """A native update under way: its plan and parameters, and what the rollout forward in front of it has saved for it."""
+
+    def __init__(self, plan, params):
+        self.plan, self.params, self.saved = plan, params, None
+
+
 class _ValuesOf(torch.autograd.Function):
     """forward: `values`, bit for bit; backward: the incoming gradient goes to `graph` (same shape), the tensor whose
     autograd graph stands in for the way `values` were computed."""
@@ -453,7 +460,9 @@ class NotePolicy(nn.Module):
         # rollout takes - and sends their gradients through its own per-op graph (a function that differs from the
         # rollout's by 16-bit rounding, as any two 16-bit evaluations do).  Rollout and update outputs are then the
         # same bits in every mode and PPO's first-epoch ratio is exactly 1, for one more (fused, ~3 ms at the recipe
-        # shape and 16384 envs) forward per update pass.  "own": the update returns its own per-op values (the gap
+        # shape and 16384 envs) forward per update pass.  Where the library takes the update's block stack from that very
+        # forward (bsrl_note_train_saves: d = 192 past 8 envs per CU) the graph is its own, and there is no forward more.
+        # "own": the update returns its own per-op values (the gap
         # bounded in the tests).  No effect on the fp32 stream, whose two forwards are the same ops.
         self.update_values = "rollout"
         # sampling-call counter of the in-kernel Philox stream; on the device so that a captured
@@ -571,24 +580,26 @@ class NotePolicy(nn.Module):
             if self.update_values == "rollout" and self.fp16 and not self.rollout_matches_update:
                 arch = self._native_desc(self.stream_dtype)
                 params = None if arch is None else self._native_params(arch)
-                with torch.no_grad():
-                    r_out, r_value = self._rollout(obs, arch, params)       # the rollout's own routes, grad-free
                 plan = None if params is None else self._train_plan(arch)
+                update = None if plan is None else _Update(plan, params)
+                with torch.no_grad():
+                    r_out, r_value = self._rollout(obs, arch, params, update)       # the rollout's own routes, grad-free
                 if plan is not None:
-                    return self._forward_train_native(plan, params, obs, r_out, r_value)
+                    return self._forward_train_native(update, obs, r_out, r_value)
                 out, value = self._forward_train(obs)
                 return _ValuesOf.apply(out, r_out), _ValuesOf.apply(value, r_value)
             return self._forward_train(obs)
         return self._rollout(obs)
 
-    def _rollout(self, obs, arch=None, params=None):
-        """The forward-only routes.  arch, params: `_native_desc` and `_native_params` of this very call, where the caller has them."""
+    def _rollout(self, obs, arch=None, params=None, update=None):
+        """The forward-only routes.  arch, params: `_native_desc` and `_native_params` of this very call, where the caller has them;
+        update: the native update that this forward is the first half of."""
         with contextlib.ExitStack() as modes:
             if self.fp16 and self.fp16_accum != "off":
                 modes.enter_context(_fl.fp16_accum(self.fp16_accum))
             if self.fp16 and self.fused_ffn != "off":
                 modes.enter_context(_fl.ffn_fusion(self.fused_ffn))
-            return self._forward_stacked(obs, arch, params)
+            return self._forward_stacked(obs, arch, params, update)
 
     # ---- the fused routes as native calls ------------------------------------------------------
     def _native_desc(self, dt):
@@ -709,8 +720,9 @@ class NotePolicy(nn.Module):
                     params[i + j] = p.data_ptr()
         return params
 
-    def _forward_native(self, desc, image, params, obs):
-        """_forward_stacked on the fused routes: one call, or its four parts with the critic on the second stream."""
+    def _forward_native(self, desc, image, params, obs, update=None):
+        """_forward_stacked on the fused routes: one call, or its four parts with the critic on the second stream.  With an update
+        behind it that takes this batch's block stack, the stack leaves its activations there."""
         lib, B, dev = _lib.load(), obs.shape[0], obs.device
         logits = torch.empty(B, N_ACTION_HEADS, self.k_max, dtype=torch.float32, device=dev)
         value = torch.empty(B, dtype=torch.float32, device=dev)
@@ -719,13 +731,20 @@ class NotePolicy(nn.Module):
         args = (desc, params, image.data_ptr(), obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype), self._saber_idx32.data_ptr(),
                 self._body_idx32.data_ptr(), self.value_centers.data_ptr(), logits.data_ptr(), value.data_ptr(), B)
 
+        saved = None
+
         def run(parts, stream):
-            rc = lib.bsrl_note_forward(*args, parts, ws.data_ptr(), n, stream.cuda_stream)
+            if saved is None:
+                rc = lib.bsrl_note_forward(*args, parts, ws.data_ptr(), n, stream.cuda_stream)
+            else:
+                rc = lib.bsrl_note_forward_saving(*args, parts, ws.data_ptr(), n, saved.data_ptr(), saved.numel(), stream.cuda_stream)
             if not _lib.check(rc, "bsrl_note_forward"):
                 raise ops.Unsupported("bsrl_note_forward")
 
         with torch.cuda.device(dev):
             main = torch.cuda.current_stream(dev)
+            if update is not None:
+                saved = update.saved = update.plan.begin(update.params, obs, self._saber_idx32, self._body_idx32)
             if not self._overlaps(B) or self.critic_overlap_min_batch is None and lib.bsrl_note_one_call(desc, B):
                 run(15, main)
             else:
@@ -739,7 +758,7 @@ class NotePolicy(nn.Module):
         self._value_logits = None
         return logits, value
 
-    def _forward_stacked(self, obs, arch=None, params=None):
+    def _forward_stacked(self, obs, arch=None, params=None, update=None):
         dt = self.stream_dtype if self.fp16 else torch.float32
         B, d = obs.shape[0], self.embed
         if obs.shape[0]:
@@ -748,7 +767,7 @@ class NotePolicy(nn.Module):
             if masters is not None:
                 if obs.dtype is not torch.float32 and obs.dtype is not dt:
                     obs = obs.float()
-                return self._forward_native(*native, masters, obs if obs.stride(1) == 1 else obs.contiguous())
+                return self._forward_native(*native, masters, obs if obs.stride(1) == 1 else obs.contiguous(), update)
         # preamble in one kernel: the obs is rounded once to the stream dtype (policy.py:1200-1209),
         # gathered into the four encoder inputs (+ note-geometry lanes, one-hots) and the key bias
         if obs.dtype is not torch.float32 and obs.dtype is not dt:
@@ -920,15 +939,15 @@ class NotePolicy(nn.Module):
             c = self._train_plan_cache = (key, NoteTrainPlan(arch, self._native_shapes(arch)))
         return c[1] if c[1].supported else None
 
-    def _forward_train_native(self, plan, params, obs, r_out, r_value):
+    def _forward_train_native(self, update, obs, r_out, r_value):
         """The update forward as one native call (its backward is another); outputs are the rollout's, see NoteTrainFn."""
         obs = obs.detach()
         if obs.dtype is not torch.float32 and obs.dtype is not self.stream_dtype:
             obs = obs.float()
         if obs.stride(1) != 1:
             obs = obs.contiguous()
-        out, value, self._value_logits = NoteTrainFn.apply(plan, obs, self._saber_idx32, self._body_idx32, self.value_centers,
-                                                           r_out, r_value, *params)
+        out, value, self._value_logits = NoteTrainFn.apply(update.plan, obs, self._saber_idx32, self._body_idx32, self.value_centers,
+                                                           r_out, r_value, update.saved, *update.params)
         return out, value
 
     def _trunk_v2_train(self, z):

@@ -644,6 +644,27 @@ int bsrl_note_train_forward(const bsrl_note_desc* desc, const float* const* para
                             int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
                             const int32_t* body_idx, float* vlogits, int64_t B, void* saved,
                             int64_t saved_bytes, bsrl_stream stream);
+/* (ABI 22) The update's forward on the rollout forward's own block stack, which leaves what the backward reads: _begin fills
+ * `saved` up to the encoders, bsrl_note_forward_saving is bsrl_note_forward whose STACK part writes the blocks' share (the
+ * same logits and values), _end does trunk and critic; together they take the place of bsrl_note_train_forward, whose
+ * forward rounds the stream to 16 bits between blocks where this one does not.  _stack_backward: bsrl_note_train_backward of
+ * what they have saved (q, k, v lie otherwise).  _saves: 1 where they take B envs. */
+int bsrl_note_train_saves(const bsrl_note_desc* desc, int64_t B);
+int bsrl_note_train_begin(const bsrl_note_desc* desc, const float* const* params, const void* obs,
+                          int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
+                          const int32_t* body_idx, int64_t B, void* saved, int64_t saved_bytes,
+                          bsrl_stream stream);
+int bsrl_note_forward_saving(const bsrl_note_desc* desc, const float* const* params, const void* image,
+                             const void* obs, int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
+                             const int32_t* body_idx, const float* centers, float* logits, float* value,
+                             int64_t B, int parts, void* workspace, int64_t workspace_bytes,
+                             void* saved, int64_t saved_bytes, bsrl_stream stream);
+int bsrl_note_train_end(const bsrl_note_desc* desc, const float* const* params, float* vlogits, int64_t B,
+                        void* saved, int64_t saved_bytes, bsrl_stream stream);
+int bsrl_note_train_stack_backward(const bsrl_note_desc* desc, const float* const* params,
+                                   const float* dlogits, const float* dvlogits, float* grads, int64_t B,
+                                   void* saved, int64_t saved_bytes, void* scratch,
+                                   int64_t scratch_bytes, bsrl_stream stream);
 int bsrl_note_train_backward(const bsrl_note_desc* desc, const float* const* params,
                              const float* dlogits, const float* dvlogits, float* grads, int64_t B,
                              void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes,

@@ -1,0 +1,72 @@
+"""NotePolicy's native update on the rollout's block stack (d = 192, more than 8 envs per CU): values are the rollout's bits, gradients are at
+least as near the fp32 update's as those of the update that computes its own 16-bit stream, and what lies past a wave's rows - odd batches,
+envs without notes, envs too long to share a wave, an env by itself - reaches no other env's."""
+import pytest
+import torch
+
+from beatsaberrl_amd import _lib
+from beatsaberrl_amd.policy import NotePolicy, hl_loss
+from oracle import note_policy_ref as nr
+
+pytestmark = pytest.mark.gpu
+CUS = 256
+SCALE = 1024.0
+
+
+def _grads(m, obs, action, ret):
+    m.zero_grad(set_to_none=True)
+    _, logp, ent, value = m.get_action_and_value(obs, action)
+    loss = -(ret * logp).mean() - 0.01 * ent.mean() + 0.1 * ((value - ret) ** 2).mean() \
+        + 0.5 * hl_loss(m._value_logits, ret, m.value_centers, m.value_sigma)
+    (loss * (SCALE if m.fp16 else 1.0)).backward()
+    return value.detach(), {n: p.grad.detach().clone() / (SCALE if m.fp16 else 1.0) for n, p in m.named_parameters()}
+
+
+def _errors(got, want):
+    top = max(w.norm().item() for w in want.values())
+    return {n: (got[n] - w).norm().item() / (w.norm().item() + 1e-3 * top) for n, w in want.items()}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,notes,kw", [
+    (8 * CUS + 1, "mixed", dict(n_blocks=2)),
+    (8 * CUS + 63, "all", dict(n_blocks=1, ffn_mult=1)),                # nobody shares a wave
+    (9 * CUS - 1, "none", dict(n_blocks=2, ffn_mult=2)),
+    (3001, "ragged", dict(n_blocks=3, note_geo=True)),
+])
+def test_gradients_from_the_rollouts_stack(dtype, B, notes, kw):
+    torch.manual_seed(7)
+    m = NotePolicy(embed=192, trunk_dim=384, n_heads=4, n_gears=5, **kw).cuda()
+    with torch.no_grad():
+        for p in m.parameters():
+            if p.dim() == 1:
+                p.add_(0.1 * torch.randn_like(p))
+    g = torch.Generator().manual_seed(B)
+    obs = torch.randn(B, nr.OBS_DIM, generator=g) * 0.7
+    share = {"none": 0.0, "all": 1.1, "mixed": 0.6}.get(notes)
+    share = torch.rand(B, 1, generator=g) if share is None else share
+    obs[:, nr.OFF_MASK:nr.OFF_MASK + 24] = (torch.rand(B, 24, generator=g) < share).float()
+    obs, action, ret = obs.cuda(), torch.randint(0, 5, (B, 29), generator=g).cuda(), torch.randn(B, generator=g).cuda()
+    _, want = _grads(m, obs, action, ret)                               # fp32
+    m.fp16, m.stream_dtype = True, dtype
+    plan = m._train_plan()
+    assert _lib.load().bsrl_note_train_saves(plan.desc, B) == 1 and _lib.load().bsrl_note_train_saves(plan.desc, 8 * CUS) == 0
+    with torch.no_grad():
+        _, _, _, v = m.get_action_and_value(obs, action)
+    value, got = _grads(m, obs, action, ret)
+    assert torch.equal(value, v)
+    value2, again = _grads(m, obs, action, ret)
+    assert torch.equal(value2, v) and all(torch.equal(got[n], again[n]) for n in got)
+    type(plan).begin, begin = (lambda *a: None), type(plan).begin
+    try:
+        _, own = _grads(m, obs, action, ret)
+    finally:
+        type(plan).begin = begin
+    e_got, e_own = _errors(got, want), _errors(own, want)
+    worst = max(e_got.items(), key=lambda kv: kv[1])
+    mean = lambda e: sum(e.values()) / len(e)
+    print(f"\n{dtype} B={B} {notes}: worst {worst[0]} {worst[1]:.2e} (own stream {e_own[worst[0]]:.2e}), mean {mean(e_got):.3e} | {mean(e_own):.3e}")
+    # the two forwards differ in where the stream is rounded: for a single parameter either may be the nearer (seen: up to 1.7 times, a query
+    # bias at 4e-3), on average this one is
+    assert mean(e_got) <= 1.02 * mean(e_own)
+    assert all(e_got[n] <= 3 * e_own[n] + 1e-3 for n in e_got)
