@@ -89,6 +89,7 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
     uint32_t voff;                 // lane * 16
     uint32_t src_off, src_end;     // next stage to load, image length (bytes)
     uint32_t cur, prev;            // slot of the current stage and of the one before it (bytes from slot 0)
+    uint32_t due_slot[2], due_src[2];          // admit<.., SPREAD>: what the even and the odd stage of the pair have to load
     bool loader;
 
     __device__ __forceinline__ void issue(uint32_t slot_off) {
@@ -117,10 +118,22 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
 #pragma unroll
         for (int i = 0; i < SLOTS - 2; ++i) issue(i * STAGE_BYTES);
     }
+    // transfer K (of FPW) of the stage that admit<.., SPREAD> left to the even (0) or odd stage of its pair
+    template <int PARITY, int K> __device__ __forceinline__ void load_due() {
+        constexpr uint32_t step = K < 3 ? 0 : 3072;            // (the immediate offset ends at 4095)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3"
+                     ::"v"(voff), "s"(wsrc + due_src[PARITY] + step), "s"(wdst + due_slot[PARITY] + step), "n"(1024 * K - step));
+    }
+    template <int PARITY> __device__ __forceinline__ void load_due_all() {
+        static_for<0, FPW>([&](auto k) __attribute__((always_inline)) { load_due<PARITY, decltype(k)::value>(); });
+    }
     // entry of the next stage (PARITY = its index in its block, mod 2): on return it is readable in slot `cur`.  YOUNGER: other memory
     // instructions that this wave has certainly issued since the loads that are waited for, which need not be waited for then; where `more`
-    // holds, MORE of them
-    template <int PARITY, int YOUNGER = 0, int MORE = YOUNGER> __device__ __forceinline__ void admit(bool more = false) {
+    // holds, MORE of them.  SPREAD: the two stages behind are not requested here, where every wave's transfers meet in the 64 B/clk of the path
+    // into LDS and hold the waves up (350 - 600 clk per pair at four waves and 12 KB stages), but one by one by the pair's own stages
+    // (load_due; all of them before the next pair's admission).  blocks_pair.hip, 16384 envs: 2540 -> 2427 us; block_tail.h, where LDS reads
+    // take 80 - 100 % of what the LDS gives, the same to 1 % slower, and stays as it was
+    template <int PARITY, int YOUNGER = 0, int MORE = YOUNGER, bool SPREAD = false> __device__ __forceinline__ void admit(bool more = false) {
         const uint32_t older = prev;
         prev = cur;
         cur = cur + STAGE_BYTES == SLOTS * STAGE_BYTES ? 0 : cur + STAGE_BYTES;
@@ -135,8 +148,15 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
                              ::"s"(__builtin_amdgcn_readfirstlane((int)more)), "n"(FPW * AHEAD + YOUNGER), "n"(FPW * AHEAD + MORE) : "memory", "scc");
             else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FPW * AHEAD + YOUNGER) : "memory");
             blk_barrier();             // ... and every wave's have; every wave is done reading the two stages before this one
-            issue(older);
-            issue(prev);
+            if constexpr (SPREAD) {
+                static_assert(NLW == NW, "every wave loads");
+                due_slot[0] = older; due_slot[1] = prev;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) { due_src[i] = src_off; src_off = src_off + STAGE_BYTES == src_end ? 0 : src_off + STAGE_BYTES; }
+            } else {
+                issue(older);
+                issue(prev);
+            }
         }
     }
     // fragment i of the current stage, this lane's 16 bytes

@@ -166,9 +166,11 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
         if (ea < 0) {                                // no env: this wave only moves its share of the weight stream
             for (int l = 0; l < nl; ++l) {
                 for (int s = 0; s < a.total_stages / nl; s += 2) {
-                    pipe.template admit<0>();
+                    pipe.template admit<0, 0, 0, true>();
+                    pipe.template load_due_all<0>();
                     if (s == 0) fetch_vectors(l + 1 == nl ? 0 : l + 1);
                     pipe.template admit<1>();
+                    pipe.template load_due_all<1>();
                 }
                 vp ^= 1;
             }
@@ -279,8 +281,8 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
         // SAVE: what a wave stores, dealt behind the MFMAs of the stages of a block (0 .. 17 q|k|v, 18 .. 23 output projection, then the FFN's): the
         // rows that a LayerNorm reads where it reads them (LN), its output in the stages behind it, a head's q in the one behind it, its
         // k and v behind its attention, attention's output, the hidden in W2's.  Stores retire in order with the ring's loads, and the
-        // admission of stage s, in stage s - 1, waits for loads issued in stage s - 5: it need not wait for the stores of the three stages
-        // between.  None of them is conditional.
+        // admission of stage s, in stage s - 1, waits for loads issued up to fragment 6 of stage s - 4: it need not wait for the stores of the
+        // two stages since, nor for a LayerNorm's between them.  None of them is conditional.
         constexpr auto stored = [](int s, int tiles) {
             constexpr int Q = 2, KV = 16;
             const int t = s < 2 ? RT : tiles, first = (LINES * t + 2) / 2 - 2, all = 2 * LINES * t;           // (Rows' steps of the first stage of two; the first two of them store nothing)
@@ -289,8 +291,8 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
         };
         constexpr auto younger = [stored](int s, int tiles) {
             constexpr int LN = 2 + 2 * LINES;
-            int n = s == 2 || s == 4 ? RT * LN : s == 26 ? tiles * LN : 0;
-            for (int i = s - 4; i <= s - 2; ++i) n += i < 0 ? 0 : stored(i, tiles);
+            int n = s == 2 ? RT * LN : s == 26 ? tiles * LN : 0;
+            for (int i = s - 3; i <= s - 2; ++i) n += i < 0 ? 0 : stored(i, tiles);
             return n;
         };
         // slot i's share of n steps over a stage of `slots`
@@ -339,17 +341,19 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
                     if constexpr (n == SF) {
                         if constexpr (decltype(next)::even) {
                             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                            pipe.template admit<0, SAVE ? decltype(next)::Y : 0, SAVE ? decltype(next)::Z : 0>(more);
+                            pipe.template admit<0, SAVE ? decltype(next)::Y : 0, SAVE ? decltype(next)::Z : 0, true>(more);
                         } else pipe.template admit<1>();
                     }
                     wr[n % NBUF] = pipe.frag(n - SF, lane);              // (behind the last stage: read, not used)
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 mm(i_, wr[i % NBUF], fill);
+                // its share of the ring's loads, all before the admission above (fragment SF - NBUF + 1)
+                if constexpr (i % 3 == 0 && i / 3 < R::FPW) pipe.template load_due<std::is_same<decltype(next), Odd>::value ? 0 : 1, i / 3>();
                 __builtin_amdgcn_sched_barrier(0);
             });
         };
-        static_assert(SF % NBUF == 0, "rotating fragment registers");
+        static_assert(SF % NBUF == 0 && 3 * (R::FPW - 1) < SF - NBUF + 1, "rotating fragment registers; loads ahead of the admission");
         auto idle = [](auto) __attribute__((always_inline)) {};
 
         typedef BFrag8 Frags[RT][KC];                // LayerNorm's output
@@ -681,8 +685,11 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
             };
             typedef std::integral_constant<int, 0> K0; typedef std::integral_constant<int, 1> K1; typedef std::integral_constant<int, NH> KH; typedef std::integral_constant<int, TOT> KT;
             // chunk ch's accumulators and hidden alternate with chunk ch + 1's: two chunks per round, nothing moves
+            // (an admission among them has the stores of one odd chunk behind it: of stage s - 2, or of s - 4 behind its loads; the second
+            // one has as many of h2's)
+            static_assert(SF * QT * (QT + 2) / (2 * QT + 1) >= 7 * QT, "the hidden's stores behind fragment 6");
             auto half = [&](auto odd_, int ch, Acc& ca, Hid& ha, Acc& na, Hid& hb) __attribute__((always_inline)) {
-                stage(Even<2 * QT, younger(26, QT)>(), up(na), act_slots(KH(), KT(), ca, ha), ch < 2);        // W1(ch + 1); the second half of chunk ch's activation
+                stage(Even<2 * QT, younger(26, QT)>(), up(na), act_slots(KH(), KT(), ca, ha), ch == 0);        // W1(ch + 1); the second half of chunk ch's activation
                 load_bias(ch + 2 < nch ? ch + 2 : 0);
                 const auto act = act_slots(K0(), KH(), na, hb);
                 stage(Odd(), down(ha), [&](auto s_) __attribute__((always_inline)) { act(s_); save_hidden(s_, odd_, ch, ha); });      // W2(ch); the first half of chunk ch + 1's
@@ -722,7 +729,7 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
                 }
             }
         };
-        pipe.template admit<0>();
+        pipe.template admit<0, 0, 0, true>();
 #pragma unroll
         for (int f = 0; f < NBUF - 1; ++f) wr[f] = pipe.frag(f, lane);
         auto layer = [&](int l, auto qt_) __attribute__((always_inline)) {        // the final block's queries, output projection and FFN are the first tile's
