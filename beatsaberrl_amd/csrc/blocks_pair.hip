@@ -8,7 +8,7 @@
 // its own.  What bounds it: vector instructions beside the MFMAs, 2.7 for each (both envs' scores for a mixed query tile, LayerNorm out of
 // accumulation registers); MFMAs are busy for 0.4 of the time, the weight stream is not felt.
 // Whole forward, recipe shape (d = 192, six blocks, F = 768), f16, us, one env per wave / two: 1250 envs 398 / 379, 2048 441 / 400,
-// 4096 800 / 704, 8192 1598 / 1374, 16384 2986 / 2565; up to 4 envs per CU, where one env per wave leaves half of the waves away,
+// 4096 800 / 704, 8192 1598 / 1374, 16384 2986 / 2565 (the rollout since the ring's loads are spread over the stages: 2618 -> 2550); up to 4 envs per CU, where one env per wave leaves half of the waves away,
 // 328 / 379.  Narrower FFNs gain less and lose at F = d (blocks_pair.h).  At d = 128 the share of vector work is larger and two lost:
 // 16384 envs, bf16, 828 / 928.
 // Rows of a wave: lead tokens of A, lead tokens of B, A's attendable notes, B's; queries of the final block are then the first tile's.
@@ -21,7 +21,7 @@
 // blocks_pairs_pay.
 // SAVE: the update's forward is this kernel too (note_train.h).  It leaves what the backward reads of a block, 4.6 KB a row, as it goes:
 // 9 GB for 16384 envs at the recipe's shape, where the update's own forward had seven launches per block, each an HBM stream (4.8 ms beside
-// the 2.4 of this kernel without SAVE).  3.65 ms in one launch, and its stream is not rounded between blocks.  2.9 of them are the arithmetic
+// the 2.4 of this kernel without SAVE).  3.65 - 3.9 ms in one launch, by the card, and its stream is not rounded between blocks.  2.9 of them are the arithmetic
 // with every store taken out (LDS transposes, packing, addresses); the rest is the stores, which lie scattered over 40 000 rows at a time.
 #include "block_stage.h"
 #include "blocks_pair.h"
