@@ -388,9 +388,14 @@ class NoteTrainPlan:
     def pointers(self, params):
         return (ctypes.c_void_p * len(params))(*[p.data_ptr() for p in params])
 
+    def saves(self, B, device):
+        """Whether the update of B envs takes its block stack from the rollout forward (the size rule is the library's)."""
+        with torch.cuda.device(device):
+            return bool(_lib.load().bsrl_note_train_saves(self.desc, B))
+
     def begin(self, params, obs, saber_idx, body_idx):
         """The update's saved activations with everything in front of the block stack in them, for a rollout forward that writes
-        the blocks'; None where the update computes them itself (the size rule is the library's)."""
+        the blocks'; None where the update computes them itself."""
         lib, B = _lib.load(), obs.shape[0]
         if not lib.bsrl_note_train_saves(self.desc, B):
             return None

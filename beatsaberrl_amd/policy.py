@@ -660,9 +660,11 @@ class NotePolicy(nn.Module):
                 return None
         return params
 
-    def _native_image(self, dt, arch=None, params=None):
+    def _native_image(self, dt, arch=None, params=None, update=None, B=0):
         """(descriptor, weight image) of the native forward for the current weights version, or None where the forward runs op
-        by op.  The image is rebuilt IN PLACE, as `blocks_image` is: its address is stable under a captured graph."""
+        by op.  The image is rebuilt IN PLACE, as `blocks_image` is: its address is stable under a captured graph.  For an update
+        of B envs that takes this forward's block stack it is an image of its own, of the masters as they are now: the rest of
+        that update reads the masters themselves, and gradients must not mix two generations of them."""
         if (dt is torch.float32 or not self.fused_blocks_ok(dt) or not self.critic_pool
                 or not ops.critic_pool_supported(self.n_lead + N_NOTE_SLOTS, self.embed, self.n_heads, dt)):
             return None
@@ -677,16 +679,20 @@ class NotePolicy(nn.Module):
             c = self._native_cache = [-1, key, torch.zeros(n, dtype=torch.uint8, device=dev), desc]
         if c[2].numel() == 0:
             return None
-        if c[0] != _fl._weights_version:
+        own = update is not None and update.plan.saves(B, dev)
+        if own or c[0] != _fl._weights_version:
             params = params or self._native_params(arch)
             if params is None:
                 return None
+            image = torch.zeros_like(c[2]) if own else c[2]
             ptrs = (ctypes.c_void_p * len(params))(*[p.data_ptr() for p in params])
             gears = (ctypes.c_int32 * N_ACTION_HEADS)(*self.head_sizes)
             with torch.cuda.device(dev):
-                rc = _lib.load().bsrl_note_pack(c[3], ptrs, gears, c[2].data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+                rc = _lib.load().bsrl_note_pack(c[3], ptrs, gears, image.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
             if not _lib.check(rc, "bsrl_note_pack"):
                 raise ops.Unsupported("bsrl_note_pack")
+            if own:
+                return c[3], image
             c[0] = _fl._weights_version
         return c[3], c[2]
 
@@ -762,7 +768,7 @@ class NotePolicy(nn.Module):
         dt = self.stream_dtype if self.fp16 else torch.float32
         B, d = obs.shape[0], self.embed
         if obs.shape[0]:
-            native = self._native_image(dt, arch, params)
+            native = self._native_image(dt, arch, params, update, B)
             masters = None if native is None else self._native_masters(native[0])
             if masters is not None:
                 if obs.dtype is not torch.float32 and obs.dtype is not dt:
