@@ -424,9 +424,8 @@ class NoteTrainFn(torch.autograd.Function):
     def forward(ctx, plan, obs, saber_idx, body_idx, centers, r_logits, r_value, saved, *params):
         lib, B, dev = _lib.load(), obs.shape[0], obs.device
         vlogits = torch.empty(B, plan.desc.bins, dtype=torch.float32, device=dev)
-        ctx.stack = saved is not None
         with torch.cuda.device(dev):
-            if ctx.stack:                              # the rollout's block stack has left its activations there
+            if saved is not None:                      # the rollout's block stack has left its activations there
                 rc = lib.bsrl_note_train_end(plan.desc, plan.pointers(params), vlogits.data_ptr(), B, saved.data_ptr(), saved.numel(), ops._stream(obs))
             else:
                 size = lib.bsrl_note_train_size(plan.desc, B, 0)
@@ -463,8 +462,7 @@ class NoteTrainFn(torch.autograd.Function):
         n_scratch = lib.bsrl_note_train_size(plan.desc, B, 1)
         scratch = torch.empty(n_scratch, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
-            backward = lib.bsrl_note_train_stack_backward if ctx.stack else lib.bsrl_note_train_backward
-            rc = backward(plan.desc, plan.bwd_pointers(scales), g_logits.data_ptr(), g_vlogits.data_ptr(), flat.data_ptr(),
+            rc = lib.bsrl_note_train_backward(plan.desc, plan.bwd_pointers(scales), g_logits.data_ptr(), g_vlogits.data_ptr(), flat.data_ptr(),
                                               B, saved.data_ptr(), saved.numel(), scratch.data_ptr(), n_scratch, ops._stream(saved))
         if not _lib.check(rc, "bsrl_note_train_backward"):
             raise ops.Unsupported("bsrl_note_train_backward")

@@ -41,8 +41,11 @@ struct AttnBwdArgs {
     // compacted stream: env b's tokens are rows lead b + j (j < lead) and lead B + noff[b] + j - lead of k, v and their
     // gradients (batch strides unused, key_bias: of the optional rows); q, dout, dq likewise, or rows nq b + j with nq set
     const int32_t* noff; int lead, nq;
-    uint32_t q_hs = 0, kv_hs = 0;  // ... elements from a head to the next in q | k and v, where that is not dh
 };
+
+// compacted stream: where k, v lie, and how far rows and heads of q | k, v are apart (elements) - in[0], or in[1] where *apart is not zero.
+// (A parameter of its own: as a part of the one above it costs four registers at 4 x 48, which are spilled ones, and 11 % of the time.)
+struct AttnBwdWhere { struct In { const void *k, *v; int64_t q_rs, kv_rs; uint32_t q_hs, kv_hs; } in[2]; const float* apart; };
 
 typedef short s16x4v __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
@@ -72,7 +75,7 @@ __device__ __forceinline__ s16x4 row16(const u16* tile, int pitch, int r0, int c
 // RAG (COOP form only): the compacted stream.  Tile loops stop at the env's own token count; the next env's offsets are read
 // one round ahead, so that its row loads never wait for them.
 template <typename DT, int DH, bool COOP, int NKT, bool RAG = false>
-__global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwdArgs a) {
+__global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwdArgs a, AttnBwdWhere where) {
     constexpr int DHP = DH == 32 ? 48 : 56;     // LDS row pitch of the token tiles (elements)
     constexpr int FT = DH / 16;
     extern __shared__ __attribute__((aligned(16))) u16 smem[];
@@ -108,8 +111,10 @@ __global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwd
     u32x4v buf[4][NIT];                                             // native vectors: arrays of the uint4 class that live across a loop stay in scratch
     u16 kraw[NKT][4];                                            // key bias of keys 16 kt + 4 g + e, raw
     int nv_next = 0;
-    const int64_t rss[4] = {a.q_rs, a.do_rs, a.k_rs, a.v_rs};
-    const uint32_t q_hs = RAG && a.q_hs ? a.q_hs : DH, kv_hs = RAG && a.kv_hs ? a.kv_hs : DH, hss[4] = {q_hs, DH, kv_hs, kv_hs};
+    const AttnBwdWhere::In& in = where.in[RAG && where.apart && __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, *where.apart)) != 0 ? 1 : 0];
+    const int64_t rss[4] = {RAG ? in.q_rs : a.q_rs, a.do_rs, RAG ? in.kv_rs : a.k_rs, RAG ? in.kv_rs : a.v_rs};
+    const uint32_t hss[4] = {RAG ? in.q_hs : DH, DH, RAG ? in.kv_hs : DH, RAG ? in.kv_hs : DH};
+    const u16 *const ks = static_cast<const u16*>(RAG ? in.k : a.k), *const vs = static_cast<const u16*>(RAG ? in.v : a.v);
     const int prows[4] = {TQP, TQP, TP, TP};
     const int offs[4] = {0, TQP * DHP, 2 * TQP * DHP, 2 * TQP * DHP + TP * DHP};          // Qs, dOs, Ks, Vs inside a wave's region
     // piece c = it * gthreads + gt of a matrix is (row c / rp, head (c % rp) / PPR, part (c % rp) % PPR)
@@ -123,7 +128,7 @@ __global__ __launch_bounds__(COOP ? 512 : 128) void attn_bwd_mfma_kernel(AttnBwd
         const int nrows[4] = {nq_, nq_, nk_, nk_};
         const int64_t lead0 = be * a.lead, opt0 = a.B * a.lead + cur[0] - a.lead;       // RAG: row of token j
         const u16* srcs[4] = {static_cast<const u16*>(a.q) + (RAG ? 0 : be * a.q_bs) + h0 * DH, static_cast<const u16*>(a.dout) + (RAG ? 0 : be * a.do_bs) + h0 * DH,
-                              static_cast<const u16*>(a.k) + (RAG ? 0 : be * a.k_bs) + h0 * DH, static_cast<const u16*>(a.v) + (RAG ? 0 : be * a.v_bs) + h0 * DH};
+                              ks + (RAG ? 0 : be * a.k_bs) + h0 * DH, vs + (RAG ? 0 : be * a.v_bs) + h0 * DH};
 #pragma unroll
         for (int mtx = 0; mtx < 4; ++mtx) {
             int row = row_first, cp = cp_first;
@@ -434,17 +439,18 @@ extern "C" int bsrl_attn_bwd(const void* q, int64_t q_bs, int64_t q_rs, const vo
         // COOP workgroups are persistent (two resident per CU by LDS) and prefetch their next env
         int cus = 256, dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+        const AttnBwdWhere where = {};
         const int64_t resident = (int64_t)cus * 2;
         const dim3 grid(coop ? (unsigned)(B < resident ? B : resident) : (unsigned)((B * H + 1) / 2)), block(coop ? (unsigned)(64 * H) : 128u);
 #define AB_COOP(DT, DH) do { \
             auto kern = attn_bwd_mfma_kernel<DT, DH, true, 2>; \
             if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
                 (void)hipGetLastError(); return BSRL_UNSUPPORTED; } \
-            hipLaunchKernelGGL(kern, grid, block, lds, st, a); } while (0)
+            hipLaunchKernelGGL(kern, grid, block, lds, st, a, where); } while (0)
 #define AB_T(DT, DH) do { \
             if (coop) AB_COOP(DT, DH); \
-            else if (T <= 32) hipLaunchKernelGGL((attn_bwd_mfma_kernel<DT, DH, false, 2>), grid, block, lds, st, a); \
-            else hipLaunchKernelGGL((attn_bwd_mfma_kernel<DT, DH, false, 3>), grid, block, lds, st, a); } while (0)
+            else if (T <= 32) hipLaunchKernelGGL((attn_bwd_mfma_kernel<DT, DH, false, 2>), grid, block, lds, st, a, where); \
+            else hipLaunchKernelGGL((attn_bwd_mfma_kernel<DT, DH, false, 3>), grid, block, lds, st, a, where); } while (0)
         if (dtype == BSRL_F16) { if (dh == 32) AB_T(F16, 32); else AB_T(F16, 48); }
         else { if (dh == 32) AB_T(BF16, 32); else AB_T(BF16, 48); }
 #undef AB_T
@@ -455,23 +461,29 @@ extern "C" int bsrl_attn_bwd(const void* q, int64_t q_bs, int64_t q_rs, const vo
 }
 
 // Backward over the compacted stream (16-bit; workgroup = the heads of one env): dq, dk, dv row for row as q, k, v.  nq: queries
-// per env (q, dout, dq then hold nq B rows), 0 = every token.  q_hs, kv_hs: a head's rows of q | k and v by themselves, so many elements
-// from the next head's (0: beside it).
+// per env (q, dout, dq then hold nq B rows), 0 = every token.  apart: the other way that q, k, v may lie, which only the device knows.
 int bsrl_attn_bwd_ragged(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, const int32_t* noff,
                          const void* opt_bias, const void* dout, int64_t do_ld, void* dq, int64_t dq_ld, void* dk, int64_t dk_ld,
                          void* dv, int64_t dv_ld, int64_t B, int64_t lead, int64_t opt, int64_t nq, int64_t H, int64_t dh, int dtype,
-                         bsrl_stream stream, int64_t q_hs, int64_t kv_hs) {
+                         bsrl_stream stream, const AttnHeadsApart* apart) {
     const int64_t T = lead + opt, TQ = nq ? nq : T;
     if (!bsrl_attn_bwd_ragged_ok(T, H, dh, dtype) || lead < 1 || opt < 0 || nq < 0 || nq > lead || B * H > 0x7fffffff) return BSRL_UNSUPPORTED;
-    const int64_t lds_[] = {do_ld, dq_ld, dk_ld, dv_ld}, in_[] = {q_ld, k_ld, v_ld}, hs_[] = {q_hs, kv_hs, kv_hs};
+    const int64_t lds_[] = {q_ld, k_ld, v_ld, do_ld, dq_ld, dk_ld, dv_ld};
     for (int64_t s : lds_) if (s % 8 != 0 || s < H * dh) return BSRL_UNSUPPORTED;
-    for (int i = 0; i < 3; ++i) if (in_[i] % 8 != 0 || hs_[i] % 8 != 0 || hs_[i] < 0 || H * hs_[i] > 0xffffffffLL || in_[i] < (hs_[i] ? dh : H * dh)) return BSRL_UNSUPPORTED;
+    if (v_ld != k_ld) return BSRL_UNSUPPORTED;      // (k and v are of one buffer)
     const void* ptrs[] = {q, k, v, dout, dq, dk, dv};
     for (const void* p : ptrs) if (!p || !bsrl_aligned(p, 16)) return BSRL_UNSUPPORTED;
+    if (apart) {
+        const int64_t hs_[] = {apart->q_hs, apart->kv_hs};
+        for (int64_t s : hs_) if (s % 8 != 0 || s < dh || H * s > 0xffffffffLL) return BSRL_UNSUPPORTED;
+        if (!apart->flag || !apart->k || !apart->v || !bsrl_aligned(apart->k, 16) || !bsrl_aligned(apart->v, 16)) return BSRL_UNSUPPORTED;
+    }
     if (B == 0) return BSRL_OK;
     const int tp = (int)((T + 15) / 16) * 16, tqp = (int)((TQ + 15) / 16) * 16;
     AttnBwdArgs a{q, k, v, dout, 0, q_ld, 0, k_ld, 0, v_ld, 0, do_ld, opt_bias, nullptr, dq, dk, dv, 0, dq_ld, 0, dk_ld, 0, dv_ld,
-                  B, (int)T, (int)TQ, (int)H, (float)(1.0 / sqrt((double)dh)), wave_elems_of(tp, tqp, (int)dh), 1, noff, (int)lead, (int)nq, (uint32_t)q_hs, (uint32_t)kv_hs};
+                  B, (int)T, (int)TQ, (int)H, (float)(1.0 / sqrt((double)dh)), wave_elems_of(tp, tqp, (int)dh), 1, noff, (int)lead, (int)nq};
+    AttnBwdWhere where = {{{k, v, q_ld, k_ld, (uint32_t)dh, (uint32_t)dh}, {}}, nullptr};
+    if (apart) { where.apart = apart->flag; where.in[1] = {apart->k, apart->v, dh, dh, (uint32_t)apart->q_hs, (uint32_t)apart->kv_hs}; }
     const size_t lds = (size_t)H * a.wave_elems * sizeof(u16);
     const int64_t resident = (int64_t)bsrl_cus() * 2;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -479,7 +491,7 @@ int bsrl_attn_bwd_ragged(const void* q, int64_t q_ld, const void* k, int64_t k_l
         auto kern = attn_bwd_mfma_kernel<DT, DH, true, 2, true>; \
         if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
             (void)hipGetLastError(); return BSRL_UNSUPPORTED; } \
-        hipLaunchKernelGGL(kern, dim3((unsigned)(B < resident ? B : resident)), dim3((unsigned)(64 * H)), lds, st, a); } while (0)
+        hipLaunchKernelGGL(kern, dim3((unsigned)(B < resident ? B : resident)), dim3((unsigned)(64 * H)), lds, st, a, where); } while (0)
     if (dtype == BSRL_F16) { if (dh == 32) AB_RAG(F16, 32); else AB_RAG(F16, 48); }
     else { if (dh == 32) AB_RAG(BF16, 32); else AB_RAG(BF16, 48); }
 #undef AB_RAG

@@ -93,10 +93,13 @@ int bsrl_attn_ragged_slots(const void* q, int64_t q_ld, const void* k, int64_t k
                            const uint8_t* slots, const void* opt_bias, void* out, int64_t out_ld, int64_t B, int64_t lead, int64_t opt,
                            int64_t n_queries, int64_t H, int64_t dh, int dtype, bsrl_stream stream, const int32_t* go = nullptr);
 bool bsrl_attn_bwd_ragged_ok(int64_t T, int64_t H, int64_t dh, int dtype);
+// apart: where *flag (device) is not zero, q, k, v lie head after head, a head's rows one after another and the next head's q_hs | kv_hs
+// elements on, k and v at these addresses; where it is zero as the other arguments say
+struct AttnHeadsApart { const float* flag; const void *k, *v; int64_t q_hs, kv_hs; };
 int bsrl_attn_bwd_ragged(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, const int32_t* noff,
                          const void* opt_bias, const void* dout, int64_t do_ld, void* dq, int64_t dq_ld, void* dk, int64_t dk_ld,
                          void* dv, int64_t dv_ld, int64_t B, int64_t lead, int64_t opt, int64_t nq, int64_t H, int64_t dh, int dtype,
-                         bsrl_stream stream, int64_t q_hs = 0, int64_t kv_hs = 0);
+                         bsrl_stream stream, const AttnHeadsApart* apart = nullptr);
 // NotePolicy front end into the compacted stream (frontend.hip): counts of the attendable notes, then the padded encoder inputs
 // with the note rows and their key bias at noff[b], and the token in each key slot (slots (B, 32), 255 = dropped)
 int bsrl_note_counts(const void* obs, int64_t obs_ld, int obs_dtype, int32_t* counts, int64_t B, int dtype, bsrl_stream stream);

@@ -45,7 +45,7 @@ struct Stats { float *mean, *rstd; };
 struct Saved {
     struct Enc { u16 *in, *hid, *w0, *w2, *t2; } enc[4];
     struct Blk { u16 *x, *h, *qkv, *q, *att, *xm, *h2, *hid; Stats s1, s2; u16 *wqkv, *tqkv, *tq, *wo, *to, *w0, *t0, *w2, *t2; float* bqkv; } blk[BSRL_MAX_LAYERS];
-    int32_t *noff, *cnt; u16* bias; uint8_t* slots;
+    int32_t *noff, *cnt; u16* bias; uint8_t* slots; float* apart;               // apart: 1 where the blocks' q, k, v lie head after head (blocks_pair.h), else 0
     u16 *lead, *t, *u, *r, *t2; Stats s1, s2;                                  // trunk
     u16 *wp, *tp, *wf1, *tf1, *wf2, *tf2, *th;
     u16 *hv, *cq, *ckv, *catt, *z, *c1, *c2; Stats sc;                              // critic
@@ -63,7 +63,7 @@ struct Net : NoteIndex {
         Saved s; Bump b{base};
         auto mat = [&](int64_t r, int64_t c) { return b.take<u16>((size_t)(r * c)); };
         auto stats = [&](int64_t r) { Stats st; st.mean = b.take<float>(r); st.rstd = b.take<float>(r); return st; };
-        s.noff = b.take<int32_t>(B + 1); s.cnt = b.take<int32_t>(B); s.bias = b.take<u16>(B * N_NOTES); s.slots = b.take<uint8_t>(B * 32);
+        s.noff = b.take<int32_t>(B + 1); s.cnt = b.take<int32_t>(B); s.bias = b.take<u16>(B * N_NOTES); s.slots = b.take<uint8_t>(B * 32); s.apart = b.take<float>(1);
         for (int e = 0; e < 4; ++e) s.enc[e] = {mat(B * ENC_ROWS[e], PITCH), mat(B * ENC_ROWS[e], D), mat(D, PITCH), mat(D, D), mat(D, D)};
         for (int i = 0; i < L; ++i) {
             auto& k = s.blk[i];
@@ -166,8 +166,9 @@ bool desc_ok(const bsrl_note_desc* d) {
            bsrl_attn_bwd_ragged_ok(N_LEAD + N_NOTES, d->n_heads, d->d / d->n_heads, d->dtype);
 }
 
-void pack_all(const Net& n, const Saved& s, const float* const* P, hipStream_t st) {
+void pack_all(const Net& n, const Saved& s, const float* const* P, bool apart, hipStream_t st) {
     Packer k(st, n.d.dtype);
+    k.add(P[0], 1, 0, s.apart, 1, nullptr, 0, 1, 1, true, apart ? 1.f : 0.f);      // (nothing but its fill)
     const int64_t D = n.D, F = n.F, TR = n.TR, H = n.H;
     for (int e = 0; e < 4; ++e) {
         k.add(P[4 * e], D, n.enc_in(e), s.enc[e].w0, PITCH, nullptr, 0, 0, PITCH);
@@ -234,16 +235,9 @@ struct Ops {
         return bsrl_attn_ragged_slots(q, q_ld, k, kv_ld, v, kv_ld, s.noff, s.slots, s.bias, out, n.D, n.B, N_LEAD, N_NOTES, nq, n.d.n_heads, n.D / n.d.n_heads, dt, st);
     }
     int attn_bwd(const u16* q, int64_t q_ld, const u16* k, const u16* v, int64_t kv_ld, const Saved& s, const u16* dout, u16* dq, u16* dk, u16* dv,
-                 int64_t nq) const {
+                 int64_t nq, const AttnHeadsApart* apart = nullptr) const {
         return bsrl_attn_bwd_ragged(q, q_ld, k, kv_ld, v, kv_ld, s.noff, s.bias, dout, n.D, dq, q_ld, dk, kv_ld, dv, kv_ld, n.B, N_LEAD, N_NOTES, nq,
-                                    n.d.n_heads, n.D / n.d.n_heads, dt, st);
-    }
-    // q, k, v as the rollout's block stack left them: a head's rows after another's (blocks_pair.h)
-    int attn_bwd_heads(const u16* q, int64_t q_rows, const u16* k, const u16* v, const Saved& s, const u16* dout, u16* dq, int64_t dq_ld, u16* dk, u16* dv,
-                       int64_t dkv_ld, int64_t nq) const {
-        const int64_t dh = n.D / n.d.n_heads;
-        return bsrl_attn_bwd_ragged(q, dh, k, dh, v, dh, s.noff, s.bias, dout, n.D, dq, dq_ld, dk, dkv_ld, dv, dkv_ld, n.B, N_LEAD, N_NOTES, nq, n.d.n_heads, dh,
-                                    dt, st, q_rows * dh, n.R * dh);
+                                    n.d.n_heads, n.D / n.d.n_heads, dt, st, apart);
     }
     void copy(u16* dst, int64_t dld, const u16* src, int64_t sld, int group, int64_t gstride, int64_t rows, int64_t cols) const {
         const int64_t total = rows * (cols / 8);
@@ -260,12 +254,12 @@ struct Ops {
 
 #define STEP(call) do { const int rc_ = (call); if (rc_ != BSRL_OK) return rc_; } while (0)
 
-// weights, offsets and the encoders; tokens: down to the first block's input (else to the encoders' hidden)
+// weights, offsets and the encoders; tokens: down to the first block's input, for `blocks` (else to the encoders' hidden, for the rollout's stack)
 int front(const Net& n, const Saved& s, const float* const* P, const void* obs, int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
           const int32_t* body_idx, bool tokens, hipStream_t st) {
     const int64_t B = n.B, D = n.D, LB = N_LEAD * B;
     const int dt = n.d.dtype;
-    pack_all(n, s, P, st);
+    pack_all(n, s, P, !tokens, st);
     STEP(bsrl_note_counts(obs, obs_ld, obs_dtype, s.cnt, B, dt, st));
     STEP(bsrl_token_offsets(s.cnt, B, N_NOTES, s.noff, st));
     STEP(bsrl_note_frontend_rows(obs, obs_ld, obs_dtype, saber_idx, body_idx, n.d.note_geo, n.d.flux, n.d.z_asinh, s.noff, s.enc[0].in, s.enc[1].in,
@@ -333,11 +327,12 @@ int readout(const Net& n, const Saved& s, const float* const* P, float* vlogits,
 }
 
 int backward(const Net& n, const Saved& s, const Scratch& c, const float* const* P, const float* dlogits, const float* dvlogits, float* grads,
-             const int64_t* off, bool by_head, hipStream_t st) {
+             const int64_t* off, hipStream_t st) {
     const int64_t B = n.B, D = n.D, F = n.F, TR = n.TR, H = n.H, LB = N_LEAD * B, HP = pad32(n.NL), BP = pad32(n.BINS);
     const Ops o{n, s.noff + B, st, n.d.dtype};
     auto G = [&](int p) { return grads + off[p]; };
     const auto& last = s.blk[n.L - 1];
+    const bool either = note_train_saves(n.d, B);      // the forward may have been either: Saved::apart says which
     // weight gradients wait for each other: one launch per part of the net and tile shape, before their operands' buffers are used again
     WgradProblem batch[12];
     int nb = 0;
@@ -388,8 +383,8 @@ int backward(const Net& n, const Saved& s, const Scratch& c, const float* const*
         batch[nb++] = o.wgrad(c.xm, D, k.att, D, G(q + 8), G(q + 9), D, D, !fin, LB);
         STEP(o.linear(c.xm, D, k.to, nullptr, c.dm, D, D, D, !fin, LB));
         if (fin) {
-            if (by_head) STEP(o.attn_bwd_heads(k.q, LB, k.qkv, k.qkv + n.R * D, s, c.dm, c.dq5, D, c.dqkv, c.dqkv + D, 2 * D, N_LEAD));
-            else STEP(o.attn_bwd(k.q, D, k.qkv, k.qkv + D, 2 * D, s, c.dm, c.dq5, c.dqkv, c.dqkv + D, N_LEAD));
+            const AttnHeadsApart apart{s.apart, k.qkv, k.qkv + n.R * D, LB * (D / n.d.n_heads), n.R * (D / n.d.n_heads)};
+            STEP(o.attn_bwd(k.q, D, k.qkv, k.qkv + D, 2 * D, s, c.dm, c.dq5, c.dqkv, c.dqkv + D, N_LEAD, either ? &apart : nullptr));
             batch[nb++] = o.wgrad(c.dqkv, 2 * D, k.h, D, G(q + 4), G(q + 5), 2 * D, D, true, 0);
             batch[nb++] = o.wgrad(c.dq5, D, k.h, D, G(q + 2), G(q + 3), D, D, false, LB);
             STEP(o.linear(c.dqkv, 2 * D, k.tqkv, nullptr, c.dm, D, 2 * D, D, true, 0));
@@ -400,8 +395,8 @@ int backward(const Net& n, const Saved& s, const Scratch& c, const float* const*
             const int qc = n.p_critic();
             STEP(o.ln_bwd(c, last.x, c.gx, P[qc], s.sc, c.dqkv, n.R, c.g, G(qc), G(qc + 1), D, true, 0));
         } else {
-            if (by_head) STEP(o.attn_bwd_heads(k.qkv, n.R, k.qkv + n.R * D, k.qkv + 2 * n.R * D, s, c.dm, c.dqkv, 3 * D, c.dqkv + D, c.dqkv + 2 * D, 3 * D, 0));
-            else STEP(o.attn_bwd(k.qkv, 3 * D, k.qkv + D, k.qkv + 2 * D, 3 * D, s, c.dm, c.dqkv, c.dqkv + D, c.dqkv + 2 * D, 0));
+            const AttnHeadsApart apart{s.apart, k.qkv + n.R * D, k.qkv + 2 * n.R * D, n.R * (D / n.d.n_heads), n.R * (D / n.d.n_heads)};
+            STEP(o.attn_bwd(k.qkv, 3 * D, k.qkv + D, k.qkv + 2 * D, 3 * D, s, c.dm, c.dqkv, c.dqkv + D, c.dqkv + 2 * D, 0, either ? &apart : nullptr));
             batch[nb++] = o.wgrad(c.dqkv, 3 * D, k.h, D, G(q + 2), G(q + 3), 3 * D, D, true, 0);
             STEP(o.linear(c.dqkv, 3 * D, k.tqkv, nullptr, c.dm, D, 3 * D, D, true, 0));
             STEP(flush());
@@ -499,9 +494,8 @@ extern "C" int bsrl_note_train_end(const bsrl_note_desc* d, const float* const* 
     return rc;
 }
 
-static int note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
-                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bool by_head,
-                               bsrl_stream stream) {
+extern "C" int bsrl_note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
+                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
     if (!desc_ok(d)) return BSRL_UNSUPPORTED;
     if (!params || !dlogits || !dvlogits || !grads || B < 1) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_train_backward: bad argument");
     if (!saved || saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256) || !scratch || scratch_bytes < bsrl_note_train_size(d, B, 1) ||
@@ -511,17 +505,13 @@ static int note_train_backward(const bsrl_note_desc* d, const float* const* para
     n.layout(off);
     const Saved s = n.saved(static_cast<char*>(saved));
     const Scratch c(n, static_cast<char*>(scratch));
-    const int rc = backward(n, s, c, params, dlogits, dvlogits, grads, off, by_head, static_cast<hipStream_t>(stream));
+    const int rc = backward(n, s, c, params, dlogits, dvlogits, grads, off, static_cast<hipStream_t>(stream));
     if (rc == BSRL_OK) BSRL_CHECK_LAUNCH("bsrl_note_train_backward");
     return rc;
 }
 
-extern "C" int bsrl_note_train_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
-                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
-    return note_train_backward(d, params, dlogits, dvlogits, grads, B, saved, saved_bytes, scratch, scratch_bytes, false, stream);
-}
-
+// (its name in ABI 22, when it took the one layout of q, k, v and bsrl_note_train_backward the other)
 extern "C" int bsrl_note_train_stack_backward(const bsrl_note_desc* d, const float* const* params, const float* dlogits, const float* dvlogits, float* grads,
-                                        int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
-    return note_train_backward(d, params, dlogits, dvlogits, grads, B, saved, saved_bytes, scratch, scratch_bytes, true, stream);
+                                              int64_t B, void* saved, int64_t saved_bytes, void* scratch, int64_t scratch_bytes, bsrl_stream stream) {
+    return bsrl_note_train_backward(d, params, dlogits, dvlogits, grads, B, saved, saved_bytes, scratch, scratch_bytes, stream);
 }

@@ -4,7 +4,7 @@ envs without notes, envs too long to share a wave, an env by itself - reaches no
 import pytest
 import torch
 
-from beatsaberrl_amd import _lib, fp16_linear
+from beatsaberrl_amd import _lib, fp16_linear, ops
 from beatsaberrl_amd.policy import NotePolicy, hl_loss
 from oracle import note_policy_ref as nr
 
@@ -104,3 +104,66 @@ def test_an_update_is_of_one_generation_of_weights():
     with torch.no_grad():
         _, _, _, v = m.get_action_and_value(*batch[:2])
     assert torch.equal(v, value)                                        # the rollout's image is the bumped version's
+
+
+class _Calls:
+    """The C entry points on a policy and a batch."""
+
+    def __init__(self, m, obs):
+        self.lib, self.m, self.obs, self.B, self.dev = _lib.load(), m, obs, obs.shape[0], obs.device
+        arch = m._native_desc(m.stream_dtype)
+        self.params, self.plan = m._native_params(arch), m._train_plan(arch)
+        self.desc, self.image = m._native_image(m.stream_dtype)
+        self.ws = self.bytes(self.lib.bsrl_note_forward_size(self.desc, self.B))
+        self.vlogits = torch.zeros(self.B, m.value_bins, device=self.dev)
+
+    def bytes(self, n):
+        return torch.zeros(n, dtype=torch.uint8, device=self.dev)
+
+    def saved(self):
+        return self.bytes(self.lib.bsrl_note_train_size(self.plan.desc, self.B, 0))
+
+    @property
+    def _in(self):
+        m, obs = self.m, self.obs
+        return obs.data_ptr(), obs.stride(0), ops.dt_code(obs.dtype), m._saber_idx32.data_ptr(), m._body_idx32.data_ptr()
+
+    def rollout(self, parts=15, saved=None, out=None):
+        m, logits, value = self.m, *(out or (torch.zeros(self.B, 29, self.m.k_max, device=self.dev), torch.zeros(self.B, device=self.dev)))
+        args = (self.desc, m._native_masters(self.desc), self.image.data_ptr(), *self._in, m.value_centers.data_ptr(), logits.data_ptr(), value.data_ptr(),
+                self.B, parts, self.ws.data_ptr(), self.ws.numel())
+        rc = self.lib.bsrl_note_forward(*args, 0) if saved is None else self.lib.bsrl_note_forward_saving(*args, saved.data_ptr(), saved.numel(), 0)
+        assert rc == 0
+        return logits, value
+
+    def own(self, saved):
+        assert self.lib.bsrl_note_train_forward(self.plan.desc, self.plan.pointers(self.params), *self._in, self.vlogits.data_ptr(), self.B, saved.data_ptr(),
+                                                saved.numel(), 0) == 0
+
+    def stack(self, saved):
+        assert self.lib.bsrl_note_train_begin(self.plan.desc, self.plan.pointers(self.params), *self._in, self.B, saved.data_ptr(), saved.numel(), 0) == 0
+        out = self.rollout(saved=saved)
+        assert self.lib.bsrl_note_train_end(self.plan.desc, self.plan.pointers(self.params), self.vlogits.data_ptr(), self.B, saved.data_ptr(), saved.numel(), 0) == 0
+        return out
+
+    def backward(self, saved, name="bsrl_note_train_backward"):
+        g = torch.Generator(device=self.dev).manual_seed(1)
+        dl, dv = (torch.randn(self.B, n, generator=g, device=self.dev) * SCALE / self.B for n in (29 * self.m.k_max, self.m.value_bins))
+        flat, scratch = torch.zeros(self.plan.total, device=self.dev), self.bytes(self.lib.bsrl_note_train_size(self.plan.desc, self.B, 1))
+        scales = [self.params[i] for i in self.plan.bwd_params]
+        assert getattr(self.lib, name)(self.plan.desc, self.plan.bwd_pointers(scales), dl.data_ptr(), dv.data_ptr(), flat.data_ptr(), self.B, saved.data_ptr(),
+                                       saved.numel(), scratch.data_ptr(), scratch.numel(), 0) == 0
+        return flat
+
+
+def test_either_backward_takes_what_either_forward_has_saved():
+    m = _policy(torch.float16, n_blocks=2)
+    c = _Calls(m, _batch(8 * CUS + 5)[0])
+    saved, flats = c.saved(), {}
+    for forward in (c.own, c.stack, c.own):                             # the last one into what the second has left
+        forward(saved)
+        flats[forward.__name__] = [c.backward(saved, n) for n in ("bsrl_note_train_backward", "bsrl_note_train_stack_backward")]
+    for name, (a, b) in flats.items():
+        assert torch.equal(a, b), name
+    a, b = flats["own"][0], flats["stack"][0]
+    assert (a - b).norm() <= 2e-2 * a.norm()                            # the same gradients, through other 16-bit roundings of the stream
