@@ -50,9 +50,10 @@ int bsrl_blocks_unless(const bsrl_blocks_desc* d, const void* packed, const void
 // < lead of env b at lead b + t, its i-th attendable note at lead B + noff[b] + i.  x, h: the block's input and its LayerNorm; qkv: q, k, v
 // (k, v in the final block, q by itself: its lead rows), each head after head, a head's rows (d / heads wide) one after another - a whole line
 // at a time, where rows of all heads took its 96 bytes each at a time: 4.1 -> 3.65 ms for the recipe's 16384 envs -, v without its bias; att: attention's output; xm, h2, hid: the stream behind it, its
-// LayerNorm, the FFN's hidden; mean, rstd: of the two LayerNorms.  In the final block q, att and what follows are the lead rows'.
+// LayerNorm, the FFN's hidden; mean, rstd: of the two LayerNorms.  In the final block q, att and what follows are the lead rows'.  lead: the
+// stack's output rows once more, beside the workspace's, from which the rollout's own readout goes on.
 struct BlocksSaveLayer { u16 *x, *h, *qkv, *q, *att, *xm, *h2, *hid; float *mean1, *rstd1, *mean2, *rstd2; };
-struct BlocksSave { const int32_t* noff; uint32_t rows; BlocksSaveLayer blk[BSRL_MAX_LAYERS]; };       // rows: what every buffer has room for
+struct BlocksSave { const int32_t* noff; u16* lead; uint32_t rows; BlocksSaveLayer blk[BSRL_MAX_LAYERS]; };       // rows: what every buffer has room for
 // bsrl_blocks_pair (every env, whether pairs pay or not: a plan with env_ns = 0) that saves them
 bool bsrl_blocks_pair_saves(int64_t B, int d, int heads, int F, int T, int cus);
 int bsrl_blocks_pair_save(const BlocksPairArgs& a, const BlocksSave& save, int dtype, hipStream_t st);

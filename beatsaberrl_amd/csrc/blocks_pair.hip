@@ -750,11 +750,13 @@ __global__ __launch_bounds__(256, 1) void blocks_pair_kernel(BlocksPairArgs a, B
         for (int l = 0; l + 1 < nl; ++l) layer(l, QA());
         layer(nl - 1, Q1());
         if (tok[0] < lead) {                         // the first 2 lead rows
-            u16* o = a.x_out + ((int64_t)(isb[0] ? eb : ea) * lead + tok[0]) * D;
+            const int64_t at = ((int64_t)(isb[0] ? eb : ea) * lead + tok[0]) * D + 4 * g;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 const f32x4 r = x[0][nt];
-                *reinterpret_cast<uint2*>(o + 16 * nt + 4 * g) = make_uint2(bpack2<DT>(r[0], r[1]), bpack2<DT>(r[2], r[3]));
+                const uint2 q = make_uint2(bpack2<DT>(r[0], r[1]), bpack2<DT>(r[2], r[3]));
+                *reinterpret_cast<uint2*>(a.x_out + at + 16 * nt) = q;
+                if constexpr (SAVE) *reinterpret_cast<uint2*>(save.lead + at + 16 * nt) = q;
             }
         }
     }

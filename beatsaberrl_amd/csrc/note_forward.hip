@@ -209,12 +209,12 @@ extern "C" int bsrl_note_forward_saving(const bsrl_note_desc* d, const float* co
         BSRL_FAIL(BSRL_EINVAL, "bsrl_note_forward: workspace too small or unaligned");
     const NoteIndex at{d->n_blocks};
     const Image m(*d, static_cast<char*>(const_cast<void*>(image)));
-    Work w(*d, B, static_cast<char*>(workspace));
+    const Work w(*d, B, static_cast<char*>(workspace));
     BlocksSave save = {};
     if (saved) {
         if (!note_train_saves(*d, B)) return BSRL_UNSUPPORTED;
         if (saved_bytes < bsrl_note_train_size(d, B, 0) || !bsrl_aligned(saved, 256)) BSRL_FAIL(BSRL_EINVAL, "bsrl_note_forward_saving: saved too small or unaligned");
-        save = note_train_blocks(*d, B, saved, &w.lead);
+        save = note_train_blocks(*d, B, saved);
     }
     const int64_t D = d->d, TR = d->trunk, H = d->hidden, HD = (int64_t)d->n_heads * D, NL = (int64_t)N_HEADS_ACT * d->n_gears;
     const int dt = d->dtype;

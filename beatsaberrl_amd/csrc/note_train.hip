@@ -460,15 +460,14 @@ bool note_train_saves(const bsrl_note_desc& d, int64_t B) {
 
 extern "C" int bsrl_note_train_saves(const bsrl_note_desc* d, int64_t B) { return d && B >= 1 && note_train_saves(*d, B); }
 
-BlocksSave note_train_blocks(const bsrl_note_desc& d, int64_t B, void* saved, u16** lead) {
+BlocksSave note_train_blocks(const bsrl_note_desc& d, int64_t B, void* saved) {
     const Net n(d, B);
     const Saved s = n.saved(static_cast<char*>(saved));
-    BlocksSave b = {s.noff, (uint32_t)n.R, {}};
+    BlocksSave b = {s.noff, s.lead, (uint32_t)n.R, {}};
     for (int i = 0; i < n.L; ++i) {
         const auto& k = s.blk[i];
         b.blk[i] = {k.x, k.h, k.qkv, k.q, k.att, k.xm, k.h2, k.hid, k.s1.mean, k.s1.rstd, k.s2.mean, k.s2.rstd};
     }
-    *lead = s.lead;
     return b;
 }
 

@@ -167,3 +167,16 @@ def test_either_backward_takes_what_either_forward_has_saved():
         assert torch.equal(a, b), name
     a, b = flats["own"][0], flats["stack"][0]
     assert (a - b).norm() <= 2e-2 * a.norm()                            # the same gradients, through other 16-bit roundings of the stream
+
+
+def test_parts_behind_a_saving_stack_are_the_forwards_own():
+    """The stack part with `saved`, actor, critic and value without: one workspace, the same logits and values."""
+    m = _policy(torch.bfloat16, n_blocks=2)
+    c = _Calls(m, _batch(8 * CUS + 5)[0])
+    want, saved = c.rollout(), c.saved()
+    c.ws.fill_(0x7f)
+    assert c.lib.bsrl_note_train_begin(c.plan.desc, c.plan.pointers(c.params), *c._in, c.B, saved.data_ptr(), saved.numel(), 0) == 0
+    got = c.rollout(parts=1, saved=saved)
+    for parts in (4, 2, 8):
+        c.rollout(parts=parts, out=got)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
