@@ -54,6 +54,6 @@ int bsrl_blocks_unless(const bsrl_blocks_desc* d, const void* packed, const void
 // stack's output rows once more, beside the workspace's, from which the rollout's own readout goes on.
 struct BlocksSaveLayer { u16 *x, *h, *qkv, *q, *att, *xm, *h2, *hid; float *mean1, *rstd1, *mean2, *rstd2; };
 struct BlocksSave { const int32_t* noff; u16* lead; uint32_t rows; BlocksSaveLayer blk[BSRL_MAX_LAYERS]; };       // rows: what every buffer has room for
-// bsrl_blocks_pair (every env, whether pairs pay or not: a plan with env_ns = 0) that saves them
+// bsrl_blocks_pair that saves them, over every env, whether pairs pay or not
 bool bsrl_blocks_pair_saves(int64_t B, int d, int heads, int F, int T, int cus);
 int bsrl_blocks_pair_save(const BlocksPairArgs& a, const BlocksSave& save, int dtype, hipStream_t st);

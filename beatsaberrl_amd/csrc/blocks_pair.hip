@@ -794,6 +794,8 @@ bool bsrl_blocks_pair_saves(int64_t B, int d, int heads, int F, int T, int cus) 
 }
 
 int bsrl_blocks_pair_save(const BlocksPairArgs& a, const BlocksSave& save, int dtype, hipStream_t st) {
-    if (a.lead < 1 || a.lead > 5 || a.T <= a.lead || a.T - a.lead > 24 || a.n_layers < 1) return BSRL_UNSUPPORTED;
-    return dtype == BSRL_F16 ? go<F16, true>(a, save, st) : go<BF16, true>(a, save, st);
+    if (a.lead < 1 || a.lead > 5 || a.T <= a.lead || a.T - a.lead > 24 || a.n_layers < 1 || a.n_layers > BSRL_MAX_LAYERS) return BSRL_UNSUPPORTED;
+    BlocksPairArgs every = a;
+    every.plan.env_ns = 0;                           // no other kernel runs the envs that this one would leave
+    return dtype == BSRL_F16 ? go<F16, true>(every, save, st) : go<BF16, true>(every, save, st);
 }

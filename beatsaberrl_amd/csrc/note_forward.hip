@@ -240,8 +240,7 @@ extern "C" int bsrl_note_forward_saving(const bsrl_note_desc* d, const float* co
         if (!bsrl_mlp2_stream(e4, 4, PITCH, dt, st)) return BSRL_UNSUPPORTED;
         const bsrl_blocks_desc s = stack_of(*d);
         const int64_t frags = bsrl_blocks_pack_size(&s) - (int64_t)s.n_layers * (9 * D + s.ffn) * 4;
-        BlocksPairPlan plan = blocks_pair_plan(w.tiles, (int)bsrl_blocks_pair_chunks(B), bsrl_cus(), B, s.n_layers, s.ffn);
-        if (saved) plan.env_ns = 0;
+        const BlocksPairPlan plan = blocks_pair_plan(w.tiles, (int)bsrl_blocks_pair_chunks(B), bsrl_cus(), B, s.n_layers, s.ffn);
         const BlocksPairArgs p{static_cast<const uint4*>(m.blocks), reinterpret_cast<const float*>(static_cast<const char*>(m.blocks) + frags), w.x, w.bias, w.xres,
                                w.lead, w.pairs, plan, s.n_layers, s.ffn, T_TOK, N_LEAD, (int)(frags / (D / 16 * 1024))};
         if (saved) STEP(bsrl_blocks_pair_save(p, save, dt, st));
