@@ -120,9 +120,9 @@ template <int SF_, int SLOTS_, int NW_ = 8> struct StageRing {
     }
     // transfer K (of FPW) of the stage that admit<.., SPREAD> left to the even (0) or odd stage of its pair
     template <int PARITY, int K> __device__ __forceinline__ void load_due() {
-        constexpr uint32_t step = K < 3 ? 0 : 3072;            // (the immediate offset ends at 4095)
+        static_assert(1024 * K < 4096, "the immediate offset ends at 4095");
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3"
-                     ::"v"(voff), "s"(wsrc + due_src[PARITY] + step), "s"(wdst + due_slot[PARITY] + step), "n"(1024 * K - step));
+                     ::"v"(voff), "s"(wsrc + due_src[PARITY]), "s"(wdst + due_slot[PARITY]), "n"(1024 * K));
     }
     template <int PARITY> __device__ __forceinline__ void load_due_all() {
         static_for<0, FPW>([&](auto k) __attribute__((always_inline)) { load_due<PARITY, decltype(k)::value>(); });
