@@ -451,7 +451,7 @@ class NotePolicy(nn.Module):
         # The reference keeps the grad-free rollout forward and the grad-mode update forward bit-identical
         # (python/tests/test_fp16_accum.py:146-160): PPO's first-epoch ratio is then exactly 1.  The two fast rollout
         # routes above (fused block stack: fp32 residual in registers; pooled critic: k / v never rounded) differ from
-        # the update forward, which is the per-op route, by 16-bit rounding (log-prob of a 29-head action to ~1e-2,
+        # the per-op route, the update's own forward, by 16-bit rounding (log-prob of a 29-head action to ~1e-2,
         # value to ~2e-4 at the recipe shape).  True: the rollout takes the per-op route and the reference's critic op
         # order whatever the two switches say - same bits as the update forward, at the per-op route's speed.
         self.rollout_matches_update = False
@@ -461,7 +461,9 @@ class NotePolicy(nn.Module):
         # rollout's by 16-bit rounding, as any two 16-bit evaluations do).  Rollout and update outputs are then the
         # same bits in every mode and PPO's first-epoch ratio is exactly 1, for one more (fused, ~3 ms at the recipe
         # shape and 16384 envs) forward per update pass.  Where the library takes the update's block stack from that very
-        # forward (bsrl_note_train_saves: d = 192 past 8 envs per CU) the graph is its own, and there is no forward more.
+        # forward (bsrl_note_train_saves: d = 192 past 8 envs per CU) the graph is its own, and there is no forward more;
+        # all of it is then of the masters as they are, where otherwise the returned values are the last bumped version's.
+        # Which graph it is, the batch's size that is, is in the 16-bit rounding of an env's `_value_logits` and gradients.
         # "own": the update returns its own per-op values (the gap
         # bounded in the tests).  No effect on the fp32 stream, whose two forwards are the same ops.
         self.update_values = "rollout"
@@ -663,8 +665,9 @@ class NotePolicy(nn.Module):
     def _native_image(self, dt, arch=None, params=None, update=None, B=0):
         """(descriptor, weight image) of the native forward for the current weights version, or None where the forward runs op
         by op.  The image is rebuilt IN PLACE, as `blocks_image` is: its address is stable under a captured graph.  For an update
-        of B envs that takes this forward's block stack it is an image of its own, of the masters as they are now: the rest of
-        that update reads the masters themselves, and gradients must not mix two generations of them."""
+        of B envs that takes this forward's block stack it is of the masters as they are now - the one just rebuilt, or, within a
+        version, one of the update's own: the rest of that update reads the masters themselves, and gradients must not mix two
+        generations of them."""
         if (dt is torch.float32 or not self.fused_blocks_ok(dt) or not self.critic_pool
                 or not ops.critic_pool_supported(self.n_lead + N_NOTE_SLOTS, self.embed, self.n_heads, dt)):
             return None
@@ -679,7 +682,7 @@ class NotePolicy(nn.Module):
             c = self._native_cache = [-1, key, torch.zeros(n, dtype=torch.uint8, device=dev), desc]
         if c[2].numel() == 0:
             return None
-        own = update is not None and update.plan.saves(B, dev)
+        own = c[0] == _fl._weights_version and update is not None and update.plan.saves(B, dev)
         if own or c[0] != _fl._weights_version:
             params = params or self._native_params(arch)
             if params is None:
