@@ -12,7 +12,8 @@
 //   * every launch is enqueued here, ~3 us of host time each.
 // Past a round of the rollout's paired block stack (blocks_pair.hip, d = 192, more than 8 envs per CU) the stack's launch leaves the blocks'
 // activations here and this forward is what lies in front of it and behind it: 17.6 -> 14.2 ms for 16384 envs at the recipe's shape.  Up to
-// there the bin logits keep the op-by-op update's bits; past it the forward is the rollout's, nearer the fp32 one.
+// there the bin logits keep the op-by-op update's bits; past it the forward is the rollout's, whose stream is not rounded between blocks (its
+// error against 64 bits: blocks_pair.hip).  An env's bin logits and gradients differ by such roundings between the two.
 // Update of 16384 envs, recipe shape, before that: 26.1 -> 19.6 ms; 1500 envs, default shape: 6.4 -> 3.7 ms (the rollout's forward, the loss
 // and torch's part of the backward included).
 #include "note_train.h"
