@@ -98,12 +98,13 @@ def test_an_update_is_of_one_generation_of_weights():
         opt.step()
         if bump:
             fp16_linear.bump_weights_version()
+        image = m._native_cache[2]
         value, got = _grads(m, *batch)
+        assert m._native_cache[0] == fp16_linear._weights_version and m._native_cache[2] is image      # in place, where a captured rollout reads it
         fresh = _policy(torch.float16, n_blocks=2)
         fresh.load_state_dict(m.state_dict())
         want_value, want = _grads(fresh, *batch)
         assert torch.equal(value, want_value) and all(torch.equal(got[n], want[n]) for n in want), f"bump: {bump}"
-    assert m._native_cache[0] == fp16_linear._weights_version           # rebuilt in place, where a captured rollout reads it
     with torch.no_grad():
         _, _, _, v = m.get_action_and_value(*batch[:2])
     assert torch.equal(v, value)                                        # the rollout's image is the bumped version's
