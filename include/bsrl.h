@@ -646,10 +646,10 @@ int bsrl_note_train_forward(const bsrl_note_desc* desc, const float* const* para
                             int64_t saved_bytes, bsrl_stream stream);
 /* (ABI 22) The update's forward on the rollout forward's own block stack, which leaves what the backward reads: _begin fills
  * `saved` up to the encoders, bsrl_note_forward_saving is bsrl_note_forward whose STACK part writes the blocks' share (the
- * same logits and values; its other parts and bsrl_note_forward's are the same calls; image: of the masters in params), _end does trunk and critic; together they take the place of bsrl_note_train_forward, whose
- * forward rounds the stream to 16 bits between blocks where this one does not.  q, k, v lie otherwise in what they have
- * saved, which says so itself: bsrl_note_train_backward takes either (_stack_backward is the same call).  _saves: 1 where
- * they take B envs. */
+ * same logits and values; its other parts and bsrl_note_forward's are the same calls; image: of the masters in params), _end
+ * does trunk and critic; together they take the place of bsrl_note_train_forward, whose forward rounds the stream to 16 bits
+ * between blocks where this one does not.  q, k, v lie otherwise in what they have saved, which says so itself:
+ * bsrl_note_train_backward takes either (_stack_backward is the same call).  _saves: 1 where they take B envs. */
 int bsrl_note_train_saves(const bsrl_note_desc* desc, int64_t B);
 int bsrl_note_train_begin(const bsrl_note_desc* desc, const float* const* params, const void* obs,
                           int64_t obs_ld, int obs_dtype, const int32_t* saber_idx,
